@@ -269,7 +269,7 @@ class Mi355xBackend:
         several column windows takes its partial-sum workspace from stream-ordered memory."""
         check(
             self._lib().j4q_quant_matvec_into(
-                weights.handle, C.c_void_p(x_ptr), C.c_void_p(add_ptr or None), C.c_void_p(y_ptr), batch, C.c_void_p(stream or None)
+                weights.handle, x_ptr, add_ptr or None, y_ptr, batch, stream or None
             ),
             "quantMatvec_into",
         )
@@ -278,8 +278,7 @@ class Mi355xBackend:
         v = {"int8": N.GEMM_INT8, "bf16": N.GEMM_BF16}[variant]
         check(
             self._lib().j4q_quant_matmul_into(
-                weights.handle, C.c_void_p(x_ptr), m, v, C.c_void_p(xq_ptr or None), C.c_void_p(xs_ptr or None),
-                C.c_void_p(y_ptr), C.c_void_p(stream or None)
+                weights.handle, x_ptr, m, v, xq_ptr or None, xs_ptr or None, y_ptr, stream or None
             ),
             "quantMatmul_into",
         )
@@ -328,7 +327,7 @@ class DecodePlan:
 
     def run(self, stream: int = 0) -> None:
         """Enqueue one step on ``stream`` (0 = the engine stream); no synchronisation."""
-        check(self._be._lib().j4q_decode_plan_run(self.handle, C.c_void_p(stream or None)), "decode plan run")
+        check(self._be._lib().j4q_decode_plan_run(self.handle, stream or None), "decode plan run")
 
     def info(self) -> dict:
         d = N.DecodePlanDesc()

@@ -29,6 +29,7 @@ struct Buf {
     int64_t dims[2] = {0, 0};
     void *dev = nullptr;
     uint64_t bytes = 0;
+    uint64_t block = 0;  // bytes of its cached block (see BlockCache); 0: an allocation of its own
     uint32_t gen = 0;
     bool live = false;
     // decode plans whose captured graph reads this buffer's memory; while any lives the
@@ -56,6 +57,113 @@ bool g_ready = false;
 int g_dev = -1;
 hipStream_t g_stream = nullptr;
 thread_local std::string t_err;
+
+// Device memory the engine keeps between calls, under g_mu. hipMalloc + hipFree cost an SPI call
+// ~8 us and a wait for the device, hipMallocAsync + hipFreeAsync a call with a workspace ~15 us
+// (Q4_K 512 x 4096 at 16 rows: 19.7 us a call with them, 4.6 us of kernels).
+//  - Blocks of released F32 / BF16 / I8 buffers, in powers of two from 256 bytes to 4 MiB, at
+//    most 64 MiB in all: work on such a buffer runs on the engine stream alone, so its block may
+//    be written again behind it with no wait. A buffer whose address left the engine
+//    (j4q_buffer_info) can be in use on other streams and goes back with hipFree, which waits.
+//  - One workspace of at most 64 MiB for calls on the engine stream (which run one after another);
+//    calls on other streams take stream-ordered memory.
+//  - Neither serves a call under stream capture: a graph keeps the addresses it recorded.
+// All of it is given back when the last buffer is released.
+struct BlockCache {
+    static constexpr uint64_t kMaxBlock = 4ull << 20, kMaxBytes = 64ull << 20;
+    std::vector<void *> free_[23];  // by log2 of the block size
+    uint64_t bytes = 0;
+    static int slot(uint64_t n) {
+        int k = 8;
+        while ((1ull << k) < n) k++;
+        return k;
+    }
+    void *take(int k) {
+        if (free_[k].empty()) return nullptr;
+        void *p = free_[k].back();
+        free_[k].pop_back();
+        bytes -= 1ull << k;
+        return p;
+    }
+    bool give(void *p, int k) {
+        if (bytes + (1ull << k) > kMaxBytes) return false;
+        free_[k].push_back(p);
+        bytes += 1ull << k;
+        return true;
+    }
+    void clear() {
+        for (auto &v : free_) {
+            for (void *p : v) (void)hipFree(p);
+            v.clear();
+        }
+        bytes = 0;
+    }
+};
+BlockCache g_cache;
+constexpr uint64_t kMaxKeptWorkspace = 64ull << 20;
+void *g_kept_ws = nullptr;
+uint64_t g_kept_ws_bytes = 0;
+int64_t g_live = 0;  // live buffers
+
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
+void give_back_kept() {
+    g_cache.clear();
+    if (g_kept_ws) (void)hipFree(g_kept_ws);
+    g_kept_ws = nullptr;
+    g_kept_ws_bytes = 0;
+}
+
+// hipMalloc, a second time without what the engine keeps if memory is short.
+hipError_t dev_malloc(void **p, uint64_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && (g_kept_ws || g_cache.bytes)) {
+        (void)hipGetLastError();
+        give_back_kept();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
+// A workspace of `bytes` for the work that the caller enqueues on `s` before it calls
+// end_workspace.
+hipError_t begin_workspace(hipStream_t s, uint64_t bytes, void **out) {
+    if (s == g_stream && bytes <= kMaxKeptWorkspace && !capturing(s)) {
+        if (bytes > g_kept_ws_bytes) {
+            uint64_t want = 1ull << 20;
+            while (want < bytes) want *= 2;
+            // another stream may be under capture, where only a relaxed thread may allocate
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+            (void)hipThreadExchangeStreamCaptureMode(&mode);
+            if (g_kept_ws) (void)hipFree(g_kept_ws);  // waits for the work that uses it
+            g_kept_ws = nullptr;
+            g_kept_ws_bytes = 0;
+            if (hipMalloc(&g_kept_ws, want) == hipSuccess) {
+                g_kept_ws_bytes = want;
+            } else {
+                g_kept_ws = nullptr;
+                (void)hipGetLastError();
+            }
+            (void)hipThreadExchangeStreamCaptureMode(&mode);
+        }
+        if (bytes <= g_kept_ws_bytes) {
+            *out = g_kept_ws;
+            return hipSuccess;
+        }
+    }
+    return hipMallocAsync(out, bytes, s);
+}
+
+void end_workspace(hipStream_t s, void *p) {
+    if (p && p != g_kept_ws) (void)hipFreeAsync(p, s);
+}
 
 int fail(int code, const char *fmt, ...) {
     char buf[512];
@@ -155,6 +263,7 @@ j4q_buffer register_buf(const Buf &nb) {
     g_bufs[slot] = nb;
     g_bufs[slot].gen = gen;
     g_bufs[slot].live = true;
+    g_live++;
     return make_handle(slot, gen);
 }
 
@@ -178,7 +287,12 @@ int alloc_buf(int kind, int rank, int64_t d0, int64_t d1, uint64_t bytes, j4q_bu
     nb.dims[0] = d0;
     nb.dims[1] = d1;
     nb.bytes = bytes;
-    if (bytes) HIP_TRY("hipMalloc", hipMalloc(&nb.dev, bytes));
+    if (bytes && bytes <= BlockCache::kMaxBlock && !capturing(g_stream)) {
+        const int k = BlockCache::slot(bytes);
+        nb.block = 1ull << k;
+        nb.dev = g_cache.take(k);
+    }
+    if (bytes && !nb.dev) HIP_TRY("hipMalloc", dev_malloc(&nb.dev, nb.block ? nb.block : bytes));
     *out = register_buf(nb);
     *dev_out = nb.dev;
     return J4Q_OK;
@@ -192,6 +306,7 @@ void drop_buf(j4q_buffer *out) {
         if (b->dev) (void)hipFree(b->dev);
         b->dev = nullptr;
         b->live = false;
+        g_live--;
         g_free.push_back((uint32_t)((*out & 0xffffffffu) - 1));
     }
     *out = 0;
@@ -251,7 +366,7 @@ int upload_quant_common(int qt, const void *src, bool src_on_device, uint64_t nb
     void *staging = nullptr;
     const void *gguf = src;
     if (!src_on_device) {
-        HIP_TRY("hipMalloc", hipMalloc(&staging, nbytes));
+        HIP_TRY("hipMalloc", dev_malloc(&staging, nbytes));
         hipError_t e = hipMemcpyAsync(staging, src, nbytes, hipMemcpyHostToDevice, g_stream);
         if (e != hipSuccess) {
             (void)hipFree(staging);
@@ -260,7 +375,7 @@ int upload_quant_common(int qt, const void *src, bool src_on_device, uint64_t nb
         gguf = staging;
     }
     void *dev = nullptr;
-    hipError_t e = hipMalloc(&dev, L.total);
+    hipError_t e = dev_malloc(&dev, L.total);
     if (e == hipSuccess) e = j4q::launch_repack(qt, (const uint8_t *)gguf, (uint8_t *)dev, rows, cols, g_stream);
     if (e == hipSuccess) e = hipStreamSynchronize(g_stream);
     if (staging) (void)hipFree(staging);
@@ -347,7 +462,7 @@ int matvec_common(j4q_buffer wh, j4q_buffer xh, j4q_buffer addh, j4q_buffer *out
     const uint64_t wsb = j4q::gemv_workspace_bytes(qt, m, B);
     if (wsb) {
         void *p = nullptr;
-        if (hipMallocAsync(&p, wsb, g_stream) == hipSuccess) {
+        if (begin_workspace(g_stream, wsb, &p) == hipSuccess) {
             ws.ptr = (float *)p;
             ws.bytes = wsb;
         } else {
@@ -355,7 +470,7 @@ int matvec_common(j4q_buffer wh, j4q_buffer xh, j4q_buffer addh, j4q_buffer *out
         }
     }
     const hipError_t e = j4q::launch_gemv(qt, m, (const float *)xdev, (const float *)adev, (float *)ydev, B, g_stream, ws);
-    if (ws.ptr) (void)hipFreeAsync(ws.ptr, g_stream);
+    end_workspace(g_stream, ws.ptr);
     LAUNCH_INTO(op, out, e);
     return J4Q_OK;
 }
@@ -408,6 +523,7 @@ namespace abi {
 std::mutex &lock() { return g_mu; }
 int ready_locked() { return ensure_ready(); }
 hipStream_t stream() { return g_stream; }
+hipError_t malloc_locked(void **p, uint64_t bytes) { return dev_malloc(p, bytes); }
 
 int quant_locked(j4q_buffer h, const char *op, QuantRef *out) {
     Buf *b;
@@ -456,7 +572,7 @@ int concat_locked(const j4q_buffer *parts, int count, void **dev_out, QuantRef *
     // matching section of the result; Q8_0's block-major scale copy is rebuilt afterwards
     const SplitLayout L = split_layout(qt, rows, cols);
     void *dev = nullptr;
-    HIP_TRY("hipMalloc", hipMalloc(&dev, L.total));
+    HIP_TRY("hipMalloc", dev_malloc(&dev, L.total));
     hipError_t e = hipSuccess;
     uint64_t off[4] = {0, 0, 0, 0};
     for (int i = 0; i < count && e == hipSuccess; i++) {
@@ -599,7 +715,7 @@ int j4q_export_quantized(j4q_buffer wh, void *blocks, uint64_t nbytes) {
     if (nbytes != need) return fail(J4Q_EINVAL, "export: buffer is %llu bytes, need %llu", (unsigned long long)nbytes, (unsigned long long)need);
     if ((rc = ensure_ready())) return rc;
     void *tmp = nullptr;
-    HIP_TRY("hipMalloc", hipMalloc(&tmp, need));
+    HIP_TRY("hipMalloc", dev_malloc(&tmp, need));
     hipError_t e = j4q::launch_export(w->qtype, (const uint8_t *)w->dev, (uint8_t *)tmp, w->dims[0], w->dims[1], g_stream);
     if (e == hipSuccess) e = hipMemcpyAsync(blocks, tmp, need, hipMemcpyDeviceToHost, g_stream);
     if (e == hipSuccess) e = hipStreamSynchronize(g_stream);
@@ -677,6 +793,7 @@ int j4q_buffer_info(j4q_buffer h, j4q_buffer_desc *out) {
     out->dims[1] = b->dims[1];
     out->bytes = b->bytes;
     out->device_ptr = b->dev;
+    b->block = 0;  // its address leaves the engine: never reused without the wait of hipFree
     return J4Q_OK;
 }
 
@@ -708,11 +825,13 @@ int j4q_release(j4q_buffer h) {
     if (b->dev) {
         if ((rc = ensure_ready())) return rc;
         // hipFree waits for work that may still read the buffer.
-        HIP_TRY("hipFree", hipFree(b->dev));
+        if (!b->block || capturing(g_stream) || !g_cache.give(b->dev, BlockCache::slot(b->block)))
+            HIP_TRY("hipFree", hipFree(b->dev));
     }
     b->dev = nullptr;
     b->live = false;
     g_free.push_back((uint32_t)((h & 0xffffffffu) - 1));
+    if (--g_live == 0) give_back_kept();
     return J4Q_OK;
 }
 
@@ -816,20 +935,20 @@ int j4q_quant_matmul(j4q_buffer wh, j4q_buffer xh, int variant, j4q_buffer *out)
     if (variant == J4Q_GEMM_BF16) {
         void *ws = nullptr;
         const uint64_t wsb = gemm_bf16_workspace(qt, m, M);
-        if (wsb) LAUNCH_INTO("hipMallocAsync", out, hipMallocAsync(&ws, wsb, g_stream));
+        if (wsb) LAUNCH_INTO("hipMallocAsync", out, begin_workspace(g_stream, wsb, &ws));
         const hipError_t e = launch_gemm_bf16(qt, m, xdev, (float *)ydev, M, (float *)ws, g_stream);
-        if (ws) (void)hipFreeAsync(ws, g_stream);
+        end_workspace(g_stream, ws);
         LAUNCH_INTO("quantMatmul", out, e);
         return J4Q_OK;
     }
     void *ws = nullptr;
     const uint64_t qbytes = (uint64_t)(M * K), sbytes = (uint64_t)(M * (K / 32)) * 4;
-    LAUNCH_INTO("hipMallocAsync", out, hipMallocAsync(&ws, j4q::align256(qbytes) + sbytes, g_stream));
+    LAUNCH_INTO("hipMallocAsync", out, begin_workspace(g_stream, j4q::align256(qbytes) + sbytes, &ws));
     int8_t *xq = (int8_t *)ws;
     float *xs = (float *)((uint8_t *)ws + j4q::align256(qbytes));
     hipError_t e = j4q::launch_quantize_act(xdev, M, K, xq, xs, g_stream);
     if (e == hipSuccess) e = j4q::launch_gemm_q8_int8(m, xq, xs, (float *)ydev, M, g_stream);
-    (void)hipFreeAsync(ws, g_stream);
+    end_workspace(g_stream, ws);
     LAUNCH_INTO("quantMatmul", out, e);
     return J4Q_OK;
 }
@@ -859,12 +978,12 @@ int j4q_quant_matvec_into(j4q_buffer wh, const float *x, const float *add, float
     const uint64_t wsb = j4q::gemv_workspace_bytes(w->qtype, m, batch);
     if (wsb) {
         void *p = nullptr;
-        HIP_TRY("hipMallocAsync", hipMallocAsync(&p, wsb, s));
+        HIP_TRY("hipMallocAsync", begin_workspace(s, wsb, &p));
         ws.ptr = (float *)p;
         ws.bytes = wsb;
     }
     const hipError_t e = j4q::launch_gemv(w->qtype, m, x, add, y, batch, s, ws);
-    if (ws.ptr) (void)hipFreeAsync(ws.ptr, s);
+    end_workspace(s, ws.ptr);
     HIP_TRY("quantMatvec_into", e);
     return J4Q_OK;
 }
@@ -889,9 +1008,9 @@ int j4q_quant_matmul_into(j4q_buffer wh, const uint16_t *x, int64_t m, int varia
     if (variant == J4Q_GEMM_BF16) {
         void *ws = nullptr;
         const uint64_t wsb = gemm_bf16_workspace(w->qtype, mm, m);
-        if (wsb) HIP_TRY("hipMallocAsync", hipMallocAsync(&ws, wsb, s));
+        if (wsb) HIP_TRY("hipMallocAsync", begin_workspace(s, wsb, &ws));
         const hipError_t e = launch_gemm_bf16(w->qtype, mm, x, y, m, (float *)ws, s);
-        if (ws) (void)hipFreeAsync(ws, s);
+        end_workspace(s, ws);
         HIP_TRY("quantMatmul_into", e);
         return J4Q_OK;
     }

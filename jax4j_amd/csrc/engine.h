@@ -23,6 +23,10 @@ int ready_locked();
 // The engine stream (valid after ready_locked()).
 hipStream_t stream();
 
+// With the lock held: hipMalloc, after the memory that the engine keeps between calls has been
+// given back where it was short.
+hipError_t malloc_locked(void **p, uint64_t bytes);
+
 // A resident quantized matrix, as the kernels see it.
 struct QuantRef {
     int qtype;

@@ -147,7 +147,7 @@ int build_group(Plan &p, const j4q_buffer *parts, int count, const char *what, c
             p.ops.push_back(g);
         } else {
             void *scratch = nullptr;
-            const hipError_t e = hipMalloc(&scratch, (size_t)(p.batch * run.rows) * 4);
+            const hipError_t e = abi::malloc_locked(&scratch, (size_t)(p.batch * run.rows) * 4);
             if (e != hipSuccess) return report_hip("decode plan scratch", e);
             p.owned.push_back(scratch);
             p.desc.plan_bytes += (uint64_t)(p.batch * run.rows) * 4;
@@ -258,7 +258,7 @@ int j4q_decode_plan_create(const j4q_decode_layer *layers, int32_t n_layers, j4q
     if ((rc = check_shapes(layers, n_layers, head, &p.desc))) return rc;
     const int64_t B = batch, D = p.desc.d_model;
     void *h2 = nullptr;
-    hipError_t e = hipMalloc(&h2, (size_t)(B * D) * 4);
+    hipError_t e = abi::malloc_locked(&h2, (size_t)(B * D) * 4);
     if (e != hipSuccess) return report_hip("decode plan residual buffer", e);
     p.owned.push_back(h2);
     p.desc.plan_bytes += (uint64_t)(B * D) * 4;
@@ -281,7 +281,7 @@ int j4q_decode_plan_create(const j4q_decode_layer *layers, int32_t n_layers, j4q
     }
     if (!rc && wsb) {
         void *d = nullptr;
-        e = hipMalloc(&d, wsb);
+        e = abi::malloc_locked(&d, wsb);
         if (e != hipSuccess) {
             rc = report_hip("decode plan workspace", e);
         } else {

@@ -1,0 +1,149 @@
+"""The device memory that the engine keeps between calls: blocks of released dense buffers and
+the workspace of calls on the engine stream.
+
+Bar: bit for bit what the same call gives on memory of its own. Calls write into blocks that
+queued work has just used, sizes on both sides of a block class and above the largest one,
+workspaces grow between calls, and calls on a stream of the caller's run beside calls on the
+engine stream.
+"""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from jax4j_amd import QuantType
+from jax4j_amd import _native as N
+from jax4j_amd import synthetic as S
+
+pytestmark = pytest.mark.gpu
+
+
+def upload(backend, qt, rows, cols, seed):
+    return backend.upload_quantized(S.quant_blocks(qt, seed, rows, cols), qt, (rows, cols))
+
+
+# 64 and 65 floats: both sides of a 256-byte block; 1 Mi and 1 Mi + 32: of the largest (4 MiB)
+@pytest.mark.parametrize("rows", [1, 64, 65, 4096, 1 << 20, (1 << 20) + 32])
+def test_results_in_reused_blocks_are_those_of_fresh_ones(backend, rows):
+    w = upload(backend, QuantType.Q4_0, rows, 32, 5)
+    xs = [backend.upload(S.activations_f32(7 + i, 32)) for i in range(3)]
+    keep = [backend.quant_matvec(w, x) for x in xs]
+    fresh = [backend.download(y) for y in keep]
+    for i in range(12):  # each result's block goes to the next call while its work may be queued
+        y = backend.quant_matvec(w, xs[i % 3])
+        z = backend.quant_matvec_add(w, xs[(i + 1) % 3], y)
+        backend.release(y)
+        g = backend.quant_gather_row(w, rows - 1)
+        backend.release(g)
+        got = backend.download(z)
+        assert np.array_equal(got.view(np.uint32), (fresh[(i + 1) % 3] + fresh[i % 3]).view(np.uint32))
+        backend.release(z)
+    for b in [w, *xs, *keep]:
+        backend.release(b)
+
+
+class Hip:
+    """The HIP runtime the engine is linked to: a stream of the caller's, and stream capture."""
+
+    def __init__(self):
+        self.lib = N.load()
+        self.stream = C.c_void_p()
+        self.ok("hipStreamCreateWithFlags", C.byref(self.stream), 1)  # non-blocking
+
+    def ok(self, name, *args):
+        assert getattr(self.lib, name)(*args) == 0, name
+
+    def wait(self):
+        self.ok("hipDeviceSynchronize")
+
+    def close(self):
+        self.wait()
+        self.ok("hipStreamDestroy", self.stream)
+
+
+def test_an_address_given_out_is_not_reused_behind_its_work(backend):
+    """A buffer whose address was read may be in use on a stream of the caller's when it is released:
+    the work queued there still sees its own values."""
+    n = 1 << 18
+    hip, lib = Hip(), N.load()
+    values = S.activations_f32(11, n)
+    b, out = backend.upload(values), backend.upload(np.zeros(n, np.float32))
+    src, dst = (backend.buffer_desc(h).device_ptr for h in (b, out))
+    assert lib.j4q_spin(3000, hip.stream) == 0
+    assert lib.j4q_copy(dst, src, 4 * n, hip.stream) == 0
+    backend.release(b)
+    others = [backend.upload(np.full(n, np.nan, np.float32)) for _ in range(2)]
+    hip.wait()
+    assert np.array_equal(backend.download(out), values)
+    for h in [out, *others]:
+        backend.release(h)
+    hip.close()
+
+
+@pytest.mark.parametrize("qt", [QuantType.Q4_K, QuantType.Q8_0], ids=lambda q: q.name)
+def test_workspace_calls_on_two_streams_and_growing(backend, qt):
+    """16 rows over several column windows use a workspace: one kept for the engine stream that grows
+    from the first matrix to the second, stream-ordered memory on another stream."""
+    hip = Hip()
+    shapes = [(96, 4096), (4000, 8192)]
+    ws = [upload(backend, qt, r, k, 20 + r) for r, k in shapes]
+    xs = [backend.upload(S.activations_f32(3 + k, 16 * k), shape=(16, k)) for _, k in shapes]
+    ptr = lambda h: backend.buffer_desc(h).device_ptr
+
+    def result(i):
+        return backend.upload(np.full((16, shapes[i][0]), np.nan, np.float32))
+
+    def call(i, y, stream):
+        backend.quant_matvec_into(ws[i], ptr(xs[i]), 0, ptr(y), 16, stream)
+
+    ref = []
+    for i in range(2):  # alone, each waited for
+        y = result(i)
+        call(i, y, hip.stream.value)
+        hip.wait()
+        ref.append(backend.download(y))
+        backend.release(y)
+    calls = [(0, 0), (1, hip.stream.value), (1, 0), (0, hip.stream.value), (0, 0), (1, 0)]
+    ys = [result(i) for i, _ in calls]
+    for (i, stream), y in zip(calls, ys):
+        call(i, y, stream)
+    hip.wait()
+    for (i, _), y in zip(calls, ys):
+        assert np.array_equal(backend.download(y).view(np.uint32), ref[i].view(np.uint32))
+    for h in [*ws, *xs, *ys]:
+        backend.release(h)
+    hip.close()
+
+
+def test_workspace_call_under_capture_replays(backend):
+    """Under capture of the engine stream a call takes memory of the graph, not the kept workspace: eager
+    calls between the replays do not change what they give."""
+    r, k = 640, 4096
+    hip = Hip()
+    st = C.c_void_p(backend.stream())
+    w = upload(backend, QuantType.Q4_K, r, k, 31)
+    x = backend.upload(S.activations_f32(5, 16 * k), shape=(16, k))
+    y, z = (backend.upload(np.zeros((16, r), np.float32)) for _ in range(2))
+    px, py, pz = (backend.buffer_desc(h).device_ptr for h in (x, y, z))
+    nan = backend.upload(np.full((16, r), np.nan, np.float32))
+    pnan = backend.buffer_desc(nan).device_ptr
+    backend.quant_matvec_into(w, px, 0, pz, 16)
+    ref = backend.download(z).view(np.uint32)
+    graph, run = C.c_void_p(), C.c_void_p()
+    hip.ok("hipStreamBeginCapture", st, 2)  # relaxed
+    backend.quant_matvec_into(w, px, 0, py, 16)
+    hip.ok("hipStreamEndCapture", st, C.byref(graph))
+    hip.ok("hipGraphInstantiate", C.byref(run), graph, None, None, C.c_size_t(0))
+    for _ in range(4):
+        assert N.load().j4q_copy(py, pnan, 4 * 16 * r, None) == 0
+        hip.ok("hipGraphLaunch", run, st)
+        backend.quant_matvec_into(w, px, 0, pz, 16)
+        assert np.array_equal(backend.download(y).view(np.uint32), ref)
+        assert np.array_equal(backend.download(z).view(np.uint32), ref)
+    hip.ok("hipGraphExecDestroy", run)
+    hip.ok("hipGraphDestroy", graph)
+    for h in (w, x, y, z, nan):
+        backend.release(h)
+    hip.close()
