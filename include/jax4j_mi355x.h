@@ -202,8 +202,8 @@ int j4q_quant_matvec_into(j4q_buffer weights, const float *x_dev, const float *a
 /* Prefill GEMM into caller memory (the weight types and variants of j4q_quant_matmul).
  * x_dev bf16 [m, cols]; y_dev fp32 [m, rows]. The int8 variant also needs xq_dev int8
  * [m, cols] and xs_dev fp32 [m, cols/32] as workspace; the bf16 variant ignores them. On
- * Q4_0, Q4_K and Q6_K weights with a small grid (few rows of X) the bf16 variant splits K
- * over workgroups and keeps the partial products (at most 32 MiB) in the engine's kept
+ * Q4_0, Q4_K and Q6_K weights the bf16 variant splits K over workgroups where the tiles alone
+ * would leave CUs idle, and keeps the partial products (at most 32 MiB) in the engine's kept
  * workspace on the engine stream, else in stream-ordered memory of `stream` (hipMallocAsync /
  * hipFreeAsync); nothing else is allocated. */
 int j4q_quant_matmul_into(j4q_buffer weights, const uint16_t *x_dev, int64_t m, int variant, int8_t *xq_dev,

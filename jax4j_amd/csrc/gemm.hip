@@ -427,6 +427,8 @@ hipError_t launch_gemm_q8_int8(const QMat &w, const int8_t *xq, const float *xs,
     return launch_gemm<kVarInt8, 128, 128, 4, 3>(w, xq, xs, y, m, s);
 }
 
+// The calls that gemm_tile.hip leaves to these kernels: K % 64 != 0, and the small grids on which
+// they are faster (q8_wide_us there models their times by the rules below).
 hipError_t launch_gemm_q8_bf16(const QMat &w, const uint16_t *x, float *y, int64_t m, hipStream_t s) {
     if (m <= 0 || w.rows <= 0) return hipSuccess;
     if (m > 65535 * 64 || w.cols % 32 != 0 || (uint64_t)m * w.cols * 2 > 0x7fffffffull) return hipErrorInvalidValue;

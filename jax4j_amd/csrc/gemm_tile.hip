@@ -1,0 +1,172 @@
+// Prefill GEMM, bf16 variant: picks the tile and the K split of the LDS-tiled kernel
+// (gemm_tile.h) for the shape, and the kernels of gemm_wide.h where they are faster (Q8_0).
+#include "j4q_common.h"
+#include "gemm_tile.h"
+
+namespace j4q {
+namespace {
+
+// A launch of gemm_tile: tiles of 32 tm rows x 32 waves columns, K in `splits` ranges of
+// split_stages 64-element stages. tm = 0: the call does not run on it.
+struct Shape {
+    int waves = 0, tm = 0, splits = 1, split_stages = 0;
+};
+
+// The tiles, and what one stage of one workgroup takes in us on MI355X: few workgroups, each
+// alone on its CU (few); one on every CU (all: the chip's clock and its memory are shared); and as
+// a share of the CU's time when every CU runs several, one after another or side by side (shared).
+// From sweeps of Q4_K, Q4_0 and Q8_0 over N = 700 .. 14336, K = 1024 .. 14336, M = 8 .. 2048.
+struct Cost {
+    int waves, tm;
+    float few, all, shared;
+};
+constexpr Cost kCost[] = {{4, 1, .33f, .38f, .26f}, {4, 2, .38f, .43f, .34f}, {4, 3, .45f, .50f, .43f},
+                          {4, 4, .47f, .57f, .51f}, {4, 5, .58f, .68f, .63f}, {8, 4, .62f, 1.02f, 1.0f},
+                          {8, 8, 1.2f, 1.75f, 1.75f}};
+constexpr int kCus = 256;  // of an MI355X; a constant, so that results do not depend on the device
+
+// The fastest shape by a model of the launch: the stages that the busiest CU runs (Q6_K's take
+// longer to decode, Q8_0's to load), a launch's fixed 3 us, and with K split the sum kernel: 2 us,
+// a quarter per split, and its traffic (the partial products written and read, the result written)
+// at 5.5 MB/us. Over the sweeps (38 sizes) its choice takes 1.2 % longer than the best of all
+// shapes on average, 11 % at worst. Splits are whole multiples of four stages, and their workspace
+// is at most 32 MiB; a Q8_0 call takes no workspace, so it does not split.
+Shape pick(int id, const QMat &w, int64_t m, float *us_out) {
+    const int64_t n = w.rows, ns = w.cols / 64;
+    const float alone_add = id == Q6_K ? .12f : id == Q8_0 ? .05f : 0.f, shared_add = id == Q6_K ? .09f : id == Q8_0 ? .05f : 0.f;
+    Shape best;
+    float best_us = 0.f;
+    for (const Cost &c : kCost) {
+        const int64_t tiles = ((m + 32 * c.tm - 1) / (32 * c.tm)) * ((n + 32 * c.waves - 1) / (32 * c.waves));
+        int64_t last = 0;
+        for (int64_t want = 1; want <= (id == Q8_0 ? 1 : 16); want++) {
+            const int64_t per = want == 1 ? ns : ((ns + want - 1) / want + 3) / 4 * 4, s = (ns + per - 1) / per;
+            if (s == last || (s > 1 && s * m * n * 4 > (32ll << 20))) continue;
+            last = s;
+            const int64_t groups = tiles * s, rounds = (groups + kCus - 1) / kCus;
+            float us = rounds <= 1 ? c.few + (c.all - c.few) * (float)groups / kCus + alone_add : (float)rounds * (c.shared + shared_add);
+            us = us * (float)per + 3.0f;
+            if (s > 1) us += 2.0f + .25f * (float)s + (float)((2 * s + 1) * m * n * 4) / 5.5e6f;
+            if (!best.tm || us < best_us) {
+                best_us = us;
+                best = Shape{c.waves, c.tm, (int)s, (int)per};
+            }
+        }
+    }
+    *us_out = best_us;
+    return best;
+}
+
+// The same model of the Q8_0 kernels of gemm_wide.h (launch_gemm_q8_bf16 picks among them by these
+// rules): us per stage of one workgroup, measured at N = K = 4096. Where none of them applies,
+// the 4-wave kernel would run, which is slower at every size tried (M = 200, N = 700, K = 1024:
+// 12.0 us against 8.0).
+float q8_wide_us(const QMat &w, int64_t m) {
+    const int64_t n = w.rows, k = w.cols;
+    auto tiles = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
+    auto us = [&](int64_t t, int64_t stage, float per) { return (float)((t + kCus - 1) / kCus * ((k + stage - 1) / stage)) * per + 3.0f; };
+    if (m > 64 && n % 2 == 0) {
+        if (tiles(128, 128) >= 256) return 1e30f;  // M = 2048: 84-90 us against 71-72
+        if (tiles(128, 64) >= 192) return us(tiles(128, 64), 128, .75f);
+        if (tiles(64, 64) >= 128) return us(tiles(64, 64), 128, tiles(64, 64) > kCus ? .40f : .46f);
+    }
+    if (m >= 512) return us(tiles(128, 64), 64, .53f);
+    if (m <= 32) return us(tiles(32, 16), 512, .85f);
+    if (m <= 192) return us(tiles(64, 16), 256, .62f);
+    return 1e30f;
+}
+
+// Whether the tile kernel takes the call; the shape it runs with.
+Shape shape_of(int id, const QMat &w, int64_t m) {
+    float us = 0.f;
+    if (id == Q8_0 && w.cols % 64 != 0) return Shape{};
+    const Shape t = pick(id, w, m, &us);
+    return id == Q8_0 && q8_wide_us(w, m) <= 1.05f * us ? Shape{} : t;
+}
+
+// y[i] = ((part[0][i] + part[1][i]) + ...) for i < n: the K splits' partial products added
+// in split order (deterministic). A thread takes four consecutive elements when n % 4 == 0
+// (every split then starts 16-byte aligned; y is), else one.
+__global__ void __launch_bounds__(256)
+sum_splits_kernel(const float *__restrict__ part, int splits, int64_t n, float *__restrict__ y) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    const int64_t stride = (int64_t)gridDim.x * 256;
+    if (n % 4 == 0) {
+        for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n / 4; i += stride) {
+            f32x4 v = reinterpret_cast<const f32x4 *>(part)[i];
+            for (int r = 1; r < splits; r++) v += reinterpret_cast<const f32x4 *>(part + (int64_t)r * n)[i];
+            reinterpret_cast<f32x4 *>(y)[i] = v;
+        }
+        return;
+    }
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) {
+        float v = part[i];
+        for (int r = 1; r < splits; r++) v += part[(int64_t)r * n + i];
+        y[i] = v;
+    }
+}
+
+template <int FMT>
+hipError_t launch_fmt(const QMat &w, const uint16_t *x, float *y, int64_t m, const Shape &t, float *ws, hipStream_t s) {
+    const int64_t tiles = ((m + 32 * t.tm - 1) / (32 * t.tm)) * ((w.rows + 32 * t.waves - 1) / (32 * t.waves));
+    if (tiles > 0x7fffffff || (t.splits > 1 && !ws)) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)tiles, (unsigned)t.splits);
+    float *const part = t.splits > 1 ? ws : nullptr;
+    bool launched = false;
+#define J4Q_TILE(WV, TM)                                                                              \
+    if (t.waves == WV && t.tm == TM) {                                                                \
+        gt::gemm_tile<FMT, WV, TM><<<grid, 64 * WV, 0, s>>>(w, x, y, (int)m, t.split_stages, part);   \
+        launched = true;                                                                              \
+    }
+    J4Q_TILE(4, 1)
+    J4Q_TILE(4, 2)
+    J4Q_TILE(4, 3)
+    J4Q_TILE(4, 4)
+    J4Q_TILE(4, 5)
+    J4Q_TILE(8, 4)
+    J4Q_TILE(8, 8)
+#undef J4Q_TILE
+    if (!launched) return hipErrorInvalidValue;
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || t.splits == 1) return e;
+    const int64_t n = m * w.rows;
+    const int64_t blocks = ((n % 4 == 0 ? n / 4 : n) + 255) / 256;
+    sum_splits_kernel<<<(unsigned)(blocks < 2048 ? blocks : 2048), 256, 0, s>>>(ws, t.splits, n, y);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+bool gemm_bf16_supported(int id, int64_t cols) {
+    switch (id) {
+    case Q8_0: return cols % 32 == 0;
+    case Q4_0: return cols % 128 == 0;
+    case Q4_K:
+    case Q6_K: return cols % 256 == 0;
+    default: return false;
+    }
+}
+
+uint64_t gemm_bf16_workspace_bytes(int id, const QMat &w, int64_t m) {
+    if (!gemm_bf16_supported(id, w.cols) || m <= 0 || w.rows <= 0) return 0;
+    const Shape t = shape_of(id, w, m);
+    return t.splits > 1 ? (uint64_t)t.splits * (uint64_t)m * (uint64_t)w.rows * 4u : 0;
+}
+
+hipError_t launch_gemm_bf16(int id, const QMat &w, const uint16_t *x, float *y, int64_t m, float *ws, hipStream_t s) {
+    if (m <= 0 || w.rows <= 0) return hipSuccess;
+    const Shape t = shape_of(id, w, m);
+    if (id == Q8_0 && !t.tm) return launch_gemm_q8_bf16(w, x, y, m, s);
+    if (!gemm_bf16_supported(id, w.cols) || (uint64_t)m * (uint64_t)w.cols * 2u > 0x7fffffffull ||
+        (uint64_t)w.rows * (uint64_t)w.cols / (id == Q8_0 ? 1u : 2u) > 0x7fffffffull)
+        return hipErrorInvalidValue;
+    switch (id) {
+    case Q8_0: return launch_fmt<Q8_0>(w, x, y, m, t, ws, s);
+    case Q4_0: return launch_fmt<Q4_0>(w, x, y, m, t, ws, s);
+    case Q4_K: return launch_fmt<Q4_K>(w, x, y, m, t, ws, s);
+    case Q6_K: return launch_fmt<Q6_K>(w, x, y, m, t, ws, s);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace j4q
