@@ -73,20 +73,88 @@ __device__ __forceinline__ u32x2 deq4(uint32_t even, uint32_t odd, float s, floa
     return r;
 }
 
+// A W unit of a tile in LDS: two stages (four 32-blocks) of the 32 WV rows of W that the tile's waves
+// use, loaded by the wave that uses them: quants, Q6_K's high bits, scale words (one array, so few
+// that the compiler tracks the loads into each of them apart).
+template <int FMT, int WV>
+struct WUnit {
+    static constexpr int QR = FMT == Q8_0 ? 128 : 64;              // bytes of quants per row
+    static constexpr int QL = QR / 32;                             // their loads per wave
+    static constexpr int kLoads = QL + (FMT == Q6_K ? 3 : 1);      // all loads per wave
+    static constexpr int kH = 32 * WV * QR;                        // offset of the high bits
+    static constexpr int kS = kH + (FMT == Q6_K ? 32 * WV * 32 : 0);      // ... of the scale words
+    static constexpr int kSlot = FMT == Q4_K ? 1024 : FMT == Q6_K ? 512 : 256;  // scale words of one wave
+    static constexpr int kBytes = kS + WV * kSlot;
+
+    __amdgpu_buffer_rsrc_t qr, hr, sr;
+    uint32_t qoff[QL], hoff, soff, doff;
+    int wave;
+
+    // 16-byte chunk c of row r sits at slot c ^ swz(r): the rows of a quarter-wave read fall on
+    // distinct banks.
+    static __device__ __forceinline__ int swz(int row) { return QR == 128 ? (row >> 1) & 7 : (row >> 2) & 3; }
+
+    // nw: the wave's first row of W.
+    __device__ __forceinline__ void init(const QMat &w, int nw, int wave_, int lane) {
+        const int N = (int)w.rows, K = (int)w.cols, nsb = K / 256;
+        wave = wave_;
+        // Quants: a load fills 1024 / QR rows (QR / 16 lanes a row); the slot of a lane holds the
+        // chunk that the row's swizzle puts there.
+        const uint32_t qrow = FMT == Q8_0 ? (uint32_t)K : (uint32_t)(K / 2);
+        qr = make_rsrc(w.qs, (uint64_t)N * qrow);
+#pragma unroll
+        for (int j = 0; j < QL; j++) {
+            const int row = j * (1024 / QR) + lane / (QR / 16), c = (lane % (QR / 16)) ^ swz(row), n = nw + row;
+            qoff[j] = n < N ? (uint32_t)n * qrow + (uint32_t)c * 16u : kOob;
+        }
+        // Q6_K high bits: lane L: 16-byte half L % 2 of the unit's 32 bytes of row L / 2.
+        const int n2 = nw + (lane >> 1);
+        hr = make_rsrc(w.qh, FMT == Q6_K ? (uint64_t)N * (uint64_t)K / 4u : 0);
+        hoff = n2 < N ? (uint32_t)n2 * (uint32_t)(K / 4) + (uint32_t)(lane & 1) * 16u : kOob;
+        // Scale words into this wave's slot:
+        //  Q8_0, Q4_0: lane L: dword L % 2 of the unit's four fp16 d of row L / 2;
+        //  Q4_K: lane r < 32: row r's 16-byte superblock record (the other lanes write zeros behind:
+        //        a branch around them would blur the compiler's wait counts);
+        //  Q6_K: lane L: dword L % 2 of the unit's eight int8 group scales of row L / 2; then lane
+        //        r < 32: the aligned dword holding row r's fp16 superblock d (the d section follows
+        //        the sc section in the matrix's allocation, so one buffer resource from sc to the
+        //        end of d's 256-byte-aligned section serves both).
+        const uint32_t d_rel = FMT == Q6_K ? (uint32_t)(w.d - w.sc) : 0u;
+        sr = make_rsrc(w.sc, FMT == Q6_K ? (uint64_t)d_rel + align256((uint64_t)N * (uint64_t)nsb * 2u)
+                                         : (uint64_t)N * (uint64_t)(K / 16));
+        soff = doff = kOob;
+        if constexpr (FMT == Q4_K) {
+            if (lane < 32 && nw + lane < N) soff = (uint32_t)(nw + lane) * (uint32_t)(K / 16);
+        } else {
+            if (n2 < N) soff = (uint32_t)n2 * (uint32_t)(K / 16) + (uint32_t)(lane & 1) * 4u;
+            if (FMT == Q6_K && lane < 32 && nw + lane < N) doff = d_rel + (uint32_t)(nw + lane) * (uint32_t)(nsb * 2);
+        }
+    }
+    // Unit u (stages 2 u and 2 u + 1) into wb; zeros when not live.
+    __device__ __forceinline__ void load(int u, bool live, uint8_t *wb) const {
+        uint8_t *const slot = wb + kS + wave * kSlot;
+        const uint32_t uu = live ? (uint32_t)u : 0u;
+#pragma unroll
+        for (int j = 0; j < QL; j++) dma16(qr, wb + (wave * QL + j) * 1024, live ? qoff[j] : kOob, uu * (uint32_t)QR);
+        if constexpr (FMT == Q6_K) {
+            dma16(hr, wb + kH + wave * 1024, live ? hoff : kOob, uu * 32u);
+            dma4(sr, slot, live && soff != kOob ? soff + uu * 8u : kOob);
+            dma4(sr, slot + 256, live && doff != kOob ? (doff + (uu >> 1) * 2u) & ~3u : kOob);
+        } else if constexpr (FMT == Q4_K) {
+            dma16(sr, slot, live ? soff : kOob, (uu >> 1) * 16u);
+        } else {
+            dma4(sr, slot, live && soff != kOob ? soff + uu * 8u : kOob);
+        }
+    }
+};
+
 template <int FMT, int WV, int TM>
 struct Tile {
     static constexpr int BM = 32 * TM, BN = 32 * WV;
-    static constexpr int XL = 4 * TM / WV;                         // X loads per wave and stage
-    static constexpr int QR = FMT == Q8_0 ? 128 : 64;              // bytes of quants per row and unit
-    static constexpr int QL = QR / 32;                             // their loads per wave and unit
-    static constexpr int WL = QL + (FMT == Q6_K ? 3 : 1);          // all loads per wave and unit
+    static constexpr int XL = 4 * TM / WV;  // X loads per wave and stage
     static constexpr int kX = BM * 128;
-    static constexpr int kQ = BN * QR;
-    static constexpr int kH = FMT == Q6_K ? BN * 32 : 0;
-    static constexpr int kSlot = FMT == Q4_K || FMT == Q6_K ? 512 : 256;  // scale words of one wave
-    static constexpr int kW = kQ + kH + WV * kSlot;                // one unit's buffer
     static_assert(4 * TM % WV == 0, "whole X loads per wave");
-    static_assert(2 * (kX + kW) <= 163840, "LDS");
+    static_assert(2 * (kX + WUnit<FMT, WV>::kBytes) <= 163840, "LDS");
 };
 
 template <int FMT, int WV, int TM>
@@ -94,11 +162,10 @@ __global__ void __launch_bounds__(64 * WV, 2)
 gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, int split_stages,
           float *__restrict__ part) {
     using T = Tile<FMT, WV, TM>;
-    constexpr int BM = T::BM, BN = T::BN, QR = T::QR, QL = T::QL, WL = T::WL, XL = T::XL;
+    using U = WUnit<FMT, WV>;
+    constexpr int BM = T::BM, BN = T::BN, QR = U::QR, WL = U::kLoads, XL = T::XL;
     __shared__ __attribute__((aligned(1024))) uint8_t xs0[T::kX], xs1[T::kX];
-    // a W unit: quants, Q6_K's high bits, scale words (one array, so few that the compiler tracks
-    // the loads into each of them apart)
-    __shared__ __attribute__((aligned(1024))) uint8_t ws0[T::kW], ws1[T::kW];
+    __shared__ __attribute__((aligned(1024))) uint8_t ws0[U::kBytes], ws1[U::kBytes];
     const int N = (int)w.rows, K = (int)w.cols;
     const int sbeg = (int)blockIdx.y * split_stages, send = sbeg + split_stages, all = K / 64;
     const int ns = send < all ? send : all;  // stages [sbeg, ns)
@@ -124,41 +191,10 @@ gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, 
         const int row = 8 * (WV * j + wave) + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
         xoff[j] = m0 + row < M ? (uint32_t)(m0 + row) * (uint32_t)K * 2u + (uint32_t)c * 16u : kOob;
     }
-    // Quants: a load fills 1024 / QR of this wave's rows 32 wave .. + 31 (QR / 16 lanes a row); the
-    // slot of a lane holds the chunk that the row's swizzle puts there.
     const int nw = n0 + 32 * wave;  // this wave's first column
-    const uint32_t qrow = FMT == Q8_0 ? (uint32_t)K : (uint32_t)(K / 2);
-    const __amdgpu_buffer_rsrc_t qr = make_rsrc(w.qs, (uint64_t)N * qrow);
-    auto qswz = [](int row) __attribute__((always_inline)) { return QR == 128 ? (row >> 1) & 7 : (row >> 2) & 3; };
-    uint32_t qoff[QL];
-#pragma unroll
-    for (int j = 0; j < QL; j++) {
-        const int row = j * (1024 / QR) + lane / (QR / 16), c = (lane % (QR / 16)) ^ qswz(row), n = nw + row;
-        qoff[j] = n < N ? (uint32_t)n * qrow + (uint32_t)c * 16u : kOob;
-    }
-    // Q6_K high bits: lane L: 16-byte half L % 2 of the unit's 32 bytes of row L / 2.
-    const int n2 = nw + (lane >> 1);
-    const __amdgpu_buffer_rsrc_t hr = make_rsrc(w.qh, FMT == Q6_K ? (uint64_t)N * (uint64_t)K / 4u : 0);
-    const uint32_t hoff = n2 < N ? (uint32_t)n2 * (uint32_t)(K / 4) + (uint32_t)(lane & 1) * 16u : kOob;
-    // Scale words into this wave's slot:
-    //  Q8_0, Q4_0: lane L: dword L % 2 of the unit's four fp16 d of row L / 2;
-    //  Q4_K: lane r < 32: row r's 16-byte superblock record;
-    //  Q6_K: lane L: dword L % 2 of the unit's eight int8 group scales of row L / 2; then lane
-    //        r < 32: the aligned dword holding row r's fp16 superblock d (the d section follows
-    //        the sc section in the matrix's allocation, so one buffer resource from sc to the end
-    //        of d's 256-byte-aligned section serves both).
     const int nsb = K / 256;
-    const uint32_t d_rel = FMT == Q6_K ? (uint32_t)(w.d - w.sc) : 0u;
-    const __amdgpu_buffer_rsrc_t sr =
-        make_rsrc(w.sc, FMT == Q6_K ? (uint64_t)d_rel + align256((uint64_t)N * (uint64_t)nsb * 2u)
-                                    : (uint64_t)N * (uint64_t)(K / 16));
-    uint32_t soff = kOob, doff = kOob;
-    if constexpr (FMT == Q4_K) {
-        if (lane < 32 && nw + lane < N) soff = (uint32_t)(nw + lane) * (uint32_t)(K / 16);
-    } else {
-        if (n2 < N) soff = (uint32_t)n2 * (uint32_t)(K / 16) + (uint32_t)(lane & 1) * 4u;
-        if (FMT == Q6_K && lane < 32 && nw + lane < N) doff = d_rel + (uint32_t)(nw + lane) * (uint32_t)(nsb * 2);
-    }
+    U unit;
+    unit.init(w, nw, wave, lane);
 
     // The loads of stage i of X, and of W unit u (stages 2 u and 2 u + 1).
     auto load_x = [&](int i, uint8_t *xb) __attribute__((always_inline)) {
@@ -166,27 +202,12 @@ gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, 
 #pragma unroll
         for (int j = 0; j < XL; j++) dma16(xr, xb + (WV * j + wave) * 1024, i < ns ? xoff[j] : kOob, so);
     };
-    auto load_w = [&](int u, uint8_t *wb) __attribute__((always_inline)) {
-        uint8_t *const slot = wb + T::kQ + T::kH + wave * T::kSlot;
-        const bool live = 2 * u < ns;
-        const uint32_t uu = live ? (uint32_t)u : 0u;
-#pragma unroll
-        for (int j = 0; j < QL; j++) dma16(qr, wb + (wave * QL + j) * 1024, live ? qoff[j] : kOob, uu * (uint32_t)QR);
-        if constexpr (FMT == Q6_K) {
-            dma16(hr, wb + T::kQ + wave * 1024, live ? hoff : kOob, uu * 32u);
-            dma4(sr, slot, live && soff != kOob ? soff + uu * 8u : kOob);
-            dma4(sr, slot + 256, live && doff != kOob ? (doff + (uu >> 1) * 2u) & ~3u : kOob);
-        } else if constexpr (FMT == Q4_K) {
-            if (lane < 32) dma16(sr, slot, live ? soff : kOob, (uu >> 1) * 16u);
-        } else {
-            dma4(sr, slot, live && soff != kOob ? soff + uu * 8u : kOob);
-        }
-    };
+    auto load_w = [&](int u, uint8_t *wb) __attribute__((always_inline)) { unit.load(u, 2 * u < ns, wb); };
 
     // One block of one W row as it lies in LDS; scale s and offset o of its elements 0..15 and
     // 16..31 (s carries the power of two of the codes' units).
     struct Raw {
-        u32x4 q[FMT == Q8_0 ? 2 : 1];
+        u32x4 q[U::QL / 2];
         u32x2 hi;
         u32x4 s;
     };
@@ -195,14 +216,15 @@ gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, 
     };
     // Stage j's block h of row r32, from its unit's buffer.
     auto read_raw = [&](int j, const uint8_t *wb, Raw &o) __attribute__((always_inline)) {
-        const int swz = qswz(r32), blk = 2 * (j & 1) + h;  // blk: block within the unit
-        const uint8_t *const row = wb + (32 * wave + r32) * QR, *const slot = wb + T::kQ + T::kH + wave * T::kSlot;
+        const int swz = U::swz(r32), blk = 2 * (j & 1) + h;  // blk: block within the unit
+        const uint8_t *const row = wb + (32 * wave + r32) * QR, *const slot = wb + U::kS + wave * U::kSlot;
 #pragma unroll
-        for (int c = 0; c < QL / 2; c++) o.q[c] = *reinterpret_cast<const u32x4 *>(row + (((QL / 2 * blk + c) ^ swz) << 4));
+        for (int c = 0; c < U::QL / 2; c++)
+            o.q[c] = *reinterpret_cast<const u32x4 *>(row + (((U::QL / 2 * blk + c) ^ swz) << 4));
         if constexpr (FMT == Q4_K) o.s = *reinterpret_cast<const u32x4 *>(slot + r32 * 16);
         else o.s[0] = *reinterpret_cast<const uint16_t *>(slot + r32 * 8 + blk * 2);
         if constexpr (FMT == Q6_K) {
-            o.hi = *reinterpret_cast<const u32x2 *>(wb + T::kQ + (32 * wave + r32) * 32 + blk * 8);
+            o.hi = *reinterpret_cast<const u32x2 *>(wb + U::kH + (32 * wave + r32) * 32 + blk * 8);
             o.s[1] = *reinterpret_cast<const uint32_t *>(slot + 256 + r32 * 4);
         }
     };
@@ -287,6 +309,8 @@ gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, 
         read_raw(i + 1, wc, raw[cur ^ 1]);
         load_x(i + 1, xn);
         if constexpr (S % 2 == 1) load_w((i + 3) / 2, wn);
+        // issue the loads first (not where that costs registers: Q6_K at 256 rows would spill)
+        if constexpr (TM < 8 || FMT != Q6_K) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int p = 0; p < 4; p++) {
             if (p < 3) read_a(xb, p + 1, a[(p + 1) & 1]);
@@ -309,11 +333,22 @@ gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, 
     read_raw(sbeg, ws0, raw[0]);
     decode_scale(sbeg, raw[0], sc[0]);
     b[0] = operand(raw[0], sc[0], 0);
-#define J4Q_STAGE(S)                            \
-    stage(std::integral_constant<int, S>{}, i); \
-    if (++i >= ns) break;
-    for (int i = sbeg;;) {
+    // Whole periods in the loop: with an exit between stages the compiler takes the loads in flight at
+    // the loop's head for any stage's, and waits there for all of them (2048 x 14336 x 4096 Q4_K 230 ->
+    // 228 us, 512 x 4096 x 4096 31.9 -> 30.8).
+#define J4Q_STAGE(S) stage(std::integral_constant<int, S>{}, i + S);
+    int i = sbeg;
+    for (; i + 4 <= ns; i += 4) {
         J4Q_STAGE(0) J4Q_STAGE(1) J4Q_STAGE(2) J4Q_STAGE(3)
+    }
+    if constexpr (FMT == Q8_0 || FMT == Q4_0) {
+        if (i < ns) {
+            J4Q_STAGE(0)
+            if (i + 1 < ns) {
+                J4Q_STAGE(1)
+                if (i + 2 < ns) J4Q_STAGE(2)
+            }
+        }
     }
 #undef J4Q_STAGE
     __builtin_amdgcn_s_waitcnt(0);  // no LDS load outlives the workgroup
