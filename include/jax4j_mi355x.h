@@ -163,8 +163,9 @@ int j4q_quant_gather_row(j4q_buffer weights, int64_t row, j4q_buffer *y);
 int j4q_quant_dequantize(j4q_buffer weights, j4q_buffer *y);
 /* Arithmetic of batched GEMV, x [B, cols] with B >= 3 (engine-local; the SPI's quantMatvec is
  * one row, CpuBackend.java:712, and the engine's batch is row b = quantMatvec of x[b]):
- *  J4Q_GEMV_MATRIX_CORES (default): launches of up to 16 batch rows on the matrix cores (Q8_0,
- *    Q4_0, Q4_K, Q6_K), W streamed once per launch; x enters the products as hi + lo fp16
+ *  J4Q_GEMV_MATRIX_CORES (default): launches of up to 16 batch rows, or tiles of 32 or 64 where
+ *    there are more (from 19 to 35 rows on, by type and cols), on the matrix cores (Q8_0, Q4_0,
+ *    Q4_K, Q6_K), W streamed once per launch or tile; x enters the products as hi + lo fp16
  *    (22 significant bits under a power-of-two scale), the products are exact, and each row
  *    stays within 1e-4 of the fp64 product (within 4e-5 up to K = 40960 in the tests);
  *  J4Q_GEMV_FP32: every batch row on the batch-1 kernel (fp32 x, fp32 accumulation, no

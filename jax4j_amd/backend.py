@@ -215,7 +215,7 @@ class Mi355xBackend:
 
     def set_gemv_policy(self, policy: str) -> str:
         """Arithmetic of batched GEMV (engine-local): "matrix_cores" (default; launches of up
-        to 16 batch rows, x as hi + lo fp16) or "fp32" (every row on the batch-1 kernel, equal
+        to 16 batch rows or tiles of 32 or 64, x as hi + lo fp16) or "fp32" (every row on the batch-1 kernel, equal
         bit for bit to quantMatvec of that row). Process-wide; returns the policy replaced."""
         names = {"matrix_cores": N.GEMV_MATRIX_CORES, "fp32": N.GEMV_FP32}
         if policy not in names:

@@ -4,6 +4,7 @@
 
 #include "gemv_impl.h"
 #include "gemv_mfma.h"
+#include "gemv_tile.h"
 #include "jax4j_mi355x.h"
 
 namespace j4q {
@@ -280,6 +281,107 @@ hipError_t launch_valu(int id, const QMat &m, const float *x, const float *add, 
     }
 }
 
+// ---- more rows than one launch of the 16-row kernel (gemv_tile.h) -------------------------
+// Rows of x per chunk, tile rows, K splits, and the workspace of a chunk: x as hi and lo fp16, its
+// scales and block sums, the K splits' partial sums.
+struct TileShape {
+    int rows = 0, tm = 1, splits = 1, split_stages = 0;
+    int64_t x_bytes = 0, scale_bytes = 0, sum_bytes = 0, bytes = 0;
+};
+
+constexpr int64_t kTileWorkspace = 256ll << 20;
+
+// The fewest rows that the tile kernel takes, against 16-row launches (which stream W once per 16
+// rows, and take 1 or 2 rows over with the fp32 kernel). Its own time hardly depends on the rows up
+// to 32 (4096 x 4096 Q8_0: 19 rows 16.8 us, 32 rows 18.0; two 16-row launches 19.9, 23.3), so it wins
+// where the second launch is more than a remainder: 19 rows. The 4-bit formats' 16-row kernel is the
+// faster one (4096 x 4096 Q4_K: 19 rows 15.7 us, 25 rows 18.5; tile kernel 17.2, 18.0), and with few
+// columns it needs fewer windows (2048 x 2048 Q4_K: 25 rows 12.0, 33 rows 15.4; tile kernel 13.7,
+// 15.8). A rule on W's columns and not its rows: the matrices of a fused launch are computed as
+// each of them alone.
+int tile_min_rows(int id, int64_t cols) {
+    if (id == Q8_0 || id == Q6_K) return 19;
+    return cols > 2048 ? 27 : 35;
+}
+
+bool tile_supported(int id, const QMat &m) {
+    const int64_t unit = id == Q8_0 ? 64 : id == Q4_0 ? 128 : id == Q4_K || id == Q6_K ? 256 : 0;
+    return unit && m.cols % unit == 0 && m.rows <= (id == Q8_0 ? 0x7fffffff : 0xffffffff) / m.cols;
+}
+
+TileShape tile_shape(int id, const QMat &m, int64_t batch) {
+    TileShape t;
+    if (batch < tile_min_rows(id, m.cols) || !tile_supported(id, m)) return t;
+    const int64_t K = m.cols, N = m.rows, stages = K / 64;
+    // K splits of a quarter of the columns, within 512 .. 1024 (28672 x 4096 Q4_K, 64 rows: 512 columns
+    // 78.2 us, 1024 66.7, as the partial sums halve; 4096 x 4096, 32 tiles: 24.5, 26.1; 1000 x 2048 Q6_K:
+    // 18.8, 24.2). W's rows have no say here either.
+    int per = (int)((stages / 4 + 3) / 4 * 4);
+    per = per < 8 ? 8 : per > 16 ? 16 : per;
+    const int64_t splits = (stages + per - 1) / per;
+    // Chunks of up to 256 rows, of fewer where the partial sums would pass kTileWorkspace.
+    const int64_t row_bytes = K * 4 + 4 + (id == Q4_K ? K / 8 : 0) + (splits > 1 ? splits * N * 4 : 0);
+    int64_t rows = batch < 256 ? batch : 256;
+    if (rows * row_bytes > kTileWorkspace) rows = kTileWorkspace / row_bytes;
+    if (rows < batch && rows > 32) rows = rows / 32 * 32;
+    if (rows < 1 || rows * K * 4 > 0x7fffffff) return t;
+    t.rows = (int)rows;
+    t.tm = rows <= 32 ? 1 : 2;
+    t.splits = (int)splits;
+    t.split_stages = per;
+    t.x_bytes = (int64_t)align256((uint64_t)(rows * K * 4));
+    t.scale_bytes = (int64_t)align256((uint64_t)rows * 4);
+    t.sum_bytes = id == Q4_K ? (int64_t)align256((uint64_t)(rows * (K / 32) * 4)) : 0;
+    t.bytes = t.x_bytes + t.scale_bytes + t.sum_bytes + (splits > 1 ? splits * rows * N * 4 : 0);
+    return t;
+}
+
+template <int FMT>
+hipError_t launch_tile_fmt(const QMat &m, const float *x, const float *add, float *y, int64_t batch, const TileShape &t,
+                           uint8_t *ws, hipStream_t s) {
+    const int K = (int)m.cols;
+    _Float16 *const hi = (_Float16 *)ws;
+    float *const unscale = (float *)(ws + t.x_bytes);
+    float *const sums = t.sum_bytes ? (float *)(ws + t.x_bytes + t.scale_bytes) : nullptr;
+    float *const part = t.splits > 1 ? (float *)(ws + t.x_bytes + t.scale_bytes + t.sum_bytes) : nullptr;
+    for (int64_t b0 = 0; b0 < batch; b0 += t.rows) {
+        const int rows = (int)(batch - b0 < t.rows ? batch - b0 : t.rows);
+        const float *const ab = add ? add + b0 * m.rows : nullptr;
+        float *const yb = y + b0 * m.rows;
+        if (K <= 8192) gvt::split_x_kernel<FMT != Q8_0, 2><<<rows, 1024, 0, s>>>(x + b0 * K, K, hi, (int64_t)rows * K, unscale, sums);
+        else gvt::split_x_kernel<FMT != Q8_0, 8><<<rows, 1024, 0, s>>>(x + b0 * K, K, hi, (int64_t)rows * K, unscale, sums);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        const unsigned tiles = (unsigned)(((rows + 32 * t.tm - 1) / (32 * t.tm)) * ((m.rows + 127) / 128));
+        const dim3 grid(tiles, (unsigned)t.splits);
+        const uint16_t *const xs = (const uint16_t *)ws;
+        if (t.tm == 1) gvt::gemv_tile<FMT, 1><<<grid, 256, 0, s>>>(m, xs, unscale, sums, ab, yb, rows, t.split_stages, part);
+        else gvt::gemv_tile<FMT, 2><<<grid, 256, 0, s>>>(m, xs, unscale, sums, ab, yb, rows, t.split_stages, part);
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        if (t.splits > 1) {
+            const int64_t n = (int64_t)rows * m.rows;
+            const int64_t blocks = ((n % 4 == 0 ? n / 4 : n) + 255) / 256;
+            gmf::sum_windows_kernel<<<(unsigned)(blocks < 2048 ? blocks : 2048), 256, 0, s>>>(part, t.splits, n, ab, yb);
+            e = hipGetLastError();
+            if (e != hipSuccess) return e;
+        }
+    }
+    return hipSuccess;
+}
+
+hipError_t launch_tile(int id, const QMat &m, const float *x, const float *add, float *y, int64_t batch, const TileShape &t,
+                       const Workspace &ws, hipStream_t s) {
+    uint8_t *const p = (uint8_t *)ws.ptr;
+    switch (id) {
+    case Q4_0: return launch_tile_fmt<Q4_0>(m, x, add, y, batch, t, p, s);
+    case Q4_K: return launch_tile_fmt<Q4_K>(m, x, add, y, batch, t, p, s);
+    case Q6_K: return launch_tile_fmt<Q6_K>(m, x, add, y, batch, t, p, s);
+    case Q8_0: return launch_tile_fmt<Q8_0>(m, x, add, y, batch, t, p, s);
+    default: return hipErrorInvalidValue;
+    }
+}
+
 }  // namespace
 
 void gemv_set_cus(int cus) {
@@ -307,6 +409,8 @@ bool gemv_in_place_ok(int id, const QMat &m, int64_t batch) {
 
 uint64_t gemv_workspace_bytes(int id, const QMat &m, int64_t batch) {
     if (m.rows <= 0 || !on_matrix_cores(id, m, batch)) return 0;
+    const TileShape t = tile_shape(id, m, batch);
+    if (t.rows) return (uint64_t)t.bytes;
     // launches of 16 rows and, for a remainder of 3..15 rows, one smaller launch
     uint64_t need = mfma_ws_any(id, m, (int)(batch < 16 ? batch : 16));
     const int64_t rem = batch % 16;
@@ -332,12 +436,16 @@ hipError_t launch_gemv(int id, const QMat &m, const float *x, const float *add, 
     // element before it writes y there; without it they are chained launches that would
     // read an add overlapping y after rewriting y, so such a call keeps one window
     const bool ws_ok = mfma && ws.ptr && ws.bytes >= gemv_workspace_bytes(id, m, batch);
+    if (ws_ok) {
+        const TileShape t = tile_shape(id, m, batch);
+        if (t.rows) return launch_tile(id, m, x, add, y, batch, t, ws, s);
+    }
     if (!mfma || (alias && !ws_ok && !single_window<8>(m))) {
         if (alias && m.cols > gemv::kMaxWindow) return hipErrorInvalidValue;
         return launch_valu(id, m, x, add, y, (int)batch, s);
     }
-    // batch rows in launches of up to 16 on the matrix cores (every launch streams W once for
-    // its rows); a remainder of 1 or 2 rows takes the vector-ALU kernel, which is as fast there.
+    // fewer rows than tile_min_rows, or no workspace for the tile kernel: batch rows in launches
+    // of up to 16 on the matrix cores (every launch streams W once for its rows); a remainder of 1 or 2 rows takes the vector-ALU kernel, which is as fast there.
     // Above one vector-ALU window (K > 32768) that kernel chains its windows through y, so an
     // add that is y itself would be read after the first window rewrote it: there the last
     // full launch gives up rows so that the remainder makes 3 and stays on the matrix cores
