@@ -955,6 +955,12 @@ namespace gw {
 //    with half the barriers ran 39.7 us at M = 512).
 // Requires K % 32 == 0, N % 8 == 0, M * K < 2^31 and N * K < 2^31. Internal linkage: this header
 // is included by more than one source.
+// 1.5 * 2^23, whose bits plus I (|I| < 2^22; a block's |I| <= 32 * 127^2) are the float 1.5 * 2^23 + I: the
+// products start from its bits, and a subtraction instead of the slower conversion gives (float)I
+// exactly (N = K = 4096: M = 300 29.5 -> 28.5 us, M = 2048 117 -> 114.5). The kernel is bound by its
+// fold: MFMA and vector instructions of two waves hardly overlap on a SIMD (16 us of the two at
+// M = 512, of 27).
+constexpr float kIntBias = 12582912.0f;
 [[maybe_unused]] static __global__ void __launch_bounds__(512)
 gemm_i8_lds(QMat w, const int8_t *__restrict__ xq, const float *__restrict__ xsc, float *__restrict__ y, int M) {
     constexpr int BM = 64, BN = 128, SB = 4;  // rows, columns, blocks per stage
@@ -1026,8 +1032,9 @@ gemm_i8_lds(QMat w, const int8_t *__restrict__ xq, const float *__restrict__ xsc
     // result element v: row 8 (v / 4) + 4 (lane / 32) + v % 4, column lane % 32
     auto fold = [&](const i32x16 &I, const f32x32 &Pr, int e) __attribute__((always_inline)) {
 #pragma unroll
-        for (int v = 0; v < 16; v++) acc[v] = __builtin_fmaf((float)I[v], Pr[16 * e + v], acc[v]);
+        for (int v = 0; v < 16; v++) acc[v] = __builtin_fmaf(__builtin_bit_cast(f32x16, I)[v] - kIntBias, Pr[16 * e + v], acc[v]);
     };
+    const i32x16 bias = __builtin_bit_cast(i32x16, f32x16{} + kIntBias);
     struct Pair {
         i32x16 I0, I1;
         f32x32 Pr;
@@ -1052,15 +1059,15 @@ gemm_i8_lds(QMat w, const int8_t *__restrict__ xq, const float *__restrict__ xsc
     // outer products (block 2 p in elements 0..15, 2 p + 1 in 16..31) in the layout of the
     // int8 products
     auto products = [&](const Ops &o, Pair &out) __attribute__((always_inline)) {
-        out.I0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.a0, o.b0, i32x16{}, 0, 0, 0);
-        out.I1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.a1, o.b1, i32x16{}, 0, 0, 0);
+        out.I0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.a0, o.b0, bias, 0, 0, 0);
+        out.I1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.a1, o.b1, bias, 0, 0, 0);
         out.Pr = __builtin_amdgcn_mfma_f32_32x32x1f32(o.sx, o.dw, f32x32{}, 0, 0, 0);
     };
     // pa: pair 0 of the current stage; pb: the pair left for folding (pair 1 of the stage
     // before; zeros before the first stage, whose fold adds exact zeros: fma(0, 0, +0) = +0)
     Pair pa, pb;
-    pb.I0 = i32x16{};
-    pb.I1 = i32x16{};
+    pb.I0 = bias;
+    pb.I1 = bias;
     pb.Pr = f32x32{};
     // One stage, each step fenced from the next: read pair 0's operands, fold block 0 of the
     // left pair (its latency covers the reads), pair 0's products, read pair 1's operands,
