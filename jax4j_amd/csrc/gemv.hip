@@ -133,6 +133,19 @@ constexpr int mfma_lds() {
                      gmf::round_tiles<BB, mfma_waves<FMT, BB>()>()>::kBytes;
 }
 
+// Workgroups per window: those resident at once, shared out between the windows; rounded down, since
+// a workgroup past the resident count would start only when another one ends and double the
+// launch's time (4096 x 14336 Q6_K at B = 16: 518 workgroups for 512 slots took 31 us).
+template <int FMT, int BB>
+int mfma_grid(const QMat &m, int windows) {
+    constexpr int lds = mfma_lds<FMT, BB>();
+    const int tiles = (int)((m.rows + 15) / 16);
+    const int measured = g_mfma_resident[fmt_slot(FMT)][bb_slot(BB)];
+    const int per_cu = measured > 0 ? measured : (163840 / lds > 0 ? 163840 / lds : 1);
+    const int grid = g_cus * (per_cu < 8 ? per_cu : 8) / windows;
+    return grid < 1 ? 1 : grid > tiles ? tiles : grid;
+}
+
 template <int FMT, int BB>
 void measure_resident() {
     constexpr int W = mfma_waves<FMT, BB>();
@@ -150,6 +163,12 @@ void measure_resident_fmt() {
     measure_resident<FMT, 16>();
 }
 
+hipError_t launch_sum(const float *part, int windows, int64_t n, const float *add, float *y, hipStream_t s) {
+    const int64_t blocks = ((n % 4 == 0 ? n / 4 : n) + 255) / 256;  // a thread per float4 where n allows
+    gmf::sum_windows_kernel<<<(unsigned)(blocks < 2048 ? blocks : 2048), 256, 0, s>>>(part, windows, n, add, y);
+    return hipGetLastError();
+}
+
 // Batched GEMV on the matrix cores (gemv_mfma.h) for up to 16 batch rows per launch,
 // persistent workgroups of 16-row tiles, each launch window of up to 128 blocks (4096
 // columns; 64 at 16 rows) split into one slice per wave. A wider K has several windows:
@@ -161,7 +180,7 @@ void measure_resident_fmt() {
 // the two are level.
 template <int FMT, int BB>
 hipError_t launch_mfma(const QMat &m, const float *x, const float *add, float *y, int b, const Workspace &ws,
-                       hipStream_t s) {
+                       hipStream_t s, const SumJob &in, SumJob *out) {
     constexpr int W = mfma_waves<FMT, BB>(), IPW = mfma_ipw<FMT, BB>(), S = FMT == Q8_0 ? 2 : 4;
     constexpr int CAP = mfma_window<FMT, BB>();
     static_assert(CAP == W * IPW * S && CAP == (BB > 8 ? 8 * W : 128), "window = waves x items per wave x blocks per item");
@@ -171,16 +190,7 @@ hipError_t launch_mfma(const QMat &m, const float *x, const float *add, float *y
     mfma_windows<FMT, BB>(m, windows, per);
     const uint64_t need = windows > 1 ? (uint64_t)windows * (uint64_t)b * (uint64_t)m.rows * 4u : 0;
     if (windows == 1 || (ws.ptr && ws.bytes >= need)) {
-        // workgroups resident at once, shared out between the windows; rounded down, since a
-        // workgroup past the resident count would start only when another one ends and double
-        // the launch's time (4096 x 14336 Q6_K at B = 16: 518 workgroups for 512 slots took
-        // 31 us)
-        constexpr int lds = mfma_lds<FMT, BB>();
-        const int measured = g_mfma_resident[fmt_slot(FMT)][bb_slot(BB)];
-        const int per_cu = measured > 0 ? measured : (163840 / lds > 0 ? 163840 / lds : 1);
-        int grid = g_cus * (per_cu < 8 ? per_cu : 8) / windows;
-        if (grid < 1) grid = 1;
-        if (grid > tiles) grid = tiles;
+        const int grid = mfma_grid<FMT, BB>(m, windows);
         // With rounds of 4 tiles (8 waves, up to 8 rows) and at 16 rows, workgroups with at
         // least one full round take the tile loop without skip paths: A/B on one box, decode
         // step B = 4 1.853 -> 1.818 ms, B = 8 2.110 -> 2.047 ms, B = 16 (with the prologue's
@@ -193,19 +203,23 @@ hipError_t launch_mfma(const QMat &m, const float *x, const float *add, float *y
         if constexpr (RT >= 4 || BB > 8) {
             if ((tiles + grid - 1) / grid >= RT)
                 e = gmf::launch_k<FMT, BB, W, IPW, false, mfma_ring<FMT, BB>(), true>(
-                    m, x, windows == 1 ? add : nullptr, y, b, grid, s, 0, per, nb, nullptr, windows, ws.ptr);
+                    m, x, windows == 1 ? add : nullptr, y, b, grid, s, 0, per, nb, nullptr, windows, ws.ptr, in);
             else
                 e = gmf::launch_k<FMT, BB, W, IPW, false, mfma_ring<FMT, BB>()>(
-                    m, x, windows == 1 ? add : nullptr, y, b, grid, s, 0, per, nb, nullptr, windows, ws.ptr);
+                    m, x, windows == 1 ? add : nullptr, y, b, grid, s, 0, per, nb, nullptr, windows, ws.ptr, in);
         } else {
             e = gmf::launch_k<FMT, BB, W, IPW, false, mfma_ring<FMT, BB>()>(m, x, windows == 1 ? add : nullptr, y, b, grid,
                                                                              s, 0, per, nb, nullptr, windows, ws.ptr);
         }
         if (e != hipSuccess || windows == 1) return e;
-        const int64_t n = (int64_t)b * m.rows;
-        const int64_t blocks = ((n % 4 == 0 ? n / 4 : n) + 255) / 256;  // a thread per float4 where n allows
-        gmf::sum_windows_kernel<<<(unsigned)(blocks < 2048 ? blocks : 2048), 256, 0, s>>>(ws.ptr, windows, n, add, y);
-        return hipGetLastError();
+        if (out && BB > 8 && !add) {
+            out->part = ws.ptr;
+            out->y = y;
+            out->windows = windows;
+            out->cols = out->pitch = (int)m.rows;
+            return hipSuccess;
+        }
+        return launch_sum(ws.ptr, windows, (int64_t)b * m.rows, add, y, s);
     }
     const int grid = tiles < g_cus ? tiles : g_cus;
     for (int kb0 = 0; kb0 < nb; kb0 += per) {
@@ -220,10 +234,10 @@ hipError_t launch_mfma(const QMat &m, const float *x, const float *add, float *y
 
 template <int FMT>
 hipError_t launch_mfma_fmt(const QMat &m, const float *x, const float *add, float *y, int b, const Workspace &ws,
-                           hipStream_t s) {
-    if (b <= 4) return launch_mfma<FMT, 4>(m, x, add, y, b, ws, s);
-    if (b <= 8) return launch_mfma<FMT, 8>(m, x, add, y, b, ws, s);
-    return launch_mfma<FMT, 16>(m, x, add, y, b, ws, s);
+                           hipStream_t s, const SumJob &in, SumJob *out) {
+    if (b <= 4) return launch_mfma<FMT, 4>(m, x, add, y, b, ws, s, in, out);
+    if (b <= 8) return launch_mfma<FMT, 8>(m, x, add, y, b, ws, s, in, out);
+    return launch_mfma<FMT, 16>(m, x, add, y, b, ws, s, in, out);
 }
 
 template <int FMT>
@@ -260,12 +274,12 @@ bool mfma_format(int id, const QMat &m) {
 }
 
 hipError_t launch_mfma_any(int id, const QMat &m, const float *x, const float *add, float *y, int b, const Workspace &ws,
-                           hipStream_t s) {
+                           hipStream_t s, const SumJob &in, SumJob *out) {
     switch (id) {
-    case Q4_0: return launch_mfma_fmt<Q4_0>(m, x, add, y, b, ws, s);
-    case Q4_K: return launch_mfma_fmt<Q4_K>(m, x, add, y, b, ws, s);
-    case Q6_K: return launch_mfma_fmt<Q6_K>(m, x, add, y, b, ws, s);
-    case Q8_0: return launch_mfma_fmt<Q8_0>(m, x, add, y, b, ws, s);
+    case Q4_0: return launch_mfma_fmt<Q4_0>(m, x, add, y, b, ws, s, in, out);
+    case Q4_K: return launch_mfma_fmt<Q4_K>(m, x, add, y, b, ws, s, in, out);
+    case Q6_K: return launch_mfma_fmt<Q6_K>(m, x, add, y, b, ws, s, in, out);
+    case Q8_0: return launch_mfma_fmt<Q8_0>(m, x, add, y, b, ws, s, in, out);
     default: return hipErrorInvalidValue;
     }
 }
@@ -360,10 +374,7 @@ hipError_t launch_tile_fmt(const QMat &m, const float *x, const float *add, floa
         e = hipGetLastError();
         if (e != hipSuccess) return e;
         if (t.splits > 1) {
-            const int64_t n = (int64_t)rows * m.rows;
-            const int64_t blocks = ((n % 4 == 0 ? n / 4 : n) + 255) / 256;
-            gmf::sum_windows_kernel<<<(unsigned)(blocks < 2048 ? blocks : 2048), 256, 0, s>>>(part, t.splits, n, ab, yb);
-            e = hipGetLastError();
+            e = launch_sum(part, t.splits, (int64_t)rows * m.rows, ab, yb, s);
             if (e != hipSuccess) return e;
         }
     }
@@ -426,8 +437,35 @@ uint64_t gemv_workspace_bytes(int id, const QMat &m, int64_t batch) {
     return need;
 }
 
+// Threads of the 16-row launch, which takes along one float4 of a job each.
+template <int FMT>
+int64_t carry_threads(const QMat &m) {
+    int windows, per;
+    mfma_windows<FMT, 16>(m, windows, per);
+    return (int64_t)mfma_grid<FMT, 16>(m, windows) * windows * mfma_waves<FMT, 16>() * 64;
+}
+
+bool gemv_carries(int id, const QMat &m, int64_t batch, const SumJob &job) {
+    if (m.rows <= 0 || batch < 9 || batch > 16 || !on_matrix_cores(id, m, batch)) return false;
+    if (job.windows > SumJob::kWindows || job.cols % 4 || job.pitch % 4 || (((uintptr_t)job.part | (uintptr_t)job.y) & 15u) ||
+        (int64_t)job.windows * batch * job.cols * 4 > 0x7fffffff || batch * job.pitch * 4 > 0x7fffffff)
+        return false;
+    const int64_t need = batch * job.cols / 4;
+    switch (id) {
+    case Q4_0: return need <= carry_threads<Q4_0>(m);
+    case Q4_K: return need <= carry_threads<Q4_K>(m);
+    case Q6_K: return need <= carry_threads<Q6_K>(m);
+    case Q8_0: return need <= carry_threads<Q8_0>(m);
+    default: return false;
+    }
+}
+
+hipError_t launch_sum_job(const SumJob &job, int64_t batch, hipStream_t s) {
+    return launch_sum(job.part, job.windows, batch * job.cols, nullptr, job.y, s);
+}
+
 hipError_t launch_gemv(int id, const QMat &m, const float *x, const float *add, float *y, int64_t batch,
-                       hipStream_t s, const Workspace &ws) {
+                       hipStream_t s, const Workspace &ws, const SumJob &in, SumJob *out) {
     if (m.rows <= 0 || batch <= 0) return hipSuccess;
     if (batch > 65535 || m.rows > (1 << 30) || m.cols > 0x7fffffff) return hipErrorInvalidValue;
     const bool alias = add && add < y + batch * m.rows && y < add + batch * m.rows;
@@ -436,6 +474,8 @@ hipError_t launch_gemv(int id, const QMat &m, const float *x, const float *add, 
     // element before it writes y there; without it they are chained launches that would
     // read an add overlapping y after rewriting y, so such a call keeps one window
     const bool ws_ok = mfma && ws.ptr && ws.bytes >= gemv_workspace_bytes(id, m, batch);
+    if (in.part && !(gemv_carries(id, m, batch, in) && (ws_ok || gemv_workspace_bytes(id, m, batch) == 0)))
+        return hipErrorInvalidValue;
     if (ws_ok) {
         const TileShape t = tile_shape(id, m, batch);
         if (t.rows) return launch_tile(id, m, x, add, y, batch, t, ws, s);
@@ -460,7 +500,8 @@ hipError_t launch_gemv(int id, const QMat &m, const float *x, const float *add, 
         const float *xb = x + b0 * m.cols;
         const float *ab = add ? add + b0 * m.rows : nullptr;
         float *yb = y + b0 * m.rows;
-        const hipError_t e = nb >= 3 ? launch_mfma_any(id, m, xb, ab, yb, (int)nb, ws_ok ? ws : Workspace(), s)
+        const hipError_t e = nb >= 3 ? launch_mfma_any(id, m, xb, ab, yb, (int)nb, ws_ok ? ws : Workspace(), s, in,
+                                                     batch <= cap ? out : nullptr)
                                      : launch_valu(id, m, xb, ab, yb, (int)nb, s);
         if (e != hipSuccess) return e;
         b0 += nb;

@@ -213,7 +213,7 @@ __device__ __forceinline__ void set_prio(int p) {
 template <int FMT, int BB, int WAVES, int IPW, bool XREG, int TS, bool NB = false>
 __global__ void __launch_bounds__(WAVES * 64)
 gemv_mfma_kernel(QMat m, const float *__restrict__ x, const float *prev, const float *__restrict__ add, float *y,
-                 int B, int kb0, int per, int nbe, float *__restrict__ wsum) {
+                 int B, int kb0, int per, int nbe, float *__restrict__ wsum, SumJob job) {
     kb0 += (int)blockIdx.y * per;
     const int kbn = nbe - kb0 < per ? nbe - kb0 : per;
     if (wsum) {
@@ -253,6 +253,23 @@ gemv_mfma_kernel(QMat m, const float *__restrict__ x, const float *prev, const f
     constexpr int XPL = (NBW * UNITS + 63) / 64;  // units per lane
     const int xb = (lane % UNITS) >> 2, xg = lane & 3;  // the batch row and lane group of this lane's units
     f32x4 xv[XPL][2];
+    // The window sums of an earlier launch (9..16 rows): a thread per 4 of them, loaded ahead of x and
+    // stored behind the weight loads, so that they cost neither a launch nor a wait of their own.
+    // Without a job its buffers are empty: loads give zeros, the store is dropped.
+    f32x4 jv[W16 ? SumJob::kWindows : 1];
+    uint32_t jo = 0;
+    if constexpr (W16) {
+        const uint32_t c4 = (uint32_t)job.cols / 4u;
+        const uint32_t i = ((uint32_t)blockIdx.y * gridDim.x + blockIdx.x) * (uint32_t)(WAVES * 64) + threadIdx.x;
+        const uint32_t row = c4 ? i / c4 : 0u;
+        const bool ok = i < (uint32_t)B * c4;
+        const uint32_t n = (uint32_t)B * (uint32_t)job.cols * 4u;  // bytes per window
+        const __amdgpu_buffer_rsrc_t jr = make_rsrc(job.part, (uint64_t)n * (uint32_t)job.windows);
+#pragma unroll
+        for (int r = 0; r < SumJob::kWindows; r++)
+            jv[r] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(jr, ok && r < job.windows ? i * 16u + r * n : kOob, 0, 0));
+        jo = ok ? (row * (uint32_t)job.pitch + (i - row * c4) * 4u) * 4u : kOob;
+    }
     {
         const __amdgpu_buffer_rsrc_t xr = make_rsrc(x, (uint64_t)B * (uint64_t)K * 4u);
 #pragma unroll
@@ -327,6 +344,14 @@ gemv_mfma_kernel(QMat m, const float *__restrict__ x, const float *prev, const f
         if constexpr (NB) __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (!NB) __builtin_amdgcn_sched_barrier(0);
+    if constexpr (W16) {  // in window order, as sum_windows_kernel
+        f32x4 v = jv[0];
+#pragma unroll
+        for (int r = 1; r < SumJob::kWindows; r++) v = r < job.windows ? v + jv[r] : v;
+        typedef uint32_t u32x4j __attribute__((ext_vector_type(4)));
+        const __amdgpu_buffer_rsrc_t yr = make_rsrc(job.y, job.part ? (uint64_t)B * (uint64_t)job.pitch * 4u : 0);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4j, v), yr, jo, 0, 0);
+    }
     // zero block for the A rows and C inputs that carry no batch row (every wave writes the
     // same zeros, so no wave depends on another)
     if constexpr (!W16)
@@ -709,13 +734,13 @@ gemv_mfma_kernel(QMat m, const float *__restrict__ x, const float *prev, const f
 // workgroups each; several windows need `part` (windows x B x rows floats).
 template <int FMT, int BB, int WAVES, int IPW, bool XREG, int TS = 2, bool NB = false>
 hipError_t launch_k(const QMat &m, const float *x, const float *add, float *y, int B, int grid, hipStream_t s, int kb0,
-                    int per, int nbe, const float *prev, int windows, float *part) {
+                    int per, int nbe, const float *prev, int windows, float *part, const SumJob &job = SumJob()) {
     constexpr int NBW = IPW * Fmt<FMT>::S;
     constexpr int lds = Plan<BB, Fmt<FMT>::GROUPS, WAVES, NBW, round_tiles<BB, WAVES>()>::kBytes;
     static_assert(lds <= 160 * 1024, "LDS of one workgroup");
     if (windows > 1 && !part) return hipErrorInvalidValue;
     gemv_mfma_kernel<FMT, BB, WAVES, IPW, XREG, TS, NB><<<dim3(grid, windows), WAVES * 64, lds, s>>>(
-        m, x, prev, add, y, B, kb0, per, nbe, windows > 1 ? part : nullptr);
+        m, x, prev, add, y, B, kb0, per, nbe, windows > 1 ? part : nullptr, job);
     return hipGetLastError();
 }
 

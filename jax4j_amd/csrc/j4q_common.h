@@ -129,6 +129,16 @@ struct Workspace {
     float *ptr = nullptr;
     uint64_t bytes = 0;
 };
+
+// The window sums that a batched GEMV left in its workspace: y[b * pitch + c] = sum over the windows,
+// in their order, of part[window][b][c], c < cols. A later GEMV of the same batch can compute them on
+// the way (gemv_carries), or launch_sum_job.
+struct SumJob {
+    static constexpr int kWindows = 4;  // the most that a GEMV takes along
+    const float *part = nullptr;
+    float *y = nullptr;
+    int windows = 0, cols = 0, pitch = 0;
+};
 // Bytes of workspace a batched GEMV of `batch` rows uses to run all its column windows in one
 // launch (0 when it has one window, or does not run on the matrix cores). With less, the
 // windows run one launch after another.
@@ -141,7 +151,11 @@ bool gemv_in_place_ok(int id, const QMat &m, int64_t batch);
 void gemv_set_policy(int policy);
 int gemv_policy();
 hipError_t launch_gemv(int id, const QMat &m, const float *x, const float *add, float *y, int64_t batch,
-                       hipStream_t s, const Workspace &ws = Workspace());
+                       hipStream_t s, const Workspace &ws = Workspace(), const SumJob &in = SumJob(), SumJob *out = nullptr);
+// Whether launch_gemv of these arguments takes the job along (with a workspace of the size asked for).
+bool gemv_carries(int id, const QMat &m, int64_t batch, const SumJob &job);
+// The job (pitch == cols) as a launch of its own.
+hipError_t launch_sum_job(const SumJob &job, int64_t batch, hipStream_t s);
 hipError_t launch_quantize_act(const uint16_t *x, int64_t m, int64_t k, int8_t *q, float *scales,
                                hipStream_t s);
 hipError_t launch_gemm_q8_int8(const QMat &w, const int8_t *xq, const float *xs, float *y, int64_t m,

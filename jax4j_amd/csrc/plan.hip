@@ -49,6 +49,7 @@ struct Op {
     QMat m;
     const float *x, *add;
     float *y;
+    bool last;  // no later launch of the step reads y (but a row copy right behind)
     // row copy
     float *dst;
     int64_t dst_pitch, cols;
@@ -58,7 +59,9 @@ struct Op {
 struct Plan {
     j4q_decode_plan_desc desc{};
     int64_t batch = 0;
-    Workspace ws;  // partial sums of batched GEMVs over several column windows (plan-owned)
+    // partial sums of batched GEMVs over several column windows (plan-owned): two, since those of a
+    // launch may stay until the next one has its own
+    Workspace ws[2];
     std::vector<Op> ops;
     std::vector<void *> owned;
     // caller buffers whose memory the graph reads (o, down, the head, and group parts that were
@@ -74,21 +77,59 @@ struct Plan {
 
 std::vector<Plan> g_plans;
 
+bool apart(const void *a, int64_t na, const void *b, int64_t nb) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return !a || !b || x + (uintptr_t)na <= y || y + (uintptr_t)nb <= x;
+}
+
+// Whether the launch of o may compute the job on its way: it neither reads nor writes what the job
+// writes (the caller's buffers may overlap).
+bool takes_along(const Op &o, const SumJob &job, int64_t batch) {
+    const int64_t n = (batch - 1) * job.pitch * 4 + (int64_t)job.cols * 4, yn = batch * o.m.rows * 4;
+    return o.gemv && gemv_carries(o.qt, o.m, batch, job) && apart(job.y, n, o.x, batch * o.m.cols * 4) &&
+           apart(job.y, n, o.add, yn) && apart(job.y, n, o.y, yn);
+}
+
+// At 9..16 rows every GEMV of several windows ended in a launch of sum_windows_kernel (4.7 us and the
+// gap; a 4096 x 14336 layer at 16 rows had 20 us of them in 77). The sums of q|k|v and of gate|up,
+// which no later GEMV of the step reads, ride on the next launch instead; with parts of different
+// types they go to their place in the group at once, and the row copy falls away
+// (step of 16 rows, 32 layers of 4096 x 14336 in Q4_K and Q6_K: 2162 -> 2060 us).
 hipError_t enqueue(const Plan &p, hipStream_t s) {
-    for (const Op &o : p.ops) {
-        hipError_t e;
+    SumJob job;  // left by the last GEMV
+    int w = 0;
+    hipError_t e = hipSuccess;
+    for (size_t i = 0; i < p.ops.size() && e == hipSuccess; i++) {
+        const Op &o = p.ops[i];
+        if (!o.gemv && job.part && job.y == o.src && i + 1 < p.ops.size()) {
+            SumJob placed = job;
+            placed.y = o.dst;
+            placed.pitch = (int)o.dst_pitch;
+            if (takes_along(p.ops[i + 1], placed, p.batch)) {
+                job = placed;
+                continue;
+            }
+        }
+        const bool along = job.part && takes_along(o, job, p.batch);
+        if (job.part && !along) {
+            e = launch_sum_job(job, p.batch, s);
+            if (e != hipSuccess) return e;
+        }
         if (o.gemv) {
-            e = launch_gemv(o.qt, o.m, o.x, o.add, o.y, p.batch, s, p.ws);
+            SumJob left;
+            e = launch_gemv(o.qt, o.m, o.x, o.add, o.y, p.batch, s, p.ws[w], along ? job : SumJob(), o.last ? &left : nullptr);
+            if (left.part) w ^= 1;
+            job = left;
         } else {
+            job = SumJob();
             const int64_t n = o.cols * p.batch;
             const int64_t blocks = (n + 255) / 256;
             copy_rows_kernel<<<(unsigned)(blocks < 1024 ? blocks : 1024), 256, 0, s>>>(o.dst, o.dst_pitch, o.src, o.cols,
                                                                                    p.batch);
             e = hipGetLastError();
         }
-        if (e != hipSuccess) return e;
     }
-    return hipSuccess;
+    return e == hipSuccess && job.part ? launch_sum_job(job, p.batch, s) : e;
 }
 
 void free_plan(Plan &p) {
@@ -142,6 +183,7 @@ int build_group(Plan &p, const j4q_buffer *parts, int count, const char *what, c
         g.qt = run.qtype;
         g.m = run.m;
         g.x = x;
+        g.last = true;
         if (run.rows == group_rows || p.batch == 1) {
             g.y = out + row0;
             p.ops.push_back(g);
@@ -280,15 +322,18 @@ int j4q_decode_plan_create(const j4q_decode_layer *layers, int32_t n_layers, j4q
         if (b > wsb) wsb = b;
     }
     if (!rc && wsb) {
+        const int n = batch >= 9 && batch <= 16 ? 2 : 1;
         void *d = nullptr;
-        e = abi::malloc_locked(&d, wsb);
+        e = abi::malloc_locked(&d, n * align256(wsb));
         if (e != hipSuccess) {
             rc = report_hip("decode plan workspace", e);
         } else {
             p.owned.push_back(d);
-            p.ws.ptr = (float *)d;
-            p.ws.bytes = wsb;
-            p.desc.plan_bytes += wsb;
+            for (int i = 0; i < 2; i++) {
+                p.ws[i].ptr = (float *)((uint8_t *)d + (i < n ? i * align256(wsb) : 0));
+                p.ws[i].bytes = wsb;
+            }
+            p.desc.plan_bytes += n * align256(wsb);
         }
     }
     if (rc) {
