@@ -5,7 +5,7 @@
 // vector instructions per 16 x 256 weights). Here the unpacked codes of a 32 x 32 block feed the
 // products of up to 64 rows. Measured (us, 16-row launches -> this): 61 rows Q6_K 4096 x 14336 83.4 ->
 // 42.7 (35 the tile kernel, 5 each the split of x and the sum of the K splits), Q4_K 4096 x 4096 36.9
-// -> 26.1, 64 rows Q4_K 28672 x 4096 97 -> 67, 256 rows Q4_K 4096 x 4096 153 -> 39, 48 rows Q8_0
+// -> 21.5, 64 rows Q4_K 28672 x 4096 97 -> 67, 256 rows Q4_K 4096 x 4096 153 -> 39, 48 rows Q8_0
 // 11008 x 4096 54.5 -> 32.5. The tile kernel is bound by no one unit: at 64 x 28672 x 4096 the matrix
 // cores are busy 18 of 61 us, the vector units about 20, and the two waves of a SIMD overlap them
 // only in part; without its loads it takes 45.

@@ -33,16 +33,17 @@ def matvec(backend, w, xs):
     return out
 
 
-# Rows of x at the first of each rule, full and ragged tiles of 32 and 64, and past a chunk of 256;
+# Rows of x at the first of each rule, full and ragged tiles of 32 and (the last two, and 65 x 20001)
+# of 64, and past a chunk of 256;
 # rows of W around a tile of 128; K of one split (512), of unequal splits (768: 512 + 256; 5120: 5 of
 # 1024; 2816: 768 three times and 512), of x rows kept in 2 (to 8192) and 8 (to 32768) groups and past
 # them (33024).
 SHAPES = [(19, 129, 512), (27, 127, 5120), (32, 300, 768), (33, 1, 2816), (35, 257, 2048), (64, 128, 512),
-          (65, 130, 768), (257, 70, 512), (35, 40, 9216), (36, 33, 33024)]
+          (65, 130, 768), (257, 70, 512), (35, 40, 9216), (36, 33, 33024), (257, 12500, 512), (130, 5001, 2816)]
 
 
 @pytest.mark.parametrize("qt", ALL, ids=lambda q: q.name)
-@pytest.mark.parametrize("b,n,k", SHAPES + [(19, 65, 64), (20, 140, 576), (40, 129, 1088), (70, 20, 640)])
+@pytest.mark.parametrize("b,n,k", SHAPES + [(19, 65, 64), (20, 140, 576), (40, 129, 1088), (70, 20, 640), (65, 20001, 576)])
 def test_gemv_tiles_match_oracle(backend, qt, b, n, k):
     if k % (64 if qt is QuantType.Q8_0 else 128 if qt is QuantType.Q4_0 else 256):
         pytest.skip("K of a whole number of blocks of the split layout")
