@@ -24,7 +24,7 @@
  *    (NULL = the engine stream) and return without synchronising.
  *  - Buffers returned through a j4q_buffer* are owned by the engine until j4q_release. The engine
  *    keeps released blocks of dense buffers (up to 4 MiB each, 64 MiB in all; not of a buffer
- *    whose address j4q_buffer_info has given out) and one workspace of its stream (up to 64 MiB)
+ *    whose address j4q_buffer_info has given out) and one workspace of its stream (up to 256 MiB)
  *    for later calls, and gives them back when the last buffer is released or memory is short.
  */
 #ifndef JAX4J_MI355X_H
@@ -195,9 +195,10 @@ int j4q_quant_matmul(j4q_buffer weights, j4q_buffer x, int variant, j4q_buffer *
  * itself (a residual updated in place) for cols <= 32768, or at batch >= 3 on Q4_0, Q8_0,
  * Q4_K and Q6_K; other adds overlapping y return J4Q_EUNSUPPORTED (column windows chained
  * one after another would read it after rewriting y). A batched call over several column
- * windows keeps their partial sums (batch x rows x windows floats) in the engine's kept
- * workspace on the engine stream, up to 64 MiB, else in stream-ordered memory of `stream`
- * (hipMallocAsync / hipFreeAsync); nothing else is allocated. */
+ * windows keeps their partial sums (batch x rows x windows floats), and one above 18 to 34 rows
+ * (by type and cols) also x in 4 bytes an element, in the engine's kept workspace on the engine
+ * stream, up to 256 MiB, else in stream-ordered memory of `stream` (hipMallocAsync /
+ * hipFreeAsync); nothing else is allocated. */
 int j4q_quant_matvec_into(j4q_buffer weights, const float *x_dev, const float *add_dev, float *y_dev,
                           int64_t batch, void *stream);
 /* Prefill GEMM into caller memory (the weight types and variants of j4q_quant_matmul).

@@ -65,7 +65,7 @@ thread_local std::string t_err;
 //    most 64 MiB in all: work on such a buffer runs on the engine stream alone, so its block may
 //    be written again behind it with no wait. A buffer whose address left the engine
 //    (j4q_buffer_info) can be in use on other streams and goes back with hipFree, which waits.
-//  - One workspace of at most 64 MiB for calls on the engine stream (which run one after another);
+//  - One workspace of at most 256 MiB for calls on the engine stream (which run one after another);
 //    calls on other streams take stream-ordered memory.
 //  - Neither serves a call under stream capture: a graph keeps the addresses it recorded.
 // All of it is given back when the last buffer is released.
@@ -100,7 +100,7 @@ struct BlockCache {
     }
 };
 BlockCache g_cache;
-constexpr uint64_t kMaxKeptWorkspace = 64ull << 20;
+constexpr uint64_t kMaxKeptWorkspace = 256ull << 20;
 void *g_kept_ws = nullptr;
 uint64_t g_kept_ws_bytes = 0;
 int64_t g_live = 0;  // live buffers
@@ -960,14 +960,18 @@ int j4q_quant_matvec_into(j4q_buffer wh, const float *x, const float *add, float
                     (long long)j4q::gemv_single_pass_cols(), (long long)K, (long long)batch);
     if ((rc = ensure_ready())) return rc;
     const hipStream_t s = pick_stream(stream);
-    // partial sums of several column windows live in stream-ordered memory of the call's stream
+    // partial sums live in the kept workspace or in stream-ordered memory of the call's stream; if
+    // there is none to be had, the batch runs without
     j4q::Workspace ws;
     const uint64_t wsb = j4q::gemv_workspace_bytes(w->qtype, m, batch);
     if (wsb) {
         void *p = nullptr;
-        HIP_TRY("hipMallocAsync", begin_workspace(s, wsb, &p));
-        ws.ptr = (float *)p;
-        ws.bytes = wsb;
+        if (begin_workspace(s, wsb, &p) == hipSuccess) {
+            ws.ptr = (float *)p;
+            ws.bytes = wsb;
+        } else {
+            (void)hipGetLastError();
+        }
     }
     const hipError_t e = j4q::launch_gemv(w->qtype, m, x, add, y, batch, s, ws);
     end_workspace(s, ws.ptr);

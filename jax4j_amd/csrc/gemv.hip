@@ -303,7 +303,7 @@ struct TileShape {
     int64_t x_bytes = 0, scale_bytes = 0, sum_bytes = 0, bytes = 0;
 };
 
-constexpr int64_t kTileWorkspace = 256ll << 20;
+constexpr int64_t kTileWorkspace = (256ll << 20) - 4096;  // within what the engine keeps, alignment included
 
 // The fewest rows that the tile kernel takes, against 16-row launches (which stream W once per 16
 // rows, and take 1 or 2 rows over with the fp32 kernel). Its own time hardly depends on the rows up

@@ -33,6 +33,8 @@
 // flight while a tile is computed.
 #pragma once
 
+#include <type_traits>
+
 #include "gemv_impl.h"
 
 namespace j4q {
@@ -202,6 +204,11 @@ constexpr int round_tiles() { return BB <= 8 && WAVES <= 8 ? 4 : 2; }
 // of 8, so every slice starts on a superblock), kbn <= WAVES * NBW and B <= BB. XREG keeps
 // the wave's A operands and C inputs in registers for the whole kernel instead of
 // re-reading them from LDS per tile.
+// The job argument of the kernel: none at up to 8 rows, whose windows are few.
+struct NoJob {};
+template <int BB>
+using JobArg = std::conditional_t<BB == 16, SumJob, NoJob>;
+
 // Wave priority p (0..3; s_setprio takes an immediate, so p must fold to a constant).
 __device__ __forceinline__ void set_prio(int p) {
     if (p >= 3) __builtin_amdgcn_s_setprio(3);
@@ -213,7 +220,7 @@ __device__ __forceinline__ void set_prio(int p) {
 template <int FMT, int BB, int WAVES, int IPW, bool XREG, int TS, bool NB = false>
 __global__ void __launch_bounds__(WAVES * 64)
 gemv_mfma_kernel(QMat m, const float *__restrict__ x, const float *prev, const float *__restrict__ add, float *y,
-                 int B, int kb0, int per, int nbe, float *__restrict__ wsum, SumJob job) {
+                 int B, int kb0, int per, int nbe, float *__restrict__ wsum, JobArg<BB> job) {
     kb0 += (int)blockIdx.y * per;
     const int kbn = nbe - kb0 < per ? nbe - kb0 : per;
     if (wsum) {
@@ -739,8 +746,10 @@ hipError_t launch_k(const QMat &m, const float *x, const float *add, float *y, i
     constexpr int lds = Plan<BB, Fmt<FMT>::GROUPS, WAVES, NBW, round_tiles<BB, WAVES>()>::kBytes;
     static_assert(lds <= 160 * 1024, "LDS of one workgroup");
     if (windows > 1 && !part) return hipErrorInvalidValue;
+    JobArg<BB> arg;
+    if constexpr (BB == 16) arg = job;
     gemv_mfma_kernel<FMT, BB, WAVES, IPW, XREG, TS, NB><<<dim3(grid, windows), WAVES * 64, lds, s>>>(
-        m, x, prev, add, y, B, kb0, per, nbe, windows > 1 ? part : nullptr, job);
+        m, x, prev, add, y, B, kb0, per, nbe, windows > 1 ? part : nullptr, arg);
     return hipGetLastError();
 }
 

@@ -124,7 +124,8 @@ hipError_t launch_export(int id, const uint8_t *split, uint8_t *gguf, int64_t ro
                          hipStream_t s);
 hipError_t launch_dequant_rows(int id, const QMat &m, int64_t row0, int64_t nrows, float *out,
                                hipStream_t s);
-// Device scratch a batched GEMV may use for the partial sums of its column windows.
+// Device scratch a batched GEMV may use: the partial sums of its column windows or K splits, and in
+// the tile kernel x as fp16.
 struct Workspace {
     float *ptr = nullptr;
     uint64_t bytes = 0;
@@ -140,8 +141,8 @@ struct SumJob {
     int windows = 0, cols = 0, pitch = 0;
 };
 // Bytes of workspace a batched GEMV of `batch` rows uses to run all its column windows in one
-// launch (0 when it has one window, or does not run on the matrix cores). With less, the
-// windows run one launch after another.
+// launch, or to take the tile kernel (0 when it has one window, or does not run on the matrix
+// cores). With less, launches of 16 rows run, window by window.
 uint64_t gemv_workspace_bytes(int id, const QMat &m, int64_t batch);
 // Whether an add that overlaps y is served for this matrix and batch (given the workspace
 // gemv_workspace_bytes asks for): one column window, or the matrix-core path.
