@@ -157,18 +157,22 @@ struct Tile {
     static_assert(2 * (kX + WUnit<FMT, WV>::kBytes) <= 163840, "LDS");
 };
 
-template <int FMT, int WV, int TM>
-__global__ void __launch_bounds__(64 * WV, 2)
+// KG = 2: two groups of WV waves, each with buffers of its own, take a half of the range of K each
+// (split_stages, a multiple of 4; K a multiple of 256), and the second's sums go to the first through LDS.
+template <int FMT, int WV, int TM, int KG = 1>
+__global__ void __launch_bounds__(64 * WV * KG, 2)
 gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, int split_stages,
           float *__restrict__ part) {
     using T = Tile<FMT, WV, TM>;
     using U = WUnit<FMT, WV>;
     constexpr int BM = T::BM, BN = T::BN, QR = U::QR, WL = U::kLoads, XL = T::XL;
-    __shared__ __attribute__((aligned(1024))) uint8_t xs0[T::kX], xs1[T::kX];
-    __shared__ __attribute__((aligned(1024))) uint8_t ws0[U::kBytes], ws1[U::kBytes];
+    __shared__ __attribute__((aligned(1024))) uint8_t xs0[KG * T::kX], xs1[KG * T::kX];
+    __shared__ __attribute__((aligned(1024))) uint8_t ws0[KG * U::kBytes], ws1[KG * U::kBytes];
     const int N = (int)w.rows, K = (int)w.cols;
-    const int sbeg = (int)blockIdx.y * split_stages, send = sbeg + split_stages, all = K / 64;
+    const int kg = KG > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / (64 * WV)) : 0;  // K group
+    const int sbeg = ((int)blockIdx.y * KG + kg) * split_stages, send = sbeg + split_stages, all = K / 64;
     const int ns = send < all ? send : all;  // stages [sbeg, ns)
+    const int nl = KG > 1 ? send : ns;       // K groups run the same number (zeros past ns), for the barriers
     // Workgroup b runs on XCD b % 8, and each XCD takes a contiguous range of tiles. Tiles go
     // down groups of 4 row tiles (a row tile's X costs about twice a column tile's W), so the
     // tiles that one XCD runs at a time share both in its L2.
@@ -179,7 +183,7 @@ gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, 
     const int m0 = (4 * mg + rem % gm) * BM, n0 = (rem / gm) * BN;
 
     const int lane = (int)threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) % WV;
     const int r32 = lane & 31, h = lane >> 5;
 
     // X load j of this wave fills rows 8 (WV j + wave) .. + 7 of the stage buffer; lane L fills
@@ -299,9 +303,9 @@ gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, 
     // i + 1.
     auto stage = [&](auto S_, int i) __attribute__((always_inline)) {
         constexpr int S = decltype(S_)::value, cur = S & 1;
-        uint8_t *const xb = cur ? xs1 : xs0, *const xn = cur ? xs0 : xs1;
+        uint8_t *const xb = (cur ? xs1 : xs0) + kg * T::kX, *const xn = (cur ? xs0 : xs1) + kg * T::kX;
         constexpr int ur = (S + 1) / 2 % 2, un = (S + 3) / 2 % 2;
-        uint8_t *const wc = ur ? ws1 : ws0, *const wn = un ? ws1 : ws0;
+        uint8_t *const wc = (ur ? ws1 : ws0) + kg * U::kBytes, *const wn = (un ? ws1 : ws0) + kg * U::kBytes;
         wait_vm_lgkm0<S % 2 == 0 ? WL : 0>();
         lds_barrier();
         bf16x8 a[2][TM];
@@ -325,12 +329,12 @@ gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, 
 
     // Prologue: what the stages before the first would have issued, in their order, then the
     // first stage's block and first operand.
-    load_w(sbeg / 2, ws0);
-    load_x(sbeg, xs0);
-    load_w(sbeg / 2 + 1, ws1);
+    load_w(sbeg / 2, ws0 + kg * U::kBytes);
+    load_x(sbeg, xs0 + kg * T::kX);
+    load_w(sbeg / 2 + 1, ws1 + kg * U::kBytes);
     wait_vm_lgkm0<XL + WL>();
     asm volatile("" ::: "memory");
-    read_raw(sbeg, ws0, raw[0]);
+    read_raw(sbeg, ws0 + kg * U::kBytes, raw[0]);
     decode_scale(sbeg, raw[0], sc[0]);
     b[0] = operand(raw[0], sc[0], 0);
     // Whole periods in the loop: with an exit between stages the compiler takes the loads in flight at
@@ -338,10 +342,10 @@ gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, 
     // 228 us, 512 x 4096 x 4096 31.9 -> 30.8).
 #define J4Q_STAGE(S) stage(std::integral_constant<int, S>{}, i + S);
     int i = sbeg;
-    for (; i + 4 <= ns; i += 4) {
+    for (; i + 4 <= nl; i += 4) {
         J4Q_STAGE(0) J4Q_STAGE(1) J4Q_STAGE(2) J4Q_STAGE(3)
     }
-    if constexpr (FMT == Q8_0 || FMT == Q4_0) {
+    if constexpr (KG == 1 && (FMT == Q8_0 || FMT == Q4_0)) {
         if (i < ns) {
             J4Q_STAGE(0)
             if (i + 1 < ns) {
@@ -352,6 +356,26 @@ gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, 
     }
 #undef J4Q_STAGE
     __builtin_amdgcn_s_waitcnt(0);  // no LDS load outlives the workgroup
+    if constexpr (KG == 2) {
+        // The second group's sums through the X buffers (which hold them exactly); the first adds them.
+        typedef float f32x8 __attribute__((ext_vector_type(8)));
+        f32x8 *const r0 = reinterpret_cast<f32x8 *>(xs0), *const r1 = reinterpret_cast<f32x8 *>(xs1);
+        __syncthreads();
+        if (kg) {
+#pragma unroll
+            for (int t = 0; t < TM; t++) {
+                r0[(t * WV + wave) * 64 + lane] = __builtin_shufflevector(acc[t], acc[t], 0, 1, 2, 3, 4, 5, 6, 7);
+                r1[(t * WV + wave) * 64 + lane] = __builtin_shufflevector(acc[t], acc[t], 8, 9, 10, 11, 12, 13, 14, 15);
+            }
+        }
+        __syncthreads();
+        if (kg) return;
+#pragma unroll
+        for (int t = 0; t < TM; t++) {
+            const f32x8 a = r0[(t * WV + wave) * 64 + lane], b = r1[(t * WV + wave) * 64 + lane];
+            acc[t] += __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+        }
+    }
 
     // Result element v of tile t: row 32 t + 8 (v / 4) + 4 h + v % 4, column r32.
     float *const out = part ? part + (int64_t)blockIdx.y * M * N : y;

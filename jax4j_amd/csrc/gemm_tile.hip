@@ -10,6 +10,7 @@ namespace {
 // split_stages 64-element stages. tm = 0: the call does not run on it.
 struct Shape {
     int waves = 0, tm = 0, splits = 1, split_stages = 0;
+    int groups = 1;  // 2: each workgroup's two groups of waves take a half of K each, split_stages long
 };
 
 // The tiles, and what one stage of one workgroup takes in us on MI355X: few workgroups, each
@@ -49,7 +50,21 @@ Shape pick(int id, const QMat &w, int64_t m, float *us_out) {
             if (s > 1) us += 2.0f + .25f * (float)s + (float)((2 * s + 1) * m * n * 4) / 5.5e6f;
             if (!best.tm || us < best_us) {
                 best_us = us;
-                best = Shape{c.waves, c.tm, (int)s, (int)per};
+                best = Shape{c.waves, c.tm, (int)s, (int)per, 1};
+            }
+        }
+    }
+    // Few tiles without the sum kernel: two groups of four waves in a workgroup, half of K each
+    // (950 x 1040 x 2560 Q4_K 19.8 -> 17.3 us, 500 x 1040 x 2560 16.8 -> 14.3, 600 x 2000 x 2048 Q6_K 20.8 -> 17.0).
+    if (id != Q8_0 && ns % 4 == 0) {
+        constexpr Cost kTwo[] = {{4, 1, .45f, .56f, 0.f}, {4, 2, .58f, .70f, 0.f}};
+        for (const Cost &c : kTwo) {
+            const int64_t tiles = ((m + 32 * c.tm - 1) / (32 * c.tm)) * ((n + 127) / 128), per = ((ns + 1) / 2 + 3) / 4 * 4;
+            if (tiles > kCus) continue;
+            const float us = (c.few + (c.all - c.few) * (float)tiles / kCus + (id == Q6_K ? .32f : 0.f)) * (float)per + 3.5f;
+            if (us < best_us) {
+                best_us = us;
+                best = Shape{4, c.tm, 1, (int)per, 2};
             }
         }
     }
@@ -114,7 +129,7 @@ hipError_t launch_fmt(const QMat &w, const uint16_t *x, float *y, int64_t m, con
     float *const part = t.splits > 1 ? ws : nullptr;
     bool launched = false;
 #define J4Q_TILE(WV, TM)                                                                              \
-    if (t.waves == WV && t.tm == TM) {                                                                \
+    if (t.waves == WV && t.tm == TM && t.groups == 1) {                                               \
         gt::gemm_tile<FMT, WV, TM><<<grid, 64 * WV, 0, s>>>(w, x, y, (int)m, t.split_stages, part);   \
         launched = true;                                                                              \
     }
@@ -126,6 +141,15 @@ hipError_t launch_fmt(const QMat &w, const uint16_t *x, float *y, int64_t m, con
     J4Q_TILE(8, 4)
     J4Q_TILE(8, 8)
 #undef J4Q_TILE
+    if constexpr (FMT != Q8_0) {
+        if (t.groups == 2 && t.tm == 1) {
+            gt::gemm_tile<FMT, 4, 1, 2><<<grid, 512, 0, s>>>(w, x, y, (int)m, t.split_stages, part);
+            launched = true;
+        } else if (t.groups == 2 && t.tm == 2) {
+            gt::gemm_tile<FMT, 4, 2, 2><<<grid, 512, 0, s>>>(w, x, y, (int)m, t.split_stages, part);
+            launched = true;
+        }
+    }
     if (!launched) return hipErrorInvalidValue;
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess || t.splits == 1) return e;

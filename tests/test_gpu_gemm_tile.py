@@ -28,9 +28,11 @@ def bits(a):
 # One size or more for every tile that the launch model picks, with rows and columns past the last
 # tile, one superblock up to many, and K splits of unequal length: 32 rows (5, 24: 8 splits, 70: 5
 # splits), 64 (97), 96 (90: 4 to 6 splits; 160), 128 (777, 1024), 160 (300, 2049: 14337 columns), 128
-# x 256 (512), 256 x 256 (2048). Q8_0 also with an odd number of 64-element stages (K = 192).
+# x 256 (512), 256 x 256 (2048), K in two wave groups of a workgroup (950: 64 rows; 500, with unequal
+# halves, and 700: 32). Q8_0 also with an odd number of 64-element stages (K = 192).
 SHAPES = [(5, 37, 512), (24, 4096, 4096), (70, 130, 1280), (97, 10007, 256), (90, 5001, 3072), (160, 14336, 512),
-          (777, 4097, 768), (1024, 4096, 256), (300, 14336, 256), (2049, 14337, 256), (512, 14336, 512), (2048, 14336, 256)]
+          (777, 4097, 768), (1024, 4096, 256), (300, 14336, 256), (2049, 14337, 256), (512, 14336, 512), (2048, 14336, 256),
+          (950, 1040, 2560), (500, 1041, 1280), (700, 700, 1024)]
 
 
 @pytest.mark.parametrize("qt", ALL, ids=lambda q: q.name)
