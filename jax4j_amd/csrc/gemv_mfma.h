@@ -204,10 +204,10 @@ constexpr int round_tiles() { return BB <= 8 && WAVES <= 8 ? 4 : 2; }
 // of 8, so every slice starts on a superblock), kbn <= WAVES * NBW and B <= BB. XREG keeps
 // the wave's A operands and C inputs in registers for the whole kernel instead of
 // re-reading them from LDS per tile.
-// The job argument of the kernel: none at up to 8 rows, whose windows are few.
+// The job argument of the kernel; none without a job (its masked loads and store cost 0.2 us a launch).
 struct NoJob {};
-template <int BB>
-using JobArg = std::conditional_t<BB == 16, SumJob, NoJob>;
+template <bool JOB>
+using JobArg = std::conditional_t<JOB, SumJob, NoJob>;
 
 // Wave priority p (0..3; s_setprio takes an immediate, so p must fold to a constant).
 __device__ __forceinline__ void set_prio(int p) {
@@ -217,10 +217,10 @@ __device__ __forceinline__ void set_prio(int p) {
     else __builtin_amdgcn_s_setprio(0);
 }
 
-template <int FMT, int BB, int WAVES, int IPW, bool XREG, int TS, bool NB = false>
+template <int FMT, int BB, int WAVES, int IPW, bool XREG, int TS, bool NB = false, bool JOB = false>
 __global__ void __launch_bounds__(WAVES * 64)
 gemv_mfma_kernel(QMat m, const float *__restrict__ x, const float *prev, const float *__restrict__ add, float *y,
-                 int B, int kb0, int per, int nbe, float *__restrict__ wsum, JobArg<BB> job) {
+                 int B, int kb0, int per, int nbe, float *__restrict__ wsum, JobArg<JOB> job) {
     kb0 += (int)blockIdx.y * per;
     const int kbn = nbe - kb0 < per ? nbe - kb0 : per;
     if (wsum) {
@@ -262,10 +262,9 @@ gemv_mfma_kernel(QMat m, const float *__restrict__ x, const float *prev, const f
     f32x4 xv[XPL][2];
     // The window sums of an earlier launch (9..16 rows): a thread per 4 of them, loaded ahead of x and
     // stored behind the weight loads, so that they cost neither a launch nor a wait of their own.
-    // Without a job its buffers are empty: loads give zeros, the store is dropped.
-    f32x4 jv[W16 ? SumJob::kWindows : 1];
+    f32x4 jv[JOB ? SumJob::kWindows : 1];
     uint32_t jo = 0;
-    if constexpr (W16) {
+    if constexpr (JOB) {
         const uint32_t c4 = (uint32_t)job.cols / 4u;
         const uint32_t i = ((uint32_t)blockIdx.y * gridDim.x + blockIdx.x) * (uint32_t)(WAVES * 64) + threadIdx.x;
         const uint32_t row = c4 ? i / c4 : 0u;
@@ -351,7 +350,7 @@ gemv_mfma_kernel(QMat m, const float *__restrict__ x, const float *prev, const f
         if constexpr (NB) __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (!NB) __builtin_amdgcn_sched_barrier(0);
-    if constexpr (W16) {  // in window order, as sum_windows_kernel
+    if constexpr (JOB) {  // in window order, as sum_windows_kernel
         f32x4 v = jv[0];
 #pragma unroll
         for (int r = 1; r < SumJob::kWindows; r++) v = r < job.windows ? v + jv[r] : v;
@@ -746,10 +745,15 @@ hipError_t launch_k(const QMat &m, const float *x, const float *add, float *y, i
     constexpr int lds = Plan<BB, Fmt<FMT>::GROUPS, WAVES, NBW, round_tiles<BB, WAVES>()>::kBytes;
     static_assert(lds <= 160 * 1024, "LDS of one workgroup");
     if (windows > 1 && !part) return hipErrorInvalidValue;
-    JobArg<BB> arg;
-    if constexpr (BB == 16) arg = job;
-    gemv_mfma_kernel<FMT, BB, WAVES, IPW, XREG, TS, NB><<<dim3(grid, windows), WAVES * 64, lds, s>>>(
-        m, x, prev, add, y, B, kb0, per, nbe, windows > 1 ? part : nullptr, arg);
+    float *const ws = windows > 1 ? part : nullptr;
+    const dim3 g(grid, windows);
+    if constexpr (BB == 16) {
+        if (job.part) {
+            gemv_mfma_kernel<FMT, BB, WAVES, IPW, XREG, TS, NB, true><<<g, WAVES * 64, lds, s>>>(m, x, prev, add, y, B, kb0, per, nbe, ws, job);
+            return hipGetLastError();
+        }
+    }
+    gemv_mfma_kernel<FMT, BB, WAVES, IPW, XREG, TS, NB><<<g, WAVES * 64, lds, s>>>(m, x, prev, add, y, B, kb0, per, nbe, ws, NoJob());
     return hipGetLastError();
 }
 
