@@ -94,7 +94,7 @@ bool takes_along(const Op &o, const SumJob &job, int64_t batch) {
 // gap; a 4096 x 14336 layer at 16 rows had 20 us of them in 77). The sums of q|k|v and of gate|up,
 // which no later GEMV of the step reads, ride on the next launch instead; with parts of different
 // types they go to their place in the group at once, and the row copy falls away
-// (step of 16 rows, 32 layers of 4096 x 14336 in Q4_K and Q6_K: 2162 -> 2060 us).
+// (step of 16 rows, 32 layers of 4096 x 14336 in Q4_K and Q6_K: 2216 -> 2087 us).
 hipError_t enqueue(const Plan &p, hipStream_t s) {
     SumJob job;  // left by the last GEMV
     int w = 0;
