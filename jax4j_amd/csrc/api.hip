@@ -5,6 +5,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -67,7 +68,8 @@ thread_local std::string t_err;
 //    (j4q_buffer_info) can be in use on other streams and goes back with hipFree, which waits.
 //  - One workspace of at most 256 MiB for calls on the engine stream (which run one after another);
 //    calls on other streams take stream-ordered memory.
-//  - Neither serves a call under stream capture: a graph keeps the addresses it recorded.
+//  - Neither serves a call under stream capture: a graph keeps the addresses it recorded, its operands'
+//    too, and may be launched on any stream. Those buffers go back with hipFree as well.
 // All of it is given back when the last buffer is released.
 struct BlockCache {
     static constexpr uint64_t kMaxBlock = 4ull << 20, kMaxBytes = 64ull << 20;
@@ -279,15 +281,20 @@ int64_t elements_of(const Buf &b) { return b.rank == 1 ? b.dims[0] : b.dims[0] *
 
 // Allocates a device buffer of `bytes` (0 allowed) and registers it.
 // Registering may grow the buffer table, so callers keep the returned device pointer, not
-// a Buf* taken before the call.
-int alloc_buf(int kind, int rank, int64_t d0, int64_t d1, uint64_t bytes, j4q_buffer *out, void **dev_out) {
+// a Buf* taken before the call. operands: the dense buffers that the call reads.
+int alloc_buf(int kind, int rank, int64_t d0, int64_t d1, uint64_t bytes, j4q_buffer *out, void **dev_out,
+              std::initializer_list<Buf *> operands = {}) {
     Buf nb;
     nb.kind = kind;
     nb.rank = rank;
     nb.dims[0] = d0;
     nb.dims[1] = d1;
     nb.bytes = bytes;
-    if (bytes && bytes <= BlockCache::kMaxBlock && !capturing(g_stream)) {
+    const bool captured = capturing(g_stream);
+    if (captured)
+        for (Buf *b : operands)
+            if (b) b->block = 0;
+    if (bytes && bytes <= BlockCache::kMaxBlock && !captured) {
         const int k = BlockCache::slot(bytes);
         nb.block = 1ull << k;
         nb.dev = g_cache.take(k);
@@ -454,7 +461,7 @@ int matvec_common(j4q_buffer wh, j4q_buffer xh, j4q_buffer addh, j4q_buffer *out
     const j4q::QMat m = qmat_of(*w);
     const int qt = w->qtype;
     void *ydev;
-    if ((rc = alloc_buf(J4Q_KIND_F32, B == 1 ? 1 : 2, B == 1 ? N : B, B == 1 ? 0 : N, (uint64_t)(B * N) * 4, out, &ydev)))
+    if ((rc = alloc_buf(J4Q_KIND_F32, B == 1 ? 1 : 2, B == 1 ? N : B, B == 1 ? 0 : N, (uint64_t)(B * N) * 4, out, &ydev, {x, add})))
         return rc;
     // a batched call over several column windows runs them in one launch on a stream-ordered
     // workspace for their partial sums; if it cannot be had, the windows run one after another
@@ -884,7 +891,7 @@ int j4q_quantize_act(j4q_buffer xh, j4q_buffer *xq, j4q_buffer *xs) {
     const int64_t M = x->dims[0], K = x->dims[1];
     const void *xdev = x->dev;
     void *qdev, *sdev;
-    if ((rc = alloc_buf(J4Q_KIND_I8, 2, M, K, (uint64_t)(M * K), xq, &qdev))) return rc;
+    if ((rc = alloc_buf(J4Q_KIND_I8, 2, M, K, (uint64_t)(M * K), xq, &qdev, {x}))) return rc;
     if ((rc = alloc_buf(J4Q_KIND_F32, 2, M, K / 32, (uint64_t)(M * (K / 32)) * 4, xs, &sdev))) {
         drop_buf(xq);
         return rc;
@@ -918,7 +925,7 @@ int j4q_quant_matmul(j4q_buffer wh, j4q_buffer xh, int variant, j4q_buffer *out)
     const uint16_t *xdev = (const uint16_t *)x->dev;
     // w and x are not used past this point: registering y below may move the buffer table
     void *ydev;
-    if ((rc = alloc_buf(J4Q_KIND_F32, 2, M, N, (uint64_t)(M * N) * 4, out, &ydev))) return rc;
+    if ((rc = alloc_buf(J4Q_KIND_F32, 2, M, N, (uint64_t)(M * N) * 4, out, &ydev, {x}))) return rc;
     if (variant == J4Q_GEMM_BF16) {
         void *ws = nullptr;
         const uint64_t wsb = j4q::gemm_bf16_workspace_bytes(qt, m, M);
