@@ -53,6 +53,7 @@ using gw::dma4;
 using gw::f32x2;
 using gw::kOob;
 using gw::lds_barrier;
+using gw::load_order;
 using gw::make_rsrc;
 using gw::u32x2;
 using gw::u32x4;
@@ -312,6 +313,7 @@ gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, 
         read_a(xb, 0, a[0]);
         read_raw(i + 1, wc, raw[cur ^ 1]);
         load_x(i + 1, xn);
+        load_order();  // X first: the wait at an even stage leaves the newest unit of W outstanding
         if constexpr (S % 2 == 1) load_w((i + 3) / 2, wn);
         // issue the loads first (not where that costs registers: Q6_K at 256 rows would spill)
         if constexpr (TM < 8 || FMT != Q6_K) __builtin_amdgcn_sched_barrier(0);
@@ -330,7 +332,9 @@ gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, 
     // Prologue: what the stages before the first would have issued, in their order, then the
     // first stage's block and first operand.
     load_w(sbeg / 2, ws0 + kg * U::kBytes);
+    load_order();
     load_x(sbeg, xs0 + kg * T::kX);
+    load_order();
     load_w(sbeg / 2 + 1, ws1 + kg * U::kBytes);
     wait_vm_lgkm0<XL + WL>();
     asm volatile("" ::: "memory");

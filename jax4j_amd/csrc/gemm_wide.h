@@ -292,6 +292,11 @@ __device__ __forceinline__ void wait_vm_lgkm0() {
     __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | ((N >> 4) << 14));
 }
 
+// Keeps the global loads before and behind it in their order, on which a wait for all but the newest N
+// loads relies: the scheduler may move arithmetic and LDS reads across (with everything held in place
+// gemv_tile took up to 37 registers more), loads not.
+__device__ __forceinline__ void load_order() { __builtin_amdgcn_sched_barrier(0x001 | 0x080 | 0x100 | 0x200 | 0x400); }
+
 // A workgroup barrier without __syncthreads()'s release fence: the fence would wait for every
 // LDS load in flight (vmcnt(0)), which is the ring this kernel keeps open. The empty asm
 // statements keep the compiler from moving memory accesses across it.

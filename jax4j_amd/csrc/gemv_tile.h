@@ -39,6 +39,7 @@ using gw::dma4;
 using gw::dma4s;
 using gw::kOob;
 using gw::lds_barrier;
+using gw::load_order;
 using gw::make_rsrc;
 using gw::u32x2;
 using gw::u32x4;
@@ -303,6 +304,7 @@ gemv_tile(QMat w, const uint16_t *__restrict__ xs, const float *__restrict__ uns
         read_a(xb, 0, 0, a[0]);
         read_raw(i + 1, wc, raw[cur ^ 1]);
         load_x(i + 1, xn);
+        load_order();  // X first: the wait at an even stage leaves the newest unit of W outstanding
         if constexpr (S % 2 == 1) load_w((i + 3) / 2, wn);
         __builtin_amdgcn_sched_barrier(0);  // issue the loads first
 #pragma unroll
@@ -332,7 +334,9 @@ gemv_tile(QMat w, const uint16_t *__restrict__ xs, const float *__restrict__ uns
     };
 
     load_w(sbeg / 2, ws0);
+    load_order();
     load_x(sbeg, xs0);
+    load_order();
     load_w(sbeg / 2 + 1, ws1);
     wait_vm_lgkm0<XL + WL>();
     asm volatile("" ::: "memory");
