@@ -117,10 +117,14 @@ bool capturing(hipStream_t s) {
 }
 
 void give_back_kept() {
+    // another stream may be under capture, where only a relaxed thread may free
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
     g_cache.clear();
     if (g_kept_ws) (void)hipFree(g_kept_ws);
     g_kept_ws = nullptr;
     g_kept_ws_bytes = 0;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
 }
 
 // hipMalloc, a second time without what the engine keeps if memory is short.
@@ -147,10 +151,17 @@ hipError_t begin_workspace(hipStream_t s, uint64_t bytes, void **out) {
             if (g_kept_ws) (void)hipFree(g_kept_ws);  // waits for the work that uses it
             g_kept_ws = nullptr;
             g_kept_ws_bytes = 0;
-            if (hipMalloc(&g_kept_ws, want) == hipSuccess) {
-                g_kept_ws_bytes = want;
-            } else {
+            g_kept_ws_bytes = want;
+            hipError_t e = hipMalloc(&g_kept_ws, want);
+            if (e == hipErrorOutOfMemory) {  // no more than is needed, and with the cached blocks given back
+                (void)hipGetLastError();
+                g_cache.clear();
+                g_kept_ws_bytes = bytes;
+                e = hipMalloc(&g_kept_ws, bytes);
+            }
+            if (e != hipSuccess) {
                 g_kept_ws = nullptr;
+                g_kept_ws_bytes = 0;
                 (void)hipGetLastError();
             }
             (void)hipThreadExchangeStreamCaptureMode(&mode);
@@ -160,7 +171,13 @@ hipError_t begin_workspace(hipStream_t s, uint64_t bytes, void **out) {
             return hipSuccess;
         }
     }
-    return hipMallocAsync(out, bytes, s);
+    hipError_t e = hipMallocAsync(out, bytes, s);
+    if (e == hipErrorOutOfMemory && (g_kept_ws || g_cache.bytes) && !capturing(s)) {
+        (void)hipGetLastError();
+        give_back_kept();
+        e = hipMallocAsync(out, bytes, s);
+    }
+    return e;
 }
 
 void end_workspace(hipStream_t s, void *p) {
@@ -929,7 +946,7 @@ int j4q_quant_matmul(j4q_buffer wh, j4q_buffer xh, int variant, j4q_buffer *out)
     if (variant == J4Q_GEMM_BF16) {
         void *ws = nullptr;
         const uint64_t wsb = j4q::gemm_bf16_workspace_bytes(qt, m, M);
-        if (wsb) LAUNCH_INTO("hipMallocAsync", out, begin_workspace(g_stream, wsb, &ws));
+        if (wsb) LAUNCH_INTO("quantMatmul workspace", out, begin_workspace(g_stream, wsb, &ws));
         const hipError_t e = j4q::launch_gemm_bf16(qt, m, xdev, (float *)ydev, M, (float *)ws, g_stream);
         end_workspace(g_stream, ws);
         LAUNCH_INTO("quantMatmul", out, e);
@@ -937,7 +954,7 @@ int j4q_quant_matmul(j4q_buffer wh, j4q_buffer xh, int variant, j4q_buffer *out)
     }
     void *ws = nullptr;
     const uint64_t qbytes = (uint64_t)(M * K), sbytes = (uint64_t)(M * (K / 32)) * 4;
-    LAUNCH_INTO("hipMallocAsync", out, begin_workspace(g_stream, j4q::align256(qbytes) + sbytes, &ws));
+    LAUNCH_INTO("quantMatmul workspace", out, begin_workspace(g_stream, j4q::align256(qbytes) + sbytes, &ws));
     int8_t *xq = (int8_t *)ws;
     float *xs = (float *)((uint8_t *)ws + j4q::align256(qbytes));
     hipError_t e = j4q::launch_quantize_act(xdev, M, K, xq, xs, g_stream);
@@ -1006,7 +1023,7 @@ int j4q_quant_matmul_into(j4q_buffer wh, const uint16_t *x, int64_t m, int varia
     if (variant == J4Q_GEMM_BF16) {
         void *ws = nullptr;
         const uint64_t wsb = j4q::gemm_bf16_workspace_bytes(w->qtype, mm, m);
-        if (wsb) HIP_TRY("hipMallocAsync", begin_workspace(s, wsb, &ws));
+        if (wsb) HIP_TRY("quantMatmul_into workspace", begin_workspace(s, wsb, &ws));
         const hipError_t e = j4q::launch_gemm_bf16(w->qtype, mm, x, y, m, (float *)ws, s);
         end_workspace(s, ws);
         HIP_TRY("quantMatmul_into", e);

@@ -51,3 +51,33 @@ def test_operands_of_other_calls_are_reused(shim):
         result = len(log("free")), len(log("malloc"))
     """)
     assert (freed, taken) == (0, 0)
+
+
+MIB = 1 << 20
+
+
+@pytest.mark.parametrize("stream", ["be.stream()", "0x77770"])
+def test_kept_memory_is_given_back_before_a_workspace_is_refused(shim, stream):
+    """A call that needs a workspace has it as long as what is free and what the engine keeps suffice."""
+    ok, refused = fakehip.run(shim, f"""
+        w = zeros(QuantType.Q4_K, 512, 14336)
+        x, y = address(24 * 14336 * 2), address(24 * 512 * 4)
+        log()
+        be.quant_matmul_into(w, x, 24, "bf16", 0, 0, y, {stream})
+        need = max(int(l.split()[1]) for l in log("malloc", "malloc_async"))
+        assert need <= {MIB}
+        held = [be.upload(np.zeros(1 << 18, np.float32)) for _ in range(8)]
+        for b in held:
+            be.release(b)  # 8 MiB of blocks
+        fake.fake_capacity(fake.fake_used() + 4096)
+        be.quant_matmul_into(w, address(64 * 14336 * 2), 64, "bf16", 0, 0, address(64 * 512 * 4), {stream})
+        assert max(int(l.split()[1]) for l in log("malloc", "malloc_async")) > {MIB}
+        fake.fake_capacity(0)
+        try:
+            be.quant_matmul_into(w, address(640 * 14336 * 2), 640, "bf16", 0, 0, address(640 * 512 * 4), 0x99990)
+            refused = None
+        except RuntimeError as e:
+            refused = str(e)
+        result = True, refused
+    """)
+    assert ok and "out of memory" in refused and "workspace" in refused
