@@ -24,8 +24,9 @@
  *    (NULL = the engine stream) and return without synchronising.
  *  - Buffers returned through a j4q_buffer* are owned by the engine until j4q_release. The engine
  *    keeps released blocks of dense buffers (up to 4 MiB each, 64 MiB in all; not of a buffer
- *    whose address j4q_buffer_info has given out) and one workspace of its stream (up to 256 MiB)
- *    for later calls, and gives them back when the last buffer is released or memory is short.
+ *    whose address j4q_buffer_info has given out) and workspaces (up to 256 MiB each, 512 MiB in
+ *    all; one of its own stream, the others of callers' streams) for later calls, and gives them
+ *    back when the last buffer is released or memory is short, which waits for the device.
  */
 #ifndef JAX4J_MI355X_H
 #define JAX4J_MI355X_H
@@ -196,18 +197,17 @@ int j4q_quant_matmul(j4q_buffer weights, j4q_buffer x, int variant, j4q_buffer *
  * Q4_K and Q6_K; other adds overlapping y return J4Q_EUNSUPPORTED (column windows chained
  * one after another would read it after rewriting y). A batched call over several column
  * windows keeps their partial sums (batch x rows x windows floats), and one above 18 to 34 rows
- * (by type and cols) also x in 4 bytes an element, in the engine's kept workspace on the engine
- * stream, up to 256 MiB, else in stream-ordered memory of `stream` (hipMallocAsync /
- * hipFreeAsync); nothing else is allocated. */
+ * (by type and cols) also x in 4 bytes an element, in a workspace that the engine keeps (on every
+ * stream); above 256 MiB, under stream capture, and where the kept ones are all in use, in
+ * stream-ordered memory of `stream` (hipMallocAsync / hipFreeAsync). Nothing else is allocated. */
 int j4q_quant_matvec_into(j4q_buffer weights, const float *x_dev, const float *add_dev, float *y_dev,
                           int64_t batch, void *stream);
 /* Prefill GEMM into caller memory (the weight types and variants of j4q_quant_matmul).
  * x_dev bf16 [m, cols]; y_dev fp32 [m, rows]. The int8 variant also needs xq_dev int8
  * [m, cols] and xs_dev fp32 [m, cols/32] as workspace; the bf16 variant ignores them. On
  * Q4_0, Q4_K and Q6_K weights the bf16 variant splits K over workgroups where the tiles alone
- * would leave CUs idle, and keeps the partial products (at most 32 MiB) in the engine's kept
- * workspace on the engine stream, else in stream-ordered memory of `stream` (hipMallocAsync /
- * hipFreeAsync); nothing else is allocated. */
+ * would leave CUs idle, and keeps the partial products (at most 32 MiB) in a workspace as
+ * j4q_quant_matvec_into does; nothing else is allocated. */
 int j4q_quant_matmul_into(j4q_buffer weights, const uint16_t *x_dev, int64_t m, int variant, int8_t *xq_dev,
                           float *xs_dev, float *y_dev, void *stream);
 /* The int8 variant on activations already quantized (engine-local; no counterpart in the

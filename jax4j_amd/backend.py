@@ -265,8 +265,8 @@ class Mi355xBackend:
         return s.value or 0
 
     def quant_matvec_into(self, weights: DeviceBuffer, x_ptr: int, add_ptr: int, y_ptr: int, batch: int = 1, stream: int = 0) -> None:
-        """Stream-ordered GEMV on caller device memory; does not sync. A batched call over
-        several column windows takes its partial-sum workspace from stream-ordered memory."""
+        """Stream-ordered GEMV on caller device memory; does not sync. A batched call may use a
+        workspace, which the engine keeps for later calls on any stream."""
         check(
             self._lib().j4q_quant_matvec_into(
                 weights.handle, x_ptr, add_ptr or None, y_ptr, batch, stream or None

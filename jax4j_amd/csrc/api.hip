@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "engine.h"
+#include "kept_memory.h"
 #include "synth.h"
 
 namespace j4q {
@@ -30,7 +31,7 @@ struct Buf {
     int64_t dims[2] = {0, 0};
     void *dev = nullptr;
     uint64_t bytes = 0;
-    uint64_t block = 0;  // bytes of its cached block (see BlockCache); 0: an allocation of its own
+    uint64_t block = 0;  // bytes of its cached block (see j4q::BlockCache); 0: an allocation of its own
     uint32_t gen = 0;
     bool live = false;
     // decode plans whose captured graph reads this buffer's memory; while any lives the
@@ -59,129 +60,21 @@ int g_dev = -1;
 hipStream_t g_stream = nullptr;
 thread_local std::string t_err;
 
-// Device memory the engine keeps between calls, under g_mu. hipMalloc + hipFree cost an SPI call
-// ~8 us and a wait for the device, hipMallocAsync + hipFreeAsync a call with a workspace ~15 us
-// (Q4_K 512 x 4096 at 16 rows: 19.7 us a call with them, 4.6 us of kernels).
-//  - Blocks of released F32 / BF16 / I8 buffers, in powers of two from 256 bytes to 4 MiB, at
-//    most 64 MiB in all: work on such a buffer runs on the engine stream alone, so its block may
-//    be written again behind it with no wait. A buffer whose address left the engine
-//    (j4q_buffer_info) can be in use on other streams and goes back with hipFree, which waits.
-//  - One workspace of at most 256 MiB for calls on the engine stream (which run one after another);
-//    calls on other streams take stream-ordered memory.
-//  - Neither serves a call under stream capture: a graph keeps the addresses it recorded, its operands'
-//    too, and may be launched on any stream. Those buffers go back with hipFree as well.
-// All of it is given back when the last buffer is released.
-struct BlockCache {
-    static constexpr uint64_t kMaxBlock = 4ull << 20, kMaxBytes = 64ull << 20;
-    std::vector<void *> free_[23];  // by log2 of the block size
-    uint64_t bytes = 0;
-    static int slot(uint64_t n) {
-        int k = 8;
-        while ((1ull << k) < n) k++;
-        return k;
-    }
-    void *take(int k) {
-        if (free_[k].empty()) return nullptr;
-        void *p = free_[k].back();
-        free_[k].pop_back();
-        bytes -= 1ull << k;
-        return p;
-    }
-    bool give(void *p, int k) {
-        if (bytes + (1ull << k) > kMaxBytes) return false;
-        free_[k].push_back(p);
-        bytes += 1ull << k;
-        return true;
-    }
-    void clear() {
-        for (auto &v : free_) {
-            for (void *p : v) (void)hipFree(p);
-            v.clear();
-        }
-        bytes = 0;
-    }
-};
-BlockCache g_cache;
-constexpr uint64_t kMaxKeptWorkspace = 256ull << 20;
-void *g_kept_ws = nullptr;
-uint64_t g_kept_ws_bytes = 0;
+j4q::BlockCache g_cache;
+j4q::Workspaces g_workspaces(g_cache);
 int64_t g_live = 0;  // live buffers
 
-bool capturing(hipStream_t s) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
-        (void)hipGetLastError();
-        return true;
-    }
-    return st != hipStreamCaptureStatusNone;
-}
-
-void give_back_kept() {
-    // another stream may be under capture, where only a relaxed thread may free
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
-    g_cache.clear();
-    if (g_kept_ws) (void)hipFree(g_kept_ws);
-    g_kept_ws = nullptr;
-    g_kept_ws_bytes = 0;
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
-}
+using j4q::capturing;
 
 // hipMalloc, a second time without what the engine keeps if memory is short.
 hipError_t dev_malloc(void **p, uint64_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
-    if (e == hipErrorOutOfMemory && (g_kept_ws || g_cache.bytes)) {
+    if (e == hipErrorOutOfMemory && (g_workspaces.bytes() || g_cache.bytes())) {
         (void)hipGetLastError();
-        give_back_kept();
+        g_workspaces.give_back();
         e = hipMalloc(p, bytes);
     }
     return e;
-}
-
-// A workspace of `bytes` for the work that the caller enqueues on `s` before it calls
-// end_workspace.
-hipError_t begin_workspace(hipStream_t s, uint64_t bytes, void **out) {
-    if (s == g_stream && bytes <= kMaxKeptWorkspace && !capturing(s)) {
-        if (bytes > g_kept_ws_bytes) {
-            uint64_t want = 1ull << 20;
-            while (want < bytes) want *= 2;
-            // another stream may be under capture, where only a relaxed thread may allocate
-            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-            (void)hipThreadExchangeStreamCaptureMode(&mode);
-            if (g_kept_ws) (void)hipFree(g_kept_ws);  // waits for the work that uses it
-            g_kept_ws = nullptr;
-            g_kept_ws_bytes = 0;
-            g_kept_ws_bytes = want;
-            hipError_t e = hipMalloc(&g_kept_ws, want);
-            if (e == hipErrorOutOfMemory) {  // no more than is needed, and with the cached blocks given back
-                (void)hipGetLastError();
-                g_cache.clear();
-                g_kept_ws_bytes = bytes;
-                e = hipMalloc(&g_kept_ws, bytes);
-            }
-            if (e != hipSuccess) {
-                g_kept_ws = nullptr;
-                g_kept_ws_bytes = 0;
-                (void)hipGetLastError();
-            }
-            (void)hipThreadExchangeStreamCaptureMode(&mode);
-        }
-        if (bytes <= g_kept_ws_bytes) {
-            *out = g_kept_ws;
-            return hipSuccess;
-        }
-    }
-    hipError_t e = hipMallocAsync(out, bytes, s);
-    if (e == hipErrorOutOfMemory && (g_kept_ws || g_cache.bytes) && !capturing(s)) {
-        (void)hipGetLastError();
-        give_back_kept();
-        e = hipMallocAsync(out, bytes, s);
-    }
-    return e;
-}
-
-void end_workspace(hipStream_t s, void *p) {
-    if (p && p != g_kept_ws) (void)hipFreeAsync(p, s);
 }
 
 int fail(int code, const char *fmt, ...) {
@@ -311,8 +204,8 @@ int alloc_buf(int kind, int rank, int64_t d0, int64_t d1, uint64_t bytes, j4q_bu
     if (captured)
         for (Buf *b : operands)
             if (b) b->block = 0;
-    if (bytes && bytes <= BlockCache::kMaxBlock && !captured) {
-        const int k = BlockCache::slot(bytes);
+    if (bytes && bytes <= j4q::BlockCache::kMaxBlock && !captured) {
+        const int k = j4q::BlockCache::slot(bytes);
         nb.block = 1ull << k;
         nb.dev = g_cache.take(k);
     }
@@ -480,21 +373,12 @@ int matvec_common(j4q_buffer wh, j4q_buffer xh, j4q_buffer addh, j4q_buffer *out
     void *ydev;
     if ((rc = alloc_buf(J4Q_KIND_F32, B == 1 ? 1 : 2, B == 1 ? N : B, B == 1 ? 0 : N, (uint64_t)(B * N) * 4, out, &ydev, {x, add})))
         return rc;
-    // a batched call over several column windows runs them in one launch on a stream-ordered
-    // workspace for their partial sums; if it cannot be had, the windows run one after another
+    // for partial sums of a batched call; if there is none to be had, the batch runs without
     j4q::Workspace ws;
     const uint64_t wsb = j4q::gemv_workspace_bytes(qt, m, B);
-    if (wsb) {
-        void *p = nullptr;
-        if (begin_workspace(g_stream, wsb, &p) == hipSuccess) {
-            ws.ptr = (float *)p;
-            ws.bytes = wsb;
-        } else {
-            (void)hipGetLastError();
-        }
-    }
+    if (wsb && g_workspaces.begin(g_stream, g_stream, wsb, &ws) != hipSuccess) (void)hipGetLastError();
     const hipError_t e = j4q::launch_gemv(qt, m, (const float *)xdev, (const float *)adev, (float *)ydev, B, g_stream, ws);
-    end_workspace(g_stream, ws.ptr);
+    g_workspaces.end(g_stream, ws, e == hipSuccess);
     LAUNCH_INTO(op, out, e);
     return J4Q_OK;
 }
@@ -836,13 +720,13 @@ int j4q_release(j4q_buffer h) {
     if (b->dev) {
         if ((rc = ensure_ready())) return rc;
         // hipFree waits for work that may still read the buffer.
-        if (!b->block || capturing(g_stream) || !g_cache.give(b->dev, BlockCache::slot(b->block)))
+        if (!b->block || capturing(g_stream) || !g_cache.give(b->dev, j4q::BlockCache::slot(b->block)))
             HIP_TRY("hipFree", hipFree(b->dev));
     }
     b->dev = nullptr;
     b->live = false;
     g_free.push_back((uint32_t)((h & 0xffffffffu) - 1));
-    if (--g_live == 0) give_back_kept();
+    if (--g_live == 0) g_workspaces.give_back();
     return J4Q_OK;
 }
 
@@ -944,22 +828,22 @@ int j4q_quant_matmul(j4q_buffer wh, j4q_buffer xh, int variant, j4q_buffer *out)
     void *ydev;
     if ((rc = alloc_buf(J4Q_KIND_F32, 2, M, N, (uint64_t)(M * N) * 4, out, &ydev, {x}))) return rc;
     if (variant == J4Q_GEMM_BF16) {
-        void *ws = nullptr;
+        j4q::Workspace ws;
         const uint64_t wsb = j4q::gemm_bf16_workspace_bytes(qt, m, M);
-        if (wsb) LAUNCH_INTO("quantMatmul workspace", out, begin_workspace(g_stream, wsb, &ws));
-        const hipError_t e = j4q::launch_gemm_bf16(qt, m, xdev, (float *)ydev, M, (float *)ws, g_stream);
-        end_workspace(g_stream, ws);
+        if (wsb) LAUNCH_INTO("quantMatmul workspace", out, g_workspaces.begin(g_stream, g_stream, wsb, &ws));
+        const hipError_t e = j4q::launch_gemm_bf16(qt, m, xdev, (float *)ydev, M, ws, g_stream);
+        g_workspaces.end(g_stream, ws, e == hipSuccess);
         LAUNCH_INTO("quantMatmul", out, e);
         return J4Q_OK;
     }
-    void *ws = nullptr;
+    j4q::Workspace ws;
     const uint64_t qbytes = (uint64_t)(M * K), sbytes = (uint64_t)(M * (K / 32)) * 4;
-    LAUNCH_INTO("quantMatmul workspace", out, begin_workspace(g_stream, j4q::align256(qbytes) + sbytes, &ws));
-    int8_t *xq = (int8_t *)ws;
-    float *xs = (float *)((uint8_t *)ws + j4q::align256(qbytes));
+    LAUNCH_INTO("quantMatmul workspace", out, g_workspaces.begin(g_stream, g_stream, j4q::align256(qbytes) + sbytes, &ws));
+    int8_t *xq = (int8_t *)ws.ptr;
+    float *xs = (float *)((uint8_t *)ws.ptr + j4q::align256(qbytes));
     hipError_t e = j4q::launch_quantize_act(xdev, M, K, xq, xs, g_stream);
     if (e == hipSuccess) e = j4q::launch_gemm_q8_int8(m, xq, xs, (float *)ydev, M, g_stream);
-    end_workspace(g_stream, ws);
+    g_workspaces.end(g_stream, ws, e == hipSuccess);
     LAUNCH_INTO("quantMatmul", out, e);
     return J4Q_OK;
 }
@@ -984,21 +868,12 @@ int j4q_quant_matvec_into(j4q_buffer wh, const float *x, const float *add, float
                     (long long)j4q::gemv_single_pass_cols(), (long long)K, (long long)batch);
     if ((rc = ensure_ready())) return rc;
     const hipStream_t s = pick_stream(stream);
-    // partial sums live in the kept workspace or in stream-ordered memory of the call's stream; if
-    // there is none to be had, the batch runs without
+    // if there is no workspace to be had, the batch runs without
     j4q::Workspace ws;
     const uint64_t wsb = j4q::gemv_workspace_bytes(w->qtype, m, batch);
-    if (wsb) {
-        void *p = nullptr;
-        if (begin_workspace(s, wsb, &p) == hipSuccess) {
-            ws.ptr = (float *)p;
-            ws.bytes = wsb;
-        } else {
-            (void)hipGetLastError();
-        }
-    }
+    if (wsb && g_workspaces.begin(s, g_stream, wsb, &ws) != hipSuccess) (void)hipGetLastError();
     const hipError_t e = j4q::launch_gemv(w->qtype, m, x, add, y, batch, s, ws);
-    end_workspace(s, ws.ptr);
+    g_workspaces.end(s, ws, e == hipSuccess);
     HIP_TRY("quantMatvec_into", e);
     return J4Q_OK;
 }
@@ -1021,11 +896,11 @@ int j4q_quant_matmul_into(j4q_buffer wh, const uint16_t *x, int64_t m, int varia
     const hipStream_t s = pick_stream(stream);
     const j4q::QMat mm = qmat_of(*w);
     if (variant == J4Q_GEMM_BF16) {
-        void *ws = nullptr;
+        j4q::Workspace ws;
         const uint64_t wsb = j4q::gemm_bf16_workspace_bytes(w->qtype, mm, m);
-        if (wsb) HIP_TRY("quantMatmul_into workspace", begin_workspace(s, wsb, &ws));
-        const hipError_t e = j4q::launch_gemm_bf16(w->qtype, mm, x, y, m, (float *)ws, s);
-        end_workspace(s, ws);
+        if (wsb) HIP_TRY("quantMatmul_into workspace", g_workspaces.begin(s, g_stream, wsb, &ws));
+        const hipError_t e = j4q::launch_gemm_bf16(w->qtype, mm, x, y, m, ws, s);
+        g_workspaces.end(s, ws, e == hipSuccess);
         HIP_TRY("quantMatmul_into", e);
         return J4Q_OK;
     }
@@ -1073,7 +948,10 @@ int j4q_quant_matmul_noalloc(j4q_buffer wh, const uint16_t *x, int64_t m, int va
     if (variant == J4Q_GEMM_BF16) {
         // the K-quant kernels' split partials (at most 32 MiB) go to the engine's array
         static_assert(kScratchBytes >= (32ull << 20), "scratch holds the bf16 GEMM's workspace");
-        HIP_TRY("quantMatmul_noalloc", j4q::launch_gemm_bf16(w->qtype, mm, x, y, m, (float *)g_scratch, s));
+        j4q::Workspace ws;
+        ws.ptr = (float *)g_scratch;
+        ws.bytes = kScratchBytes;
+        HIP_TRY("quantMatmul_noalloc", j4q::launch_gemm_bf16(w->qtype, mm, x, y, m, ws, s));
         return J4Q_OK;
     }
     int8_t *xq = (int8_t *)g_scratch;

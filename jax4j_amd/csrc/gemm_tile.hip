@@ -122,11 +122,11 @@ sum_splits_kernel(const float *__restrict__ part, int splits, int64_t n, float *
 }
 
 template <int FMT>
-hipError_t launch_fmt(const QMat &w, const uint16_t *x, float *y, int64_t m, const Shape &t, float *ws, hipStream_t s) {
+hipError_t launch_fmt(const QMat &w, const uint16_t *x, float *y, int64_t m, const Shape &t, const Workspace &ws, hipStream_t s) {
     const int64_t tiles = ((m + 32 * t.tm - 1) / (32 * t.tm)) * ((w.rows + 32 * t.waves - 1) / (32 * t.waves));
-    if (tiles > 0x7fffffff || (t.splits > 1 && !ws)) return hipErrorInvalidValue;
+    if (tiles > 0x7fffffff || (t.splits > 1 && !ws.ptr)) return hipErrorInvalidValue;
     const dim3 grid((unsigned)tiles, (unsigned)t.splits);
-    float *const part = t.splits > 1 ? ws : nullptr;
+    float *const part = t.splits > 1 ? ws.ptr : nullptr;
     bool launched = false;
 #define J4Q_TILE(WV, TM)                                                                              \
     if (t.waves == WV && t.tm == TM && t.groups == 1) {                                               \
@@ -155,8 +155,7 @@ hipError_t launch_fmt(const QMat &w, const uint16_t *x, float *y, int64_t m, con
     if (e != hipSuccess || t.splits == 1) return e;
     const int64_t n = m * w.rows;
     const int64_t blocks = ((n % 4 == 0 ? n / 4 : n) + 255) / 256;
-    sum_splits_kernel<<<(unsigned)(blocks < 2048 ? blocks : 2048), 256, 0, s>>>(ws, t.splits, n, y);
-    return hipGetLastError();
+    return launch_with_event(sum_splits_kernel, dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(256), s, ws.done, ws.ptr, t.splits, n, y);
 }
 
 }  // namespace
@@ -177,7 +176,7 @@ uint64_t gemm_bf16_workspace_bytes(int id, const QMat &w, int64_t m) {
     return t.splits > 1 ? (uint64_t)t.splits * (uint64_t)m * (uint64_t)w.rows * 4u : 0;
 }
 
-hipError_t launch_gemm_bf16(int id, const QMat &w, const uint16_t *x, float *y, int64_t m, float *ws, hipStream_t s) {
+hipError_t launch_gemm_bf16(int id, const QMat &w, const uint16_t *x, float *y, int64_t m, const Workspace &ws, hipStream_t s) {
     if (m <= 0 || w.rows <= 0) return hipSuccess;
     const Shape t = shape_of(id, w, m);
     if (id == Q8_0 && !t.tm) return launch_gemm_q8_bf16(w, x, y, m, s);

@@ -163,10 +163,10 @@ void measure_resident_fmt() {
     measure_resident<FMT, 16>();
 }
 
-hipError_t launch_sum(const float *part, int windows, int64_t n, const float *add, float *y, hipStream_t s) {
+hipError_t launch_sum(const float *part, int windows, int64_t n, const float *add, float *y, hipStream_t s, hipEvent_t done) {
     const int64_t blocks = ((n % 4 == 0 ? n / 4 : n) + 255) / 256;  // a thread per float4 where n allows
-    gmf::sum_windows_kernel<<<(unsigned)(blocks < 2048 ? blocks : 2048), 256, 0, s>>>(part, windows, n, add, y);
-    return hipGetLastError();
+    return launch_with_event(gmf::sum_windows_kernel, dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(256), s, done, part,
+                             windows, n, add, y);
 }
 
 // Batched GEMV on the matrix cores (gemv_mfma.h) for up to 16 batch rows per launch,
@@ -219,7 +219,7 @@ hipError_t launch_mfma(const QMat &m, const float *x, const float *add, float *y
             out->cols = out->pitch = (int)m.rows;
             return hipSuccess;
         }
-        return launch_sum(ws.ptr, windows, (int64_t)b * m.rows, add, y, s);
+        return launch_sum(ws.ptr, windows, (int64_t)b * m.rows, add, y, s, ws.done);
     }
     const int grid = tiles < g_cus ? tiles : g_cus;
     for (int kb0 = 0; kb0 < nb; kb0 += per) {
@@ -357,7 +357,8 @@ TileShape tile_shape(int id, const QMat &m, int64_t batch) {
 
 template <int FMT>
 hipError_t launch_tile_fmt(const QMat &m, const float *x, const float *add, float *y, int64_t batch, const TileShape &t,
-                           uint8_t *ws, hipStream_t s) {
+                           const Workspace &space, hipStream_t s) {
+    uint8_t *const ws = (uint8_t *)space.ptr;
     const int K = (int)m.cols;
     _Float16 *const hi = (_Float16 *)ws;
     float *const unscale = (float *)(ws + t.x_bytes);
@@ -374,12 +375,11 @@ hipError_t launch_tile_fmt(const QMat &m, const float *x, const float *add, floa
         const unsigned tiles = (unsigned)(((rows + 32 * t.tm - 1) / (32 * t.tm)) * ((m.rows + 127) / 128));
         const dim3 grid(tiles, (unsigned)t.splits);
         const uint16_t *const xs = (const uint16_t *)ws;
-        if (t.tm == 1) gvt::gemv_tile<FMT, 1><<<grid, 256, 0, s>>>(m, xs, unscale, sums, ab, yb, rows, t.split_stages, part);
-        else gvt::gemv_tile<FMT, 2><<<grid, 256, 0, s>>>(m, xs, unscale, sums, ab, yb, rows, t.split_stages, part);
-        e = hipGetLastError();
+        e = launch_with_event(t.tm == 1 ? gvt::gemv_tile<FMT, 1> : gvt::gemv_tile<FMT, 2>, grid, dim3(256), s,
+                              t.splits > 1 ? nullptr : space.done, m, xs, unscale, sums, ab, yb, rows, t.split_stages, part);
         if (e != hipSuccess) return e;
         if (t.splits > 1) {
-            e = launch_sum(part, t.splits, (int64_t)rows * m.rows, ab, yb, s);
+            e = launch_sum(part, t.splits, (int64_t)rows * m.rows, ab, yb, s, space.done);
             if (e != hipSuccess) return e;
         }
     }
@@ -388,12 +388,11 @@ hipError_t launch_tile_fmt(const QMat &m, const float *x, const float *add, floa
 
 hipError_t launch_tile(int id, const QMat &m, const float *x, const float *add, float *y, int64_t batch, const TileShape &t,
                        const Workspace &ws, hipStream_t s) {
-    uint8_t *const p = (uint8_t *)ws.ptr;
     switch (id) {
-    case Q4_0: return launch_tile_fmt<Q4_0>(m, x, add, y, batch, t, p, s);
-    case Q4_K: return launch_tile_fmt<Q4_K>(m, x, add, y, batch, t, p, s);
-    case Q6_K: return launch_tile_fmt<Q6_K>(m, x, add, y, batch, t, p, s);
-    case Q8_0: return launch_tile_fmt<Q8_0>(m, x, add, y, batch, t, p, s);
+    case Q4_0: return launch_tile_fmt<Q4_0>(m, x, add, y, batch, t, ws, s);
+    case Q4_K: return launch_tile_fmt<Q4_K>(m, x, add, y, batch, t, ws, s);
+    case Q6_K: return launch_tile_fmt<Q6_K>(m, x, add, y, batch, t, ws, s);
+    case Q8_0: return launch_tile_fmt<Q8_0>(m, x, add, y, batch, t, ws, s);
     default: return hipErrorInvalidValue;
     }
 }
@@ -466,7 +465,7 @@ bool gemv_carries(int id, const QMat &m, int64_t batch, const SumJob &job) {
 }
 
 hipError_t launch_sum_job(const SumJob &job, int64_t batch, hipStream_t s) {
-    return launch_sum(job.part, job.windows, batch * job.cols, nullptr, job.y, s);
+    return launch_sum(job.part, job.windows, batch * job.cols, nullptr, job.y, s, nullptr);
 }
 
 hipError_t launch_gemv(int id, const QMat &m, const float *x, const float *add, float *y, int64_t batch,

@@ -25,6 +25,7 @@
 //          sc  [N][K/128]  fp16 d
 #pragma once
 
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -129,7 +130,18 @@ hipError_t launch_dequant_rows(int id, const QMat &m, int64_t row0, int64_t nrow
 struct Workspace {
     float *ptr = nullptr;
     uint64_t bytes = 0;
+    hipEvent_t done = nullptr;    // completed by the last launch that uses it (every such launch is given it)
+    bool stream_ordered = false;  // of hipMallocAsync
 };
+
+// kernel<<<grid, block, 0, s>>>(args...), completing `done` if there is one: the event is the launch's own
+// completion signal (recorded behind it, it took 1.1 us of the GPU's time a call).
+template <class... P, class... A>
+hipError_t launch_with_event(void (*kernel)(P...), dim3 grid, dim3 block, hipStream_t s, hipEvent_t done, A... args) {
+    if (done) hipExtLaunchKernelGGL(kernel, grid, block, 0, s, nullptr, done, 0, static_cast<P>(args)...);
+    else kernel<<<grid, block, 0, s>>>(args...);
+    return hipGetLastError();
+}
 
 // The window sums that a batched GEMV left in its workspace: y[b * pitch + c] = sum over the windows,
 // in their order, of part[window][b][c], c < cols. A later GEMV of the same batch can compute them on
@@ -166,7 +178,7 @@ hipError_t launch_gemm_q8_bf16(const QMat &w, const uint16_t *x, float *y, int64
 bool gemm_bf16_supported(int id, int64_t cols);
 // Workspace the call needs (bytes, at most 32 MiB; 0: none): the partial products of its K splits.
 uint64_t gemm_bf16_workspace_bytes(int id, const QMat &w, int64_t m);
-hipError_t launch_gemm_bf16(int id, const QMat &w, const uint16_t *x, float *y, int64_t m, float *ws, hipStream_t s);
+hipError_t launch_gemm_bf16(int id, const QMat &w, const uint16_t *x, float *y, int64_t m, const Workspace &ws, hipStream_t s);
 hipError_t launch_synth_quant(int id, uint64_t seed, int64_t rows, int64_t cols, uint8_t *gguf,
                               hipStream_t s);
 hipError_t launch_synth_f32(uint64_t seed, int64_t n, float *out, hipStream_t s);

@@ -147,3 +147,40 @@ def test_workspace_call_under_capture_replays(backend):
     for h in (w, x, y, z, nan):
         backend.release(h)
     hip.close()
+
+
+def test_workspaces_of_many_streams(backend):
+    """Streams that take a workspace over from another, one whose work is still queued among them, and one
+    created where another was destroyed: every result is that of a call alone."""
+    b, shapes = 40, [(700, 1024), (4000, 2048)]
+    lib = N.load()
+    ws = [upload(backend, QuantType.Q6_K, r, k, 40 + r) for r, k in shapes]
+    xs = [backend.upload(S.activations_f32(6 + k, b * k), shape=(b, k)) for _, k in shapes]
+    ptr = lambda h: backend.buffer_desc(h).device_ptr
+    ref = []
+    for w, x in zip(ws, xs):
+        y = backend.quant_matvec(w, x)
+        ref.append(backend.download(y).view(np.uint32))
+        backend.release(y)
+    hips = [Hip() for _ in range(3)]
+    results = []
+
+    def call(i, hip):
+        y = backend.upload(np.full((b, shapes[i][0]), np.nan, np.float32))
+        results.append((i, y))
+        backend.quant_matvec_into(ws[i], ptr(xs[i]), 0, ptr(y), b, hip.stream.value)
+
+    for turn in range(4):
+        for k, hip in enumerate(hips):
+            assert lib.j4q_spin(200 * ((k + turn) % 3), hip.stream) == 0
+            call((k + turn) % 2, hip)
+            call((k + turn + 1) % 2, hip)
+        hips[turn % 3].ok("hipStreamDestroy", hips[turn % 3].stream)  # its calls are still queued
+        hips[turn % 3] = Hip()
+        call(turn % 2, hips[turn % 3])
+    for hip in hips:
+        hip.close()
+    for i, y in results:
+        assert np.array_equal(backend.download(y).view(np.uint32), ref[i])
+    for h in [*ws, *xs, *(y for _, y in results)]:
+        backend.release(h)

@@ -81,3 +81,61 @@ def test_kept_memory_is_given_back_before_a_workspace_is_refused(shim, stream):
         result = True, refused
     """)
     assert ok and "out of memory" in refused and "workspace" in refused
+
+
+CALLS = {
+    "matvec": ("zeros(QuantType.Q8_0, 1000, 1024)", "lambda s: be.quant_matvec_into(w, address(4 * 24 * 1024), 0, address(4 * 24 * 1000), 24, s)"),
+    "matvec of several windows": ("zeros(QuantType.Q4_K, 640, 4096)", "lambda s: be.quant_matvec_into(w, address(4 * 16 * 4096), 0, address(4 * 16 * 640), 16, s)"),
+    "matmul": ("zeros(QuantType.Q6_K, 512, 4096)", "lambda s: be.quant_matmul_into(w, address(2 * 64 * 4096), 64, 'bf16', 0, 0, address(4 * 64 * 512), s)"),
+}
+
+
+@pytest.mark.parametrize("name", CALLS)
+@pytest.mark.parametrize("done", [0, 1])
+def test_calls_on_a_callers_stream_keep_their_workspace(shim, name, done):
+    """From the second call on a stream takes no memory, whether the first is done or not, and the last
+    launch completes the event that the next user of the workspace waits for."""
+    make, call = CALLS[name]
+    first, again, waits, last, other, freed = fakehip.run(shim, f"""
+        w, call = {make}, {call}
+        fake.fake_events_done({done})
+        log()
+        call(0x77770)
+        first = log()
+        call(0x77770)
+        again = log()
+        call(0x88880)  # another stream, at the same time or later
+        other = log("malloc", "malloc_async", "wait")
+        call(0)
+        call(0)
+        be.release(w)
+        freed = len(log("free"))
+        result = (len([l for l in first if l.startswith("malloc ")]), len([l for l in again if "alloc" in l or "free" in l]),
+                  [l.split()[1] for l in again if l.startswith("wait")], again[-1].split()[-1], other, freed)
+    """)
+    assert first == 1 and again == 0
+    assert waits == [last]  # the launch's own event, waited for by the call itself
+    assert ["malloc" in l for l in other if "malloc" in l] == ([] if done else [True])
+    assert [l.split()[1] for l in other if "wait" in l] != ([last] if not done else [])
+    assert freed == 2 + (not done) + 1  # with the engine stream's own, and the matrix
+
+
+def test_a_workspace_grows_without_a_wait_for_the_device(shim):
+    """Calls return without synchronising, so a larger one leaves the smaller workspace to later calls."""
+    calls, kept, bound = fakehip.run(shim, """
+        w = zeros(QuantType.Q8_0, 1000, 1024)
+        fake.fake_events_done(0)
+        log()
+        for s in (0, 0x77770):
+            for b in (24, 256, 24):
+                be.quant_matvec_into(w, address(4 * b * 1024), 0, address(4 * b * 1000), b, s)
+        calls = log("malloc", "free", "malloc_async", "device_synchronize")
+        for i in range(400):  # ever more streams, none of them done: the rest take stream-ordered memory
+            be.quant_matvec_into(w, address(4 * 256 * 1024), 0, address(4 * 256 * 1000), 256, 0x100000 + 16 * i)
+        used = fake.fake_used()
+        many = log("malloc_async")
+        be.release(w)
+        result = calls, used, len(many)
+    """)
+    assert len(calls) == 4 and all(c.startswith("malloc ") and c.endswith("ok") for c in calls)
+    assert kept <= (512 << 20) + (16 << 20) and bound > 0
