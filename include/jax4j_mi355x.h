@@ -199,7 +199,8 @@ int j4q_quant_matmul(j4q_buffer weights, j4q_buffer x, int variant, j4q_buffer *
  * windows keeps their partial sums (batch x rows x windows floats), and one above 18 to 34 rows
  * (by type and cols) also x in 4 bytes an element, in a workspace that the engine keeps (on every
  * stream); above 256 MiB, under stream capture, and where the kept ones are all in use, in
- * stream-ordered memory of `stream` (hipMallocAsync / hipFreeAsync). Nothing else is allocated. */
+ * stream-ordered memory of `stream` (hipMallocAsync / hipFreeAsync). Nothing else is allocated.
+ * Under capture a batch over at most 2048 columns takes none and runs in launches of 16 rows. */
 int j4q_quant_matvec_into(j4q_buffer weights, const float *x_dev, const float *add_dev, float *y_dev,
                           int64_t batch, void *stream);
 /* Prefill GEMM into caller memory (the weight types and variants of j4q_quant_matmul).

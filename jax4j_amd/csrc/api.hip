@@ -349,6 +349,20 @@ int64_t matvec_batch(const Buf &w, const Buf &x) {
     return -1;
 }
 
+// The batched GEMV on a workspace of its stream, if there is one to be had. Under capture a workspace is a
+// pair of memory nodes, with which a graph launch waits on the host (8 calls in a graph: 172 us a launch
+// with them, 32 without) and a graph is instantiated only once: a batch that the 16-row launches
+// serve without one takes those there.
+hipError_t run_gemv(int qt, const j4q::QMat &m, const float *x, const float *add, float *y, int64_t batch, hipStream_t s) {
+    j4q::Workspace ws;
+    uint64_t wsb = j4q::gemv_workspace_bytes(qt, m, batch);
+    if (wsb && capturing(s) && !j4q::gemv_window_bytes(qt, m, batch)) wsb = 0;
+    if (wsb && g_workspaces.begin(s, g_stream, wsb, &ws) != hipSuccess) (void)hipGetLastError();
+    const hipError_t e = j4q::launch_gemv(qt, m, x, add, y, batch, s, ws);
+    g_workspaces.end(s, ws, e == hipSuccess);
+    return e;
+}
+
 int matvec_common(j4q_buffer wh, j4q_buffer xh, j4q_buffer addh, j4q_buffer *out, const char *op) {
     if (!out) return fail(J4Q_EINVAL, "%s: out is NULL", op);
     std::lock_guard<std::mutex> lk(g_mu);
@@ -373,12 +387,7 @@ int matvec_common(j4q_buffer wh, j4q_buffer xh, j4q_buffer addh, j4q_buffer *out
     void *ydev;
     if ((rc = alloc_buf(J4Q_KIND_F32, B == 1 ? 1 : 2, B == 1 ? N : B, B == 1 ? 0 : N, (uint64_t)(B * N) * 4, out, &ydev, {x, add})))
         return rc;
-    // for partial sums of a batched call; if there is none to be had, the batch runs without
-    j4q::Workspace ws;
-    const uint64_t wsb = j4q::gemv_workspace_bytes(qt, m, B);
-    if (wsb && g_workspaces.begin(g_stream, g_stream, wsb, &ws) != hipSuccess) (void)hipGetLastError();
-    const hipError_t e = j4q::launch_gemv(qt, m, (const float *)xdev, (const float *)adev, (float *)ydev, B, g_stream, ws);
-    g_workspaces.end(g_stream, ws, e == hipSuccess);
+    const hipError_t e = run_gemv(qt, m, (const float *)xdev, (const float *)adev, (float *)ydev, B, g_stream);
     LAUNCH_INTO(op, out, e);
     return J4Q_OK;
 }
@@ -867,14 +876,7 @@ int j4q_quant_matvec_into(j4q_buffer wh, const float *x, const float *add, float
                     "Q4_0/Q8_0/Q4_K/Q6_K, got cols %lld, batch %lld",
                     (long long)j4q::gemv_single_pass_cols(), (long long)K, (long long)batch);
     if ((rc = ensure_ready())) return rc;
-    const hipStream_t s = pick_stream(stream);
-    // if there is no workspace to be had, the batch runs without
-    j4q::Workspace ws;
-    const uint64_t wsb = j4q::gemv_workspace_bytes(w->qtype, m, batch);
-    if (wsb && g_workspaces.begin(s, g_stream, wsb, &ws) != hipSuccess) (void)hipGetLastError();
-    const hipError_t e = j4q::launch_gemv(w->qtype, m, x, add, y, batch, s, ws);
-    g_workspaces.end(s, ws, e == hipSuccess);
-    HIP_TRY("quantMatvec_into", e);
+    HIP_TRY("quantMatvec_into", run_gemv(w->qtype, m, x, add, y, batch, pick_stream(stream)));
     return J4Q_OK;
 }
 

@@ -422,10 +422,8 @@ bool gemv_in_place_ok(int id, const QMat &m, int64_t batch) {
     return m.cols <= gemv::kMaxWindow || on_matrix_cores(id, m, batch);
 }
 
-uint64_t gemv_workspace_bytes(int id, const QMat &m, int64_t batch) {
+uint64_t gemv_window_bytes(int id, const QMat &m, int64_t batch) {
     if (m.rows <= 0 || !on_matrix_cores(id, m, batch)) return 0;
-    const TileShape t = tile_shape(id, m, batch);
-    if (t.rows) return (uint64_t)t.bytes;
     // launches of 16 rows and, for a remainder of 3..15 rows, one smaller launch
     uint64_t need = mfma_ws_any(id, m, (int)(batch < 16 ? batch : 16));
     const int64_t rem = batch % 16;
@@ -439,6 +437,12 @@ uint64_t gemv_workspace_bytes(int id, const QMat &m, int64_t batch) {
         if (r > need) need = r;
     }
     return need;
+}
+
+uint64_t gemv_workspace_bytes(int id, const QMat &m, int64_t batch) {
+    if (m.rows <= 0 || !on_matrix_cores(id, m, batch)) return 0;
+    const TileShape t = tile_shape(id, m, batch);
+    return t.rows ? (uint64_t)t.bytes : gemv_window_bytes(id, m, batch);
 }
 
 // Threads of the 16-row launch, which takes along one float4 of a job each.

@@ -156,6 +156,8 @@ struct SumJob {
 // launch, or to take the tile kernel (0 when it has one window, or does not run on the matrix
 // cores). With less, launches of 16 rows run, window by window.
 uint64_t gemv_workspace_bytes(int id, const QMat &m, int64_t batch);
+// ... without the tile kernel.
+uint64_t gemv_window_bytes(int id, const QMat &m, int64_t batch);
 // Whether an add that overlaps y is served for this matrix and batch (given the workspace
 // gemv_workspace_bytes asks for): one column window, or the matrix-core path.
 bool gemv_in_place_ok(int id, const QMat &m, int64_t batch);

@@ -139,3 +139,16 @@ def test_a_workspace_grows_without_a_wait_for_the_device(shim):
     """)
     assert len(calls) == 4 and all(c.startswith("malloc ") and c.endswith("ok") for c in calls)
     assert kept <= (512 << 20) + (16 << 20) and bound > 0
+
+
+@pytest.mark.parametrize("cols,nodes", [(1024, False), (2048, False), (4096, True)])
+def test_captured_batches_take_memory_nodes_only_where_16_row_launches_do(shim, cols, nodes):
+    got, tiles = fakehip.run(shim, f"""
+        w = zeros(QuantType.Q6_K, 640, {cols})
+        fake.fake_capture(0x77770, 1)
+        log()
+        be.quant_matvec_into(w, address(4 * 24 * {cols}), 0, address(4 * 24 * 640), 24, 0x77770)
+        lines = log("malloc", "malloc_async", "launch")
+        result = any("malloc" in l for l in lines), any("gemv_tile" in l for l in lines)
+    """)
+    assert got == nodes and tiles == nodes
