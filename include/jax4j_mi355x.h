@@ -200,7 +200,10 @@ int j4q_quant_matmul(j4q_buffer weights, j4q_buffer x, int variant, j4q_buffer *
  * (by type and cols) also x in 4 bytes an element, in a workspace that the engine keeps (on every
  * stream); above 256 MiB, under stream capture, and where the kept ones are all in use, in
  * stream-ordered memory of `stream` (hipMallocAsync / hipFreeAsync). Nothing else is allocated.
- * Under capture a batch over at most 2048 columns takes none and runs in launches of 16 rows. */
+ * Under capture a batch over at most 2048 columns takes none and runs in launches of 16 rows.
+ * Where there is no memory for the workspace a batch runs in launches of 16 rows, one window after
+ * another (with add_dev = y_dev: on the fp32 kernel), whose sums are rounded otherwise within the same
+ * bound; add_dev = y_dev with cols > 32768 then returns J4Q_ENOMEM. */
 int j4q_quant_matvec_into(j4q_buffer weights, const float *x_dev, const float *add_dev, float *y_dev,
                           int64_t batch, void *stream);
 /* Prefill GEMM into caller memory (the weight types and variants of j4q_quant_matmul).

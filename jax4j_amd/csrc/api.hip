@@ -356,11 +356,16 @@ int64_t matvec_batch(const Buf &w, const Buf &x) {
 hipError_t run_gemv(int qt, const j4q::QMat &m, const float *x, const float *add, float *y, int64_t batch, hipStream_t s) {
     j4q::Workspace ws;
     uint64_t wsb = j4q::gemv_workspace_bytes(qt, m, batch);
-    if (wsb && capturing(s) && !j4q::gemv_window_bytes(qt, m, batch)) wsb = 0;
-    if (wsb && g_workspaces.begin(s, g_stream, wsb, &ws) != hipSuccess) (void)hipGetLastError();
+    const uint64_t windows = wsb ? j4q::gemv_window_bytes(qt, m, batch) : 0;
+    if (wsb && !windows && capturing(s)) wsb = 0;
+    // no memory: the 16-row launches' smaller workspace, or theirs window by window without one, and
+    // the fp32 kernel where add is y; what needs a workspace even so reports the missing memory
+    hipError_t none = hipSuccess;
+    if (wsb) none = g_workspaces.begin(s, g_stream, wsb, &ws);
+    if (none != hipSuccess && windows && windows < wsb && g_workspaces.begin(s, g_stream, windows, &ws) == hipSuccess) none = hipSuccess;
     const hipError_t e = j4q::launch_gemv(qt, m, x, add, y, batch, s, ws);
     g_workspaces.end(s, ws, e == hipSuccess);
-    return e;
+    return e == hipErrorInvalidValue && none != hipSuccess ? none : e;
 }
 
 int matvec_common(j4q_buffer wh, j4q_buffer xh, j4q_buffer addh, j4q_buffer *out, const char *op) {

@@ -481,12 +481,12 @@ hipError_t launch_gemv(int id, const QMat &m, const float *x, const float *add, 
     // with the workspace, several windows meet in sum_windows_kernel, which reads each add
     // element before it writes y there; without it they are chained launches that would
     // read an add overlapping y after rewriting y, so such a call keeps one window
-    const bool ws_ok = mfma && ws.ptr && ws.bytes >= gemv_workspace_bytes(id, m, batch);
-    if (in.part && !(gemv_carries(id, m, batch, in) && (ws_ok || gemv_workspace_bytes(id, m, batch) == 0)))
+    const bool ws_ok = mfma && ws.ptr && ws.bytes >= gemv_window_bytes(id, m, batch);
+    if (in.part && !(gemv_carries(id, m, batch, in) && (ws_ok || gemv_window_bytes(id, m, batch) == 0)))
         return hipErrorInvalidValue;
     if (ws_ok) {
         const TileShape t = tile_shape(id, m, batch);
-        if (t.rows) return launch_tile(id, m, x, add, y, batch, t, ws, s);
+        if (t.rows && ws.bytes >= (uint64_t)t.bytes) return launch_tile(id, m, x, add, y, batch, t, ws, s);
     }
     if (!mfma || (alias && !ws_ok && !single_window<8>(m))) {
         if (alias && m.cols > gemv::kMaxWindow) return hipErrorInvalidValue;

@@ -108,7 +108,10 @@ public:
             give_back();
             e = hipMallocAsync(&p, bytes, s);
         }
-        if (e != hipSuccess) return e;
+        if (e != hipSuccess) {
+            (void)hipGetLastError();  // a launch checks for errors by the last one
+            return e;
+        }
         ws->ptr = (float *)p;
         ws->bytes = bytes;
         ws->stream_ordered = true;

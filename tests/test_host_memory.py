@@ -152,3 +152,32 @@ def test_captured_batches_take_memory_nodes_only_where_16_row_launches_do(shim, 
         result = any("malloc" in l for l in lines), any("gemv_tile" in l for l in lines)
     """)
     assert got == nodes and tiles == nodes
+
+
+# 24 rows of Q8_0 over 1024 columns (one window of 16-row launches) and over 4096, and 16 rows over 4096
+@pytest.mark.parametrize("batch,cols,smaller", [(24, 1024, False), (24, 4096, True), (16, 4096, False)])
+def test_batches_run_without_memory_for_a_workspace(shim, batch, cols, smaller):
+    kernels, kernels_some, in_place = fakehip.run(shim, f"""
+        w = zeros(QuantType.Q8_0, 640, {cols})
+        x, y = address(4 * {batch * cols}), address(4 * {batch} * 640)
+        def names(add, free):
+            fake.fake_capacity(fake.fake_used() + free)
+            log()
+            be.quant_matvec_into(w, x, add, y, {batch}, 0x77770)
+            return [l.split()[1] for l in log("launch")]
+        result = names(0, 0), names(0, 2 * 16 * 640 * 4), names(y, 0)
+    """)
+    assert kernels and all("gemv_mfma" in k or "gemv_kernel" in k for k in kernels)  # no sum of windows
+    assert any("sum_windows" in k for k in kernels_some) == (cols > 2048)
+    assert not any("gemv_tile" in k for k in kernels + kernels_some + in_place) and in_place
+
+
+def test_a_batch_that_needs_its_workspace_reports_the_missing_memory(shim):
+    message, code = fakehip.run(shim, """
+        w = zeros(QuantType.Q8_0, 64, 40960)
+        x, y = address(4 * 24 * 40960), address(4 * 24 * 64)
+        fake.fake_capacity(0)
+        code = lib.j4q_quant_matvec_into(w.handle, x, y, y, 24, None)
+        result = N.last_error(), code
+    """)
+    assert code == 5 and "out of memory" in message  # J4Q_ENOMEM
