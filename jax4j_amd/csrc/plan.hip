@@ -22,6 +22,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "engine.h"
@@ -59,9 +60,10 @@ struct Op {
 struct Plan {
     j4q_decode_plan_desc desc{};
     int64_t batch = 0;
-    // partial sums of batched GEMVs over several column windows (plan-owned): two, since those of a
-    // launch may stay until the next one has its own
+    // partial sums of batched GEMVs over several column windows (plan-owned): two at 9..16 rows, since
+    // those of a launch may stay until the next one has its own
     Workspace ws[2];
+    int workspaces = 0;
     std::vector<Op> ops;
     std::vector<void *> owned;
     // caller buffers whose memory the graph reads (o, down, the head, and group parts that were
@@ -117,7 +119,7 @@ hipError_t enqueue(const Plan &p, hipStream_t s) {
         }
         if (o.gemv) {
             SumJob left;
-            e = launch_gemv(o.qt, o.m, o.x, o.add, o.y, p.batch, s, p.ws[w], along ? job : SumJob(), o.last ? &left : nullptr);
+            e = launch_gemv(o.qt, o.m, o.x, o.add, o.y, p.batch, s, p.ws[w], along ? job : SumJob(), o.last && p.workspaces == 2 ? &left : nullptr);
             if (left.part) w ^= 1;
             job = left;
         } else {
@@ -316,21 +318,29 @@ int j4q_decode_plan_create(const j4q_decode_layer *layers, int32_t n_layers, j4q
         if (!rc) rc = one_gemv(p, L.down, "decode plan down", io->x_down, h_alt, h);
     }
     if (!rc && head) rc = one_gemv(p, head, "decode plan head", h, nullptr, io->logits);
-    uint64_t wsb = 0;
+    uint64_t wsb = 0, windows = 0;  // of the largest GEMV, and with its rows of x in 16-row launches
     for (const Op &o : p.ops) {
-        const uint64_t b = o.gemv ? gemv_workspace_bytes(o.qt, o.m, batch) : 0;
-        if (b > wsb) wsb = b;
+        if (!o.gemv) continue;
+        wsb = std::max(wsb, gemv_workspace_bytes(o.qt, o.m, batch));
+        windows = std::max(windows, gemv_window_bytes(o.qt, o.m, batch));
     }
     if (!rc && wsb) {
-        const int n = batch >= 9 && batch <= 16 ? 2 : 1;
+        int n = batch >= 9 && batch <= 16 ? 2 : 1;
         void *d = nullptr;
         e = abi::malloc_locked(&d, n * align256(wsb));
+        if (e == hipErrorOutOfMemory && (n > 1 || windows < wsb)) {  // the least that the launches do with
+            (void)hipGetLastError();
+            n = 1;
+            wsb = windows;
+            e = wsb ? abi::malloc_locked(&d, align256(wsb)) : hipSuccess;
+        }
         if (e != hipSuccess) {
             rc = report_hip("decode plan workspace", e);
-        } else {
+        } else if (wsb) {
             p.owned.push_back(d);
-            for (int i = 0; i < 2; i++) {
-                p.ws[i].ptr = (float *)((uint8_t *)d + (i < n ? i * align256(wsb) : 0));
+            p.workspaces = n;
+            for (int i = 0; i < n; i++) {
+                p.ws[i].ptr = (float *)((uint8_t *)d + i * align256(wsb));
                 p.ws[i].bytes = wsb;
             }
             p.desc.plan_bytes += n * align256(wsb);

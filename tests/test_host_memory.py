@@ -181,3 +181,30 @@ def test_a_batch_that_needs_its_workspace_reports_the_missing_memory(shim):
         result = N.last_error(), code
     """)
     assert code == 5 and "out of memory" in message  # J4Q_ENOMEM
+
+
+@pytest.mark.parametrize("batch", [12, 16, 30, 40])
+def test_decode_plans_are_made_with_the_memory_of_16_row_launches(shim, batch):
+    """Where there is no memory for more, a plan runs its sums as launches of their own and its batches in
+    launches of 16 rows."""
+    full, small, jobs = fakehip.run(shim, f"""
+        d, kv, ffn, b = 4096, 1024, 4096, {batch}
+        z = lambda r, c: zeros(QuantType.Q4_K, r, c)
+        layers = [dict(q=z(d, d), k=z(kv, d), v=z(kv, d), o=z(d, d), gate=z(ffn, d), up=z(ffn, d), down=z(d, ffn)) for _ in range(2)]
+        io = dict(h=address(4 * b * d), x_o=address(4 * b * d), x_down=address(4 * b * ffn), qkv=address(8 * b * (d + 2 * kv)),
+                  gate_up=address(16 * b * ffn), logits=0)
+        log()
+        plan = be.decode_plan(layers, None, b, io)
+        full = [l.split()[1] for l in log("launch")]
+        size = plan.info()["plan_bytes"]
+        plan.destroy()
+        fake.fake_capacity(fake.fake_used() + size - 4096)
+        log()
+        plan = be.decode_plan(layers, None, b, io)
+        small = [l.split()[1] for l in log("launch")]
+        assert plan.info()["plan_bytes"] < size
+        # a job's launches are kernels whose last argument's condition holds
+        result = len(full), len(small), [sum("Lb1EEEvNS_4QMat" in k for k in ks) for ks in (full, small)]
+    """)
+    assert small > full
+    assert jobs[1] == 0 and (jobs[0] > 0) == (batch <= 16)
