@@ -748,6 +748,9 @@ hipError_t launch_k(const QMat &m, const float *x, const float *add, float *y, i
     float *const ws = windows > 1 ? part : nullptr;
     const dim3 g(grid, windows);
     if constexpr (BB == 16) {
+        // LDS admits one workgroup per CU, so the job's registers (up to 8 more) do not change how many are
+        // resident: grids sized by the kernel without a job fit the one with it.
+        static_assert(2 * lds > 160 * 1024 && WAVES == 8, "one workgroup per CU, of up to 256 registers");
         if (job.part) {
             gemv_mfma_kernel<FMT, BB, WAVES, IPW, XREG, TS, NB, true><<<g, WAVES * 64, lds, s>>>(m, x, prev, add, y, B, kb0, per, nbe, ws, job);
             return hipGetLastError();
