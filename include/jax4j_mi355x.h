@@ -167,8 +167,10 @@ int j4q_quant_dequantize(j4q_buffer weights, j4q_buffer *y);
  *  J4Q_GEMV_MATRIX_CORES (default): launches of up to 16 batch rows, or tiles of 32 or 64 where
  *    there are more (from 19 to 35 rows on, by type and cols), on the matrix cores (Q8_0, Q4_0,
  *    Q4_K, Q6_K), W streamed once per launch or tile; x enters the products as hi + lo fp16
- *    (22 significant bits under a power-of-two scale), the products are exact, and each row
- *    stays within 1e-4 of the fp64 product (within 4e-5 up to K = 40960 in the tests);
+ *    under a power-of-two scale per slice of 256 (up to 16 rows: 512) to 1024 columns (22 significant
+ *    bits; fewer for elements more than 2^12 below the slice's largest, an error of at most 2^-35 of
+ *    it), the products are exact, and each row stays within 1e-4 of the fp64 product (within 4e-5
+ *    up to K = 40960 in the tests);
  *  J4Q_GEMV_FP32: every batch row on the batch-1 kernel (fp32 x, fp32 accumulation, no
  *    matrix cores; W streamed once per row), so row b equals quantMatvec of x[b] bit for bit.
  * Process-wide, for every call issued afterwards; a decode plan keeps the launches it

@@ -334,7 +334,7 @@ TileShape tile_shape(int id, const QMat &m, int64_t batch) {
     per = per < 8 ? 8 : per > 16 ? 16 : per;
     const int64_t splits = (stages + per - 1) / per;
     // Chunks of up to 256 rows, of fewer where the partial sums would pass kTileWorkspace.
-    const int64_t row_bytes = K * 4 + 4 + (id == Q4_K ? K / 8 : 0) + (splits > 1 ? splits * N * 4 : 0);
+    const int64_t row_bytes = K * 4 + splits * 4 + (id == Q4_K ? K / 8 : 0) + (splits > 1 ? splits * N * 4 : 0);
     int64_t rows = batch < 256 ? batch : 256;
     if (rows * row_bytes > kTileWorkspace) rows = kTileWorkspace / row_bytes;
     if (rows < batch && rows > 32) rows = rows / 32 * 32;
@@ -349,7 +349,7 @@ TileShape tile_shape(int id, const QMat &m, int64_t batch) {
     t.splits = (int)splits;
     t.split_stages = per;
     t.x_bytes = (int64_t)align256((uint64_t)(rows * K * 4));
-    t.scale_bytes = (int64_t)align256((uint64_t)rows * 4);
+    t.scale_bytes = (int64_t)align256((uint64_t)(rows * splits) * 4);
     t.sum_bytes = id == Q4_K ? (int64_t)align256((uint64_t)(rows * (K / 32) * 4)) : 0;
     t.bytes = t.x_bytes + t.scale_bytes + t.sum_bytes + (splits > 1 ? splits * rows * N * 4 : 0);
     return t;
@@ -368,8 +368,8 @@ hipError_t launch_tile_fmt(const QMat &m, const float *x, const float *add, floa
         const int rows = (int)(batch - b0 < t.rows ? batch - b0 : t.rows);
         const float *const ab = add ? add + b0 * m.rows : nullptr;
         float *const yb = y + b0 * m.rows;
-        if (K <= 8192) gvt::split_x_kernel<FMT != Q8_0, 2><<<rows, 1024, 0, s>>>(x + b0 * K, K, hi, (int64_t)rows * K, unscale, sums);
-        else gvt::split_x_kernel<FMT != Q8_0, 8><<<rows, 1024, 0, s>>>(x + b0 * K, K, hi, (int64_t)rows * K, unscale, sums);
+        gvt::split_x_kernel<FMT != Q8_0><<<dim3((unsigned)rows, (unsigned)t.splits), 256, 0, s>>>(
+            x + b0 * K, K, t.split_stages, hi, (int64_t)rows * K, unscale, sums);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         const unsigned tiles = (unsigned)(((rows + 32 * t.tm - 1) / (32 * t.tm)) * ((m.rows + 127) / 128));

@@ -10,8 +10,12 @@
 // cores are busy 18 of 61 us, the vector units about 20, and the two waves of a SIMD overlap them
 // only in part; without its loads it takes 45.
 //
-// Arithmetic (as gemv_mfma.h): x is scaled per row by a power of two 2^e (max |x| 2^e over the row
-// in [2^14, 2^15)) and split into hi + lo fp16 (22 significant bits) by split_x_kernel; the codes
+// Arithmetic (as gemv_mfma.h): x is scaled per row and K split by a power of two 2^e (max |x| 2^e over
+// the split's 512 to 1024 columns of the row in [2^14, 2^15)) and split into hi + lo fp16 by
+// split_x_kernel: 22 significant bits for elements down to 2^-16 of that maximum (2^-12 for elements
+// 16..31 of a 4- or 6-bit block, stored times 1/16), below it an absolute error of up to 2^-39 (2^-35)
+// of the maximum. The error of a row's sums hardly shows it, but that of an output whose weight at a far
+// larger element is zero; other splits' sums do not depend on that element. The codes
 // enter the MFMA as exact fp16 integers (Q4_K's as subnormals q 2^-24), so products are exact; each
 // block's sum C = sum q' x' comes out of the matrix core and one FMA with the block's fp32 scale
 // folds it into the accumulator. Codes of Q8_0, Q4_0 and Q6_K carry their offset (q - 8, q - 32);
@@ -50,36 +54,24 @@ typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 
-// Row blockIdx.x of x [rows, K] as hi and lo fp16 of x 2^e in the layout above (lo `lo_off` halves
-// after hi), 2^-e to unscale, and with sums the sums of x 2^e over every 32-block. K % 64 == 0.
-// G: 4-element groups per thread that stay in registers between the two passes (the maximum, the
-// conversion); a row of more than 1024 G groups is read twice. One workgroup per row: what bounds it
-// is the memory latency, paid once instead of twice per 1024 columns (61 rows of 14336 columns with
-// 256 threads reading twice: 11.6 us).
-template <bool SIXTEENTH, int G>
-__global__ void __launch_bounds__(1024)
-split_x_kernel(const float *__restrict__ x, int K, _Float16 *__restrict__ hi, int64_t lo_off, float *__restrict__ unscale,
+// Columns [64 per s, 64 per (s + 1)) of row r of x [rows, K], r = blockIdx.x, s = blockIdx.y, as hi and lo
+// fp16 in the layout above (lo `lo_off` halves after hi), 2^-e to unscale[s rows + r], and with sums
+// the sums of x 2^e over every 32-block. K % 64 == 0, per <= 16: a thread per 4 elements. What bounds
+// it is the memory latency, paid once: x stays in registers between the maximum and the conversion.
+template <bool SIXTEENTH>
+__global__ void __launch_bounds__(256)
+split_x_kernel(const float *__restrict__ x, int K, int per, _Float16 *__restrict__ hi, int64_t lo_off, float *__restrict__ unscale,
                float *__restrict__ sums) {
-    __shared__ float wmax[16];
-    const int tid = (int)threadIdx.x, groups = K / 4;
-    const f32x4 *const xr = reinterpret_cast<const f32x4 *>(x + (int64_t)blockIdx.x * K);
-    f32x4 own[G];
-#pragma unroll
-    for (int g = 0; g < G; g++) own[g] = tid + 1024 * g < groups ? xr[tid + 1024 * g] : f32x4{};
-    float v = 0.f;
-    auto max4 = [&](const f32x4 &a) __attribute__((always_inline)) {
-        v = fmaxf(v, fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(a.w))));
-    };
-#pragma unroll
-    for (int g = 0; g < G; g++) max4(own[g]);
-    for (int i = tid + 1024 * G; i < groups; i += 1024) max4(xr[i]);
+    __shared__ float wmax[4];
+    const int tid = (int)threadIdx.x, i = 16 * per * (int)blockIdx.y + tid;  // this thread's 4 elements
+    const bool in = tid < 16 * per && i < K / 4;
+    const f32x4 raw = in ? reinterpret_cast<const f32x4 *>(x + (int64_t)blockIdx.x * K)[i] : f32x4{};
+    float v = fmaxf(fmaxf(fabsf(raw.x), fabsf(raw.y)), fmaxf(fabsf(raw.z), fabsf(raw.w)));
 #pragma unroll
     for (int o = 32; o > 0; o /= 2) v = fmaxf(v, __shfl_xor(v, o));
     if ((tid & 63) == 0) wmax[tid >> 6] = v;
     __syncthreads();
-    v = wmax[0];
-#pragma unroll
-    for (int k = 1; k < 16; k++) v = fmaxf(v, wmax[k]);
+    v = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
     int e = 0;
     if (v > 0.f && v <= 3.402823466e38f) {
         int E;
@@ -88,28 +80,22 @@ split_x_kernel(const float *__restrict__ x, int K, _Float16 *__restrict__ hi, in
         e = e < -126 ? -126 : (e > 127 ? 127 : e);
     }
     const float sx = ldexpf(1.0f, e);
-    if (tid == 0) unscale[blockIdx.x] = ldexpf(1.0f, -e);
-    h4 *const hr = reinterpret_cast<h4 *>(hi + (int64_t)blockIdx.x * K);
-    h4 *const lr = reinterpret_cast<h4 *>(hi + lo_off + (int64_t)blockIdx.x * K);
-    auto split = [&](int i, const f32x4 &raw) __attribute__((always_inline)) {
-        const f32x4 a = raw * sx;
-        const f32x4 b = SIXTEENTH && (i & 4) ? a * 0.0625f : a;
-        const h4 h = __builtin_convertvector(f32x4{b.x, b.z, b.y, b.w}, h4);
-        const f32x4 back = __builtin_convertvector(h, f32x4);
-        hr[i] = h;
-        lr[i] = __builtin_convertvector(f32x4{b.x, b.z, b.y, b.w} - back, h4);
-        if (sums) {  // the 8 lanes of a block (K % 32 == 0: all of them are here)
-            float s = (a.x + a.y) + (a.z + a.w);
-            s += __shfl_xor(s, 1);
-            s += __shfl_xor(s, 2);
-            s += __shfl_xor(s, 4);
-            if ((i & 7) == 0) sums[(int64_t)blockIdx.x * (K / 32) + (i >> 3)] = s;
-        }
-    };
-#pragma unroll
-    for (int g = 0; g < G; g++)
-        if (tid + 1024 * g < groups) split(tid + 1024 * g, own[g]);
-    for (int i = tid + 1024 * G; i < groups; i += 1024) split(i, xr[i]);
+    if (tid == 0) unscale[blockIdx.y * gridDim.x + blockIdx.x] = ldexpf(1.0f, -e);
+    if (!in) return;
+    const f32x4 a = raw * sx;
+    const f32x4 b = SIXTEENTH && (i & 4) ? a * 0.0625f : a;
+    const h4 h = __builtin_convertvector(f32x4{b.x, b.z, b.y, b.w}, h4);
+    const f32x4 back = __builtin_convertvector(h, f32x4);
+    const int64_t o = (int64_t)blockIdx.x * (K / 4) + i;
+    reinterpret_cast<h4 *>(hi)[o] = h;
+    reinterpret_cast<h4 *>(hi + lo_off)[o] = __builtin_convertvector(f32x4{b.x, b.z, b.y, b.w} - back, h4);
+    if (sums) {  // the 8 lanes of a block (K % 32 == 0: all of them are here)
+        float t = (a.x + a.y) + (a.z + a.w);
+        t += __shfl_xor(t, 1);
+        t += __shfl_xor(t, 2);
+        t += __shfl_xor(t, 4);
+        if ((i & 7) == 0) sums[o >> 3] = t;
+    }
 }
 
 template <int FMT, int TM>
@@ -371,7 +357,7 @@ gemv_tile(QMat w, const uint16_t *__restrict__ xs, const float *__restrict__ uns
             if (row < B) {
                 float r = acc[t][v];
                 if constexpr (MIN) r -= corr[t][v];
-                r *= unscale[row];
+                r *= unscale[(int)blockIdx.y * B + row];
                 const int64_t o = (int64_t)row * N + col;
                 out[o] = !part && add ? r + add[o] : r;
             }

@@ -36,8 +36,7 @@ def matvec(backend, w, xs):
 # Rows of x at the first of each rule, full and ragged tiles of 32 and (the last two, and 65 x 20001)
 # of 64, and past a chunk of 256;
 # rows of W around a tile of 128; K of one split (512), of unequal splits (768: 512 + 256; 5120: 5 of
-# 1024; 2816: 768 three times and 512), of x rows kept in 2 (to 8192) and 8 (to 32768) groups and past
-# them (33024).
+# 1024; 2816: 768 three times and 512), of many splits (9216, 33024).
 SHAPES = [(19, 129, 512), (27, 127, 5120), (32, 300, 768), (33, 1, 2816), (35, 257, 2048), (64, 128, 512),
           (65, 130, 768), (257, 70, 512), (35, 40, 9216), (36, 33, 33024), (257, 12500, 512), (130, 5001, 2816)]
 
@@ -99,3 +98,35 @@ def test_gemv_tile_sums_do_not_depend_on_the_launch(backend, qt):
         assert np.abs(got - want).max() <= 2.0**-23 * np.abs(want).max()
     for h in (*ws, both):
         backend.release(h)
+
+
+# (bytes of a block, offset of its scales, their bytes)
+SCALES = {QuantType.Q8_0: (34, 0, 2), QuantType.Q4_0: (18, 0, 2), QuantType.Q4_K: (144, 0, 4), QuantType.Q6_K: (210, 208, 2)}
+
+
+@pytest.mark.parametrize("qt", ALL, ids=lambda q: q.name)
+@pytest.mark.parametrize("large", [3.0e5, 3.0e12])
+def test_a_large_element_of_x_costs_other_splits_no_bits(backend, qt, large):
+    """x is scaled per K split (2816 columns: 768 three times and 512). Where the weights of the first split are
+    zero, an element of x there changes nothing. Where they are zero in its block alone, the others of
+    its split keep an absolute error of 2^-35 of it, and of 2^-22 of themselves."""
+    b, n, k = 40, 200, 2816
+    bb, at, nb = SCALES[qt]
+    x = S.activations_f32(3, b * k).reshape(b, k)
+    x[:, 5] = 0
+    xl = x.copy()
+    xl[:, 5] = large
+    for cols in (768, qt.block_elements):
+        blocks = S.quant_blocks(qt, 77, n, k).reshape(n, k // qt.block_elements, bb).copy()
+        blocks[:, :cols // qt.block_elements, at:at + nb] = 0
+        w = backend.upload_quantized(blocks.reshape(-1), qt, (n, k))
+        got, plain = matvec(backend, w, xl), matvec(backend, w, x)
+        if cols == 768:
+            assert np.array_equal(bits(got), bits(plain))
+        wf = np.abs(oracle.dequant_matrix(qt.id, blocks.reshape(-1), n, k).astype(np.float64))
+        ref = oracle.matmul_f64(qt.id, blocks.reshape(-1), n, k, xl)
+        # Q4_K's products of codes and of mins are each up to 16 times their difference
+        size = (16 if qt is QuantType.Q4_K else 1) * (2.0**-22 * (np.abs(x).astype(np.float64) @ wf.T) + 2.0**-35 * large * wf[:, :768].sum(axis=1))
+        bar = 4e-5 if qt is QuantType.Q4_K else 1e-5
+        assert (np.abs(got - ref) <= bar * np.abs(ref).max(axis=1, keepdims=True) + size).all()
+        backend.release(w)
