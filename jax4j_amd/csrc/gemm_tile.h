@@ -1,4 +1,4 @@
-// Prefill GEMM, bf16 variant, for grids that fill the GPU: Y[M, N] = X[M, K] . bf16(W)[N, K]^T
+// Prefill GEMM, bf16 variant: Y[M, N] = X[M, K] . bf16(W)[N, K]^T
 // with fp32 accumulation, W the exactly decoded weights of Q8_0, Q4_0, Q4_K or Q6_K blocks
 // (semantics: quantMatvec per row of X, QuantizedOps.java:27 / CpuBackend.java:708-725).
 //
@@ -6,7 +6,8 @@
 //  - Tile 32 TM x 32 WV per workgroup of WV waves. Wave w owns columns [32 w, +32) for all rows:
 //    TM v_mfma_f32_32x32x16_bf16 accumulators, no partial tiles to add at the end. With WV = 4
 //    two workgroups share a CU (one's barriers, prologue and stores are covered by the other's
-//    matrix work); with WV = 8 the two waves of a SIMD share X.
+//    matrix work); with WV = 8 the two waves of a SIMD share X. Small grids: WV = 2 and KG groups
+//    of such waves in a workgroup, which split its range of K.
 //  - K advances in stages of two 32-blocks. Lane (r, h) = (lane % 32, lane / 32) supplies block
 //    h of the stage, elements 8 p .. 8 p + 7 to the stage's MFMA p = 0..3, for A (X) and B (W)
 //    alike: every lane dequantizes one whole block of one W row, so the scale decode is paid
@@ -155,11 +156,11 @@ struct Tile {
     static constexpr int XL = 4 * TM / WV;  // X loads per wave and stage
     static constexpr int kX = BM * 128;
     static_assert(4 * TM % WV == 0, "whole X loads per wave");
-    static_assert(2 * (kX + WUnit<FMT, WV>::kBytes) <= 163840, "LDS");
 };
 
-// KG = 2: two groups of WV waves, each with buffers of its own, take a half of the range of K each
-// (split_stages, a multiple of 4; K a multiple of 256), and the second's sums go to the first through LDS.
+// KG = 2 or 4 (WV = 2): as many groups of waves, each with buffers of its own, take a part of the range of K
+// each (split_stages, a multiple of 4; K a multiple of 256). Their sums meet through LDS, a quarter of
+// the rows of a 32-row tile or a half in each group, and are added in group order.
 template <int FMT, int WV, int TM, int KG = 1>
 __global__ void __launch_bounds__(64 * WV * KG, 2)
 gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, int split_stages,
@@ -167,6 +168,7 @@ gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, 
     using T = Tile<FMT, WV, TM>;
     using U = WUnit<FMT, WV>;
     constexpr int BM = T::BM, BN = T::BN, QR = U::QR, WL = U::kLoads, XL = T::XL;
+    static_assert(2 * KG * (T::kX + U::kBytes) <= 163840, "LDS");
     __shared__ __attribute__((aligned(1024))) uint8_t xs0[KG * T::kX], xs1[KG * T::kX];
     __shared__ __attribute__((aligned(1024))) uint8_t ws0[KG * U::kBytes], ws1[KG * U::kBytes];
     const int N = (int)w.rows, K = (int)w.cols;
@@ -360,30 +362,42 @@ gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, 
     }
 #undef J4Q_STAGE
     __builtin_amdgcn_s_waitcnt(0);  // no LDS load outlives the workgroup
-    if constexpr (KG == 2) {
-        // The second group's sums through the X buffers (which hold them exactly); the first adds them.
-        typedef float f32x8 __attribute__((ext_vector_type(8)));
-        f32x8 *const r0 = reinterpret_cast<f32x8 *>(xs0), *const r1 = reinterpret_cast<f32x8 *>(xs1);
-        __syncthreads();
-        if (kg) {
-#pragma unroll
-            for (int t = 0; t < TM; t++) {
-                r0[(t * WV + wave) * 64 + lane] = __builtin_shufflevector(acc[t], acc[t], 0, 1, 2, 3, 4, 5, 6, 7);
-                r1[(t * WV + wave) * 64 + lane] = __builtin_shufflevector(acc[t], acc[t], 8, 9, 10, 11, 12, 13, 14, 15);
-            }
-        }
-        __syncthreads();
-        if (kg) return;
-#pragma unroll
-        for (int t = 0; t < TM; t++) {
-            const f32x8 a = r0[(t * WV + wave) * 64 + lane], b = r1[(t * WV + wave) * 64 + lane];
-            acc[t] += __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
-        }
-    }
-
     // Result element v of tile t: row 32 t + 8 (v / 4) + 4 h + v % 4, column r32.
     float *const out = part ? part + (int64_t)blockIdx.y * M * N : y;
     const int col = nw + r32;
+    if constexpr (KG > 1) {
+        // elements 4 q .. 4 q + 3 of the tiles: through the X buffers, two quarters in each, which hold them exactly
+        static_assert((KG == 2 || KG == 4) && WV == 2, "quarters of the sums of all groups in the X buffers");
+        typedef float f32x4 __attribute__((ext_vector_type(4)));
+        auto at = [&](int g, int t, int q) __attribute__((always_inline)) -> f32x4 & {
+            return reinterpret_cast<f32x4 *>(q < 2 ? xs0 : xs1)[(((g * TM + t) * 2 + (q & 1)) * WV + wave) * 64 + lane];
+        };
+        auto quarter = [&](int t, int q) __attribute__((always_inline)) {
+            return f32x4{acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]};
+        };
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < TM; t++)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (q / (4 / KG) != kg) at(kg, t, q) = quarter(t, q);
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < TM; t++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                if (q / (4 / KG) != kg) continue;
+                f32x4 s = kg == 0 ? quarter(t, q) : at(0, t, q);
+#pragma unroll
+                for (int g = 1; g < KG; g++) s += kg == g ? quarter(t, q) : at(g, t, q);
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int row = m0 + 32 * t + 8 * q + 4 * h + v;
+                    if (row < M && col < N) out[(int64_t)row * N + col] = s[v];
+                }
+            }
+        return;
+    }
 #pragma unroll
     for (int t = 0; t < TM; t++)
 #pragma unroll

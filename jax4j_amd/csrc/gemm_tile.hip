@@ -10,7 +10,7 @@ namespace {
 // split_stages 64-element stages. tm = 0: the call does not run on it.
 struct Shape {
     int waves = 0, tm = 0, splits = 1, split_stages = 0;
-    int groups = 1;  // 2: each workgroup's two groups of waves take a half of K each, split_stages long
+    int groups = 1;  // of waves in a workgroup, each with split_stages of K
 };
 
 // The tiles, and what one stage of one workgroup takes in us on MI355X: few workgroups, each
@@ -24,13 +24,26 @@ struct Cost {
 constexpr Cost kCost[] = {{4, 1, .33f, .38f, .26f}, {4, 2, .38f, .43f, .34f}, {4, 3, .45f, .50f, .43f},
                           {4, 4, .47f, .57f, .51f}, {4, 5, .58f, .68f, .63f}, {8, 4, .62f, 1.02f, 1.0f},
                           {8, 8, 1.2f, 1.75f, 1.75f}};
+// Workgroups of two or four K groups of two waves, one per CU: what the launch, the prologue and the sums
+// of the groups take, and a stage of all groups, as above; Q6_K's decoding comes on top. Fitted to 162
+// sizes (N = 350 .. 15000, K = 512 .. 14336, M = 4 .. 1500). us a call of the 64-column kernel of 8 waves that
+// was here before, of the shapes above, and of these: Q4_K 950 x 1040 x 2560 16.9, 17.2, 12.4; 17 x 2267 x 768
+// 5.4, 6.6, 5.3; 24 x 14336 x 4096 18.2, 15.7, 12.6; 128 x 4096 x 2048 23.0, 11.7, 8.2; Q6_K 950 x 1040 x 2560
+// 16.7, 19.2, 14.0.
+struct Group {
+    int tm, groups;
+    float base, few, all, q6_few, q6_all;
+};
+constexpr Group kGroups[] = {{1, 2, 2.73f, .326f, .393f, .054f, .074f}, {2, 2, 3.16f, .378f, .451f, .074f, .094f},
+                             {1, 4, 2.94f, .488f, .605f, .142f, .183f}, {2, 4, 3.41f, .588f, .727f, .150f, .205f},
+                             {3, 4, 3.79f, .699f, .95f, .145f, .15f}};
 constexpr int kCus = 256;  // of an MI355X; a constant, so that results do not depend on the device
 
 // The fastest shape by a model of the launch: the stages that the busiest CU runs (Q6_K's take
 // longer to decode, Q8_0's to load), a launch's fixed 3 us, and with K split the sum kernel: 2 us,
 // a quarter per split, and its traffic (the partial products written and read, the result written)
 // at 5.5 MB/us. Over the sweeps (38 sizes) its choice takes 1.2 % longer than the best of all
-// shapes on average, 11 % at worst. Splits are whole multiples of four stages, and their workspace
+// shapes on average, 11 % at worst (with the groups of kGroups, 162 sizes: 0.5 %). Splits are whole multiples of four stages, and their workspace
 // is at most 32 MiB; a Q8_0 call takes no workspace, so it does not split.
 Shape pick(int id, const QMat &w, int64_t m, float *us_out) {
     const int64_t n = w.rows, ns = w.cols / 64;
@@ -54,17 +67,17 @@ Shape pick(int id, const QMat &w, int64_t m, float *us_out) {
             }
         }
     }
-    // Few tiles without the sum kernel: two groups of four waves in a workgroup, half of K each
-    // (950 x 1040 x 2560 Q4_K 19.8 -> 17.3 us, 500 x 1040 x 2560 16.8 -> 14.3, 600 x 2000 x 2048 Q6_K 20.8 -> 17.0).
+    // At most a tile per CU without the sum kernel: tiles of 64 columns, K in two or four groups of two waves
+    // of a workgroup (kGroups).
     if (id != Q8_0 && ns % 4 == 0) {
-        constexpr Cost kTwo[] = {{4, 1, .45f, .56f, 0.f}, {4, 2, .58f, .70f, 0.f}};
-        for (const Cost &c : kTwo) {
-            const int64_t tiles = ((m + 32 * c.tm - 1) / (32 * c.tm)) * ((n + 127) / 128), per = ((ns + 1) / 2 + 3) / 4 * 4;
+        for (const Group &c : kGroups) {
+            const int64_t tiles = ((m + 32 * c.tm - 1) / (32 * c.tm)) * ((n + 63) / 64), per = ((ns + c.groups - 1) / c.groups + 3) / 4 * 4;
             if (tiles > kCus) continue;
-            const float us = (c.few + (c.all - c.few) * (float)tiles / kCus + (id == Q6_K ? .32f : 0.f)) * (float)per + 3.5f;
+            const float few = c.few + (id == Q6_K ? c.q6_few : 0.f), all = c.all + (id == Q6_K ? c.q6_all : 0.f);
+            const float us = (few + (all - few) * (float)tiles / kCus) * (float)per + c.base;
             if (us < best_us) {
                 best_us = us;
-                best = Shape{4, c.tm, 1, (int)per, 2};
+                best = Shape{2, c.tm, 1, (int)per, c.groups};
             }
         }
     }
@@ -142,13 +155,17 @@ hipError_t launch_fmt(const QMat &w, const uint16_t *x, float *y, int64_t m, con
     J4Q_TILE(8, 8)
 #undef J4Q_TILE
     if constexpr (FMT != Q8_0) {
-        if (t.groups == 2 && t.tm == 1) {
-            gt::gemm_tile<FMT, 4, 1, 2><<<grid, 512, 0, s>>>(w, x, y, (int)m, t.split_stages, part);
-            launched = true;
-        } else if (t.groups == 2 && t.tm == 2) {
-            gt::gemm_tile<FMT, 4, 2, 2><<<grid, 512, 0, s>>>(w, x, y, (int)m, t.split_stages, part);
-            launched = true;
-        }
+#define J4Q_GROUPS(TM, KG)                                                                                  \
+    if (t.waves == 2 && t.tm == TM && t.groups == KG) {                                                     \
+        gt::gemm_tile<FMT, 2, TM, KG><<<grid, 128 * KG, 0, s>>>(w, x, y, (int)m, t.split_stages, part);     \
+        launched = true;                                                                                    \
+    }
+        J4Q_GROUPS(1, 2)
+        J4Q_GROUPS(2, 2)
+        J4Q_GROUPS(1, 4)
+        J4Q_GROUPS(2, 4)
+        J4Q_GROUPS(3, 4)
+#undef J4Q_GROUPS
     }
     if (!launched) return hipErrorInvalidValue;
     const hipError_t e = hipGetLastError();
