@@ -91,7 +91,6 @@ public:
         *ws = Workspace();
         const bool captured = capturing(s);
         if (bytes <= kMaxOne && !captured) {
-            const RelaxedCapture relaxed;
             const Slot *t = s == engine ? engine_slot(engine, bytes) : shared_slot(s, bytes);
             if (t && (!t->done || hipStreamWaitEvent(s, t->done, 0) == hipSuccess)) {
                 ws->ptr = (float *)t->ptr;
@@ -166,6 +165,7 @@ private:
     }
     // Memory for a workspace of `bytes`, in powers of two so that growing calls grow it rarely.
     bool alloc(uint64_t bytes, Slot *t) {
+        const RelaxedCapture relaxed;
         uint64_t want = 1ull << 20;
         while (want < bytes) want *= 2;
         if (bytes_ + want > kMaxAll)  // what no call uses any more (hipFree waits for the device)
@@ -196,6 +196,7 @@ private:
         if (bytes <= engine_.bytes) return &engine_;
         Slot t;
         if (!alloc(bytes, &t)) return nullptr;
+        const RelaxedCapture relaxed;
         if (engine_.ptr) {  // its calls may still run: any stream's once they are done
             engine_.done = new_event();
             if (engine_.done && hipEventRecord(engine_.done, engine) == hipSuccess) {
@@ -213,8 +214,11 @@ private:
         Slot *best = nullptr;
         for (Slot &t : shared_)
             if (t.bytes >= bytes && t.last == s) best = &t;
-        for (Slot &t : shared_)
-            if (!best && t.bytes >= bytes && idle(t)) best = &t;
+        if (!best) {
+            const RelaxedCapture relaxed;
+            for (Slot &t : shared_)
+                if (!best && t.bytes >= bytes && idle(t)) best = &t;
+        }
         if (!best) {
             Slot t;
             t.done = new_event();
