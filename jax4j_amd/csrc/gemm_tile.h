@@ -158,7 +158,7 @@ struct Tile {
     static_assert(4 * TM % WV == 0, "whole X loads per wave");
 };
 
-// KG = 2 or 4 (WV = 2): as many groups of waves, each with buffers of its own, take a part of the range of K
+// KG = 2 or 4 (WV = 2; KG = 2 also WV = 4): as many groups of waves, each with buffers of its own, take a part of the range of K
 // each (split_stages, a multiple of 4; K a multiple of 256). Their sums meet through LDS, a quarter of
 // the rows of a 32-row tile or a half in each group, and are added in group order.
 template <int FMT, int WV, int TM, int KG = 1>
@@ -366,11 +366,13 @@ gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, 
     float *const out = part ? part + (int64_t)blockIdx.y * M * N : y;
     const int col = nw + r32;
     if constexpr (KG > 1) {
-        // elements 4 q .. 4 q + 3 of the tiles: through the X buffers, two quarters in each, which hold them exactly
-        static_assert((KG == 2 || KG == 4) && WV == 2, "quarters of the sums of all groups in the X buffers");
+        // elements 4 q .. 4 q + 3 of the tiles: through the X buffers, which hold them exactly (KG = 2: the two
+        // quarters that a group gives away)
+        static_assert((KG == 4 && WV == 2) || (KG == 2 && WV <= 4), "the groups' quarters in the X buffers");
         typedef float f32x4 __attribute__((ext_vector_type(4)));
         auto at = [&](int g, int t, int q) __attribute__((always_inline)) -> f32x4 & {
-            return reinterpret_cast<f32x4 *>(q < 2 ? xs0 : xs1)[(((g * TM + t) * 2 + (q & 1)) * WV + wave) * 64 + lane];
+            if (KG == 2) return reinterpret_cast<f32x4 *>(q % 2 ? xs1 : xs0)[((g * TM + t) * WV + wave) * 64 + lane];
+            return reinterpret_cast<f32x4 *>(q < 2 ? xs0 : xs1)[(((g * TM + t) * 2 + q % 2) * WV + wave) * 64 + lane];
         };
         auto quarter = [&](int t, int q) __attribute__((always_inline)) {
             return f32x4{acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]};

@@ -24,19 +24,20 @@ struct Cost {
 constexpr Cost kCost[] = {{4, 1, .33f, .38f, .26f}, {4, 2, .38f, .43f, .34f}, {4, 3, .45f, .50f, .43f},
                           {4, 4, .47f, .57f, .51f}, {4, 5, .58f, .68f, .63f}, {8, 4, .62f, 1.02f, 1.0f},
                           {8, 8, 1.2f, 1.75f, 1.75f}};
-// Workgroups of two or four K groups of two waves, one per CU: what the launch, the prologue and the sums
+// Workgroups of K groups of two waves (64 columns) or four, one per CU: what the launch, the prologue and the sums
 // of the groups take, and a stage of all groups, as above; Q6_K's decoding comes on top. Fitted to 162
-// sizes (N = 350 .. 15000, K = 512 .. 14336, M = 4 .. 1500). us a call of the 64-column kernel of 8 waves that
+// sizes (N = 350 .. 15000, K = 512 .. 14336, M = 4 .. 1500), times 1.09, by which the figures above are too
+// large at those sizes. us a call of the 64-column kernel of 8 waves that
 // was here before, of the shapes above, and of these: Q4_K 950 x 1040 x 2560 16.9, 17.2, 12.4; 17 x 2267 x 768
 // 5.4, 6.6, 5.3; 24 x 14336 x 4096 18.2, 15.7, 12.6; 128 x 4096 x 2048 23.0, 11.7, 8.2; Q6_K 950 x 1040 x 2560
 // 16.7, 19.2, 14.0.
 struct Group {
-    int tm, groups;
+    int waves, tm, groups;
     float base, few, all, q6_few, q6_all;
 };
-constexpr Group kGroups[] = {{1, 2, 2.73f, .326f, .393f, .054f, .074f}, {2, 2, 3.16f, .378f, .451f, .074f, .094f},
-                             {1, 4, 2.94f, .488f, .605f, .142f, .183f}, {2, 4, 3.41f, .588f, .727f, .150f, .205f},
-                             {3, 4, 3.79f, .699f, .95f, .145f, .15f}};
+constexpr Group kGroups[] = {{2, 1, 2, 2.98f, .355f, .428f, .059f, .081f}, {2, 2, 2, 3.44f, .412f, .492f, .081f, .102f},
+                             {2, 1, 4, 3.20f, .565f, .700f, .155f, .200f}, {2, 2, 4, 3.72f, .641f, .792f, .164f, .223f},
+                             {2, 3, 4, 4.13f, .762f, 1.035f, .158f, .164f}, {4, 2, 2, 3.80f, .590f, .700f, .130f, .170f}};
 constexpr int kCus = 256;  // of an MI355X; a constant, so that results do not depend on the device
 
 // The fastest shape by a model of the launch: the stages that the busiest CU runs (Q6_K's take
@@ -67,17 +68,16 @@ Shape pick(int id, const QMat &w, int64_t m, float *us_out) {
             }
         }
     }
-    // At most a tile per CU without the sum kernel: tiles of 64 columns, K in two or four groups of two waves
-    // of a workgroup (kGroups).
+    // At most a tile per CU without the sum kernel: K in groups of waves of a workgroup (kGroups).
     if (id != Q8_0 && ns % 4 == 0) {
         for (const Group &c : kGroups) {
-            const int64_t tiles = ((m + 32 * c.tm - 1) / (32 * c.tm)) * ((n + 63) / 64), per = ((ns + c.groups - 1) / c.groups + 3) / 4 * 4;
+            const int64_t tiles = ((m + 32 * c.tm - 1) / (32 * c.tm)) * ((n + 32 * c.waves - 1) / (32 * c.waves)), per = ((ns + c.groups - 1) / c.groups + 3) / 4 * 4;
             if (tiles > kCus) continue;
             const float few = c.few + (id == Q6_K ? c.q6_few : 0.f), all = c.all + (id == Q6_K ? c.q6_all : 0.f);
             const float us = (few + (all - few) * (float)tiles / kCus) * (float)per + c.base;
             if (us < best_us) {
                 best_us = us;
-                best = Shape{2, c.tm, 1, (int)per, c.groups};
+                best = Shape{c.waves, c.tm, 1, (int)per, c.groups};
             }
         }
     }
@@ -155,16 +155,17 @@ hipError_t launch_fmt(const QMat &w, const uint16_t *x, float *y, int64_t m, con
     J4Q_TILE(8, 8)
 #undef J4Q_TILE
     if constexpr (FMT != Q8_0) {
-#define J4Q_GROUPS(TM, KG)                                                                                  \
-    if (t.waves == 2 && t.tm == TM && t.groups == KG) {                                                     \
-        gt::gemm_tile<FMT, 2, TM, KG><<<grid, 128 * KG, 0, s>>>(w, x, y, (int)m, t.split_stages, part);     \
+#define J4Q_GROUPS(WV, TM, KG)                                                                              \
+    if (t.waves == WV && t.tm == TM && t.groups == KG) {                                                    \
+        gt::gemm_tile<FMT, WV, TM, KG><<<grid, 64 * WV * KG, 0, s>>>(w, x, y, (int)m, t.split_stages, part); \
         launched = true;                                                                                    \
     }
-        J4Q_GROUPS(1, 2)
-        J4Q_GROUPS(2, 2)
-        J4Q_GROUPS(1, 4)
-        J4Q_GROUPS(2, 4)
-        J4Q_GROUPS(3, 4)
+        J4Q_GROUPS(2, 1, 2)
+        J4Q_GROUPS(2, 2, 2)
+        J4Q_GROUPS(2, 1, 4)
+        J4Q_GROUPS(2, 2, 4)
+        J4Q_GROUPS(2, 3, 4)
+        J4Q_GROUPS(4, 2, 2)
 #undef J4Q_GROUPS
     }
     if (!launched) return hipErrorInvalidValue;
