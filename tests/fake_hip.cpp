@@ -83,6 +83,14 @@ F const char *fake_log() {  // and clears it
     return out.c_str();
 }
 
+F const char *fake_kernels() {  // the names of the kernels in the library
+    LOCK;
+    static std::string names;
+    names.clear();
+    for (auto &k : kernels) names += k.second + '\n';
+    return names.c_str();
+}
+
 // ---- the runtime
 F hipError_t hipMalloc(void **p, size_t n) {
     LOCK;

@@ -16,7 +16,7 @@ _PRELUDE = """
 import ctypes as C, json, sys
 import numpy as np
 fake = C.CDLL({shim!r}, mode=C.RTLD_GLOBAL)
-fake.fake_log.restype = C.c_char_p
+fake.fake_log.restype = fake.fake_kernels.restype = C.c_char_p
 fake.fake_used.restype = C.c_uint64
 fake.fake_capacity.argtypes = [C.c_uint64]
 fake.fake_capture.argtypes = [C.c_void_p, C.c_int]

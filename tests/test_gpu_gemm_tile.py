@@ -25,18 +25,24 @@ def bits(a):
     return np.ascontiguousarray(a, dtype=np.float32).view(np.uint32)
 
 
-# One size or more for every tile that the launch model picks, with rows and columns past the last
-# tile, one superblock up to many, and K splits of unequal length: 32 rows (5, 24: 8 splits, 70: 5
-# splits), 64 (97), 96 (90: 4 to 6 splits; 160), 128 (777, 1024), 160 (300, 2049: 14337 columns), 128
-# x 256 (512), 256 x 256 (2048), K in two wave groups of a workgroup (950: 64 rows; 500, with unequal
-# halves, and 700: 32). Q8_0 also with an odd number of 64-element stages (K = 192).
+# Rows and columns past the last tile, one superblock up to many, K splits of unequal length. Q8_0 also
+# with an odd number of 64-element stages (K = 192).
 SHAPES = [(5, 37, 512), (24, 4096, 4096), (70, 130, 1280), (97, 10007, 256), (90, 5001, 3072), (160, 14336, 512),
           (777, 4097, 768), (1024, 4096, 256), (300, 14336, 256), (2049, 14337, 256), (512, 14336, 512), (2048, 14336, 256),
           (950, 1040, 2560), (500, 1041, 1280), (700, 700, 1024)]
 
 
+# Every tile at a depth where its loop comes round several times, over an odd number of superblocks (so that
+# Q6_K's d changes its half of a dword within a row): (row tiles of 32, waves, K groups) (1, 4, 1), (2, 4, 1),
+# (3, 4, 1), (4, 4, 1), (5, 4, 1), (4, 8, 1), (8, 8, 1); for the types with K groups (1, 2, 2), (2, 2, 2),
+# (1, 2, 4), (2, 2, 4), (3, 2, 4), (2, 4, 2); and K splits. test_gemm_tile_choice.py checks that they are picked.
+DEEP = [(130, 6001, 1280), (350, 4097, 1280), (500, 4097, 1280), (500, 6001, 1280), (2049, 2049, 1280), (1025, 6001, 1280), (2049, 6001, 1280),
+        (33, 129, 1280), (500, 1041, 1280), (200, 2049, 1792), (300, 2047, 3840), (600, 2001, 2304), (523, 3459, 1792),
+        (30, 1205, 3840), (140, 1205, 4352), (257, 2049, 4352)]
+
+
 @pytest.mark.parametrize("qt", ALL, ids=lambda q: q.name)
-@pytest.mark.parametrize("m,n,k", SHAPES + [(12, 20000, 192), (2048, 2049, 64)])
+@pytest.mark.parametrize("m,n,k", SHAPES + [(12, 20000, 192), (2048, 2049, 64)] + DEEP)
 def test_gemm_tiles_match_oracle(backend, qt, m, n, k):
     if k % 256 and qt is not QuantType.Q8_0:
         pytest.skip("K of a whole number of superblocks")
