@@ -213,7 +213,8 @@ int j4q_quant_matvec_into(j4q_buffer weights, const float *x_dev, const float *a
  * [m, cols] and xs_dev fp32 [m, cols/32] as workspace; the bf16 variant ignores them. On
  * Q4_0, Q4_K and Q6_K weights the bf16 variant splits K over workgroups where the tiles alone
  * would leave CUs idle, and keeps the partial products (at most 32 MiB) in a workspace as
- * j4q_quant_matvec_into does; nothing else is allocated. */
+ * j4q_quant_matvec_into does; nothing else is allocated. Under stream capture it takes none and
+ * does not split K, so the fp32 sums may be rounded otherwise than in an eager call. */
 int j4q_quant_matmul_into(j4q_buffer weights, const uint16_t *x_dev, int64_t m, int variant, int8_t *xq_dev,
                           float *xs_dev, float *y_dev, void *stream);
 /* The int8 variant on activations already quantized (engine-local; no counterpart in the
@@ -227,7 +228,7 @@ int j4q_quant_matmul_q8_into(j4q_buffer weights, const int8_t *xq_dev, const flo
 
 /* The prefill GEMM for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). No counterpart in the
- * reference. Same result as j4q_quant_matmul_into (bit for bit), but the int8 variant's
+ * reference. Same result as an eager j4q_quant_matmul_into (bit for bit), but the int8 variant's
  * workspace (the quantized activations and their block scales) lives in one fixed engine
  * array of 36 MiB per GPU, so the call allocates nothing: x_dev bf16 [m, cols], y_dev fp32
  * [m, rows], both 16-byte aligned. The int8 variant needs m * cols <= 33554432 (32 MiB of

@@ -843,7 +843,7 @@ int j4q_quant_matmul(j4q_buffer wh, j4q_buffer xh, int variant, j4q_buffer *out)
     if ((rc = alloc_buf(J4Q_KIND_F32, 2, M, N, (uint64_t)(M * N) * 4, out, &ydev, {x}))) return rc;
     if (variant == J4Q_GEMM_BF16) {
         j4q::Workspace ws;
-        const uint64_t wsb = j4q::gemm_bf16_workspace_bytes(qt, m, M);
+        const uint64_t wsb = capturing(g_stream) ? 0 : j4q::gemm_bf16_workspace_bytes(qt, m, M);
         if (wsb) LAUNCH_INTO("quantMatmul workspace", out, g_workspaces.begin(g_stream, g_stream, wsb, &ws));
         const hipError_t e = j4q::launch_gemm_bf16(qt, m, xdev, (float *)ydev, M, ws, g_stream);
         g_workspaces.end(g_stream, ws, e == hipSuccess);
@@ -904,7 +904,8 @@ int j4q_quant_matmul_into(j4q_buffer wh, const uint16_t *x, int64_t m, int varia
     const j4q::QMat mm = qmat_of(*w);
     if (variant == J4Q_GEMM_BF16) {
         j4q::Workspace ws;
-        const uint64_t wsb = j4q::gemm_bf16_workspace_bytes(w->qtype, mm, m);
+        // under capture K is not split: the workspace would be memory nodes (see run_gemv)
+        const uint64_t wsb = capturing(s) ? 0 : j4q::gemm_bf16_workspace_bytes(w->qtype, mm, m);
         if (wsb) HIP_TRY("quantMatmul_into workspace", g_workspaces.begin(s, g_stream, wsb, &ws));
         const hipError_t e = j4q::launch_gemm_bf16(w->qtype, mm, x, y, m, ws, s);
         g_workspaces.end(s, ws, e == hipSuccess);

@@ -46,7 +46,7 @@ constexpr int kCus = 256;  // of an MI355X; a constant, so that results do not d
 // at 5.5 MB/us. Over the sweeps (38 sizes) its choice takes 1.2 % longer than the best of all
 // shapes on average, 11 % at worst (with the groups of kGroups, 162 sizes: 0.5 %). Splits are whole multiples of four stages, and their workspace
 // is at most 32 MiB; a Q8_0 call takes no workspace, so it does not split.
-Shape pick(int id, const QMat &w, int64_t m, float *us_out) {
+Shape pick(int id, const QMat &w, int64_t m, bool split, float *us_out) {
     const int64_t n = w.rows, ns = w.cols / 64;
     const float alone_add = id == Q6_K ? .12f : id == Q8_0 ? .05f : 0.f, shared_add = id == Q6_K ? .09f : id == Q8_0 ? .05f : 0.f;
     Shape best;
@@ -54,7 +54,7 @@ Shape pick(int id, const QMat &w, int64_t m, float *us_out) {
     for (const Cost &c : kCost) {
         const int64_t tiles = ((m + 32 * c.tm - 1) / (32 * c.tm)) * ((n + 32 * c.waves - 1) / (32 * c.waves));
         int64_t last = 0;
-        for (int64_t want = 1; want <= (id == Q8_0 ? 1 : 16); want++) {
+        for (int64_t want = 1; want <= (split && id != Q8_0 ? 16 : 1); want++) {
             const int64_t per = want == 1 ? ns : ((ns + want - 1) / want + 3) / 4 * 4, s = (ns + per - 1) / per;
             if (s == last || (s > 1 && s * m * n * 4 > (32ll << 20))) continue;
             last = s;
@@ -104,11 +104,11 @@ float q8_wide_us(const QMat &w, int64_t m) {
     return 1e30f;
 }
 
-// Whether the tile kernel takes the call; the shape it runs with.
-Shape shape_of(int id, const QMat &w, int64_t m) {
+// Whether the tile kernel takes the call; the shape it runs with. split: K may be split over workgroups.
+Shape shape_of(int id, const QMat &w, int64_t m, bool split) {
     float us = 0.f;
     if (id == Q8_0 && w.cols % 64 != 0) return Shape{};
-    const Shape t = pick(id, w, m, &us);
+    const Shape t = pick(id, w, m, split, &us);
     return id == Q8_0 && q8_wide_us(w, m) <= 1.05f * us ? Shape{} : t;
 }
 
@@ -137,7 +137,7 @@ sum_splits_kernel(const float *__restrict__ part, int splits, int64_t n, float *
 template <int FMT>
 hipError_t launch_fmt(const QMat &w, const uint16_t *x, float *y, int64_t m, const Shape &t, const Workspace &ws, hipStream_t s) {
     const int64_t tiles = ((m + 32 * t.tm - 1) / (32 * t.tm)) * ((w.rows + 32 * t.waves - 1) / (32 * t.waves));
-    if (tiles > 0x7fffffff || (t.splits > 1 && !ws.ptr)) return hipErrorInvalidValue;
+    if (tiles > 0x7fffffff || (t.splits > 1 && ws.bytes < (uint64_t)t.splits * (uint64_t)m * (uint64_t)w.rows * 4u)) return hipErrorInvalidValue;
     const dim3 grid((unsigned)tiles, (unsigned)t.splits);
     float *const part = t.splits > 1 ? ws.ptr : nullptr;
     bool launched = false;
@@ -190,13 +190,13 @@ bool gemm_bf16_supported(int id, int64_t cols) {
 
 uint64_t gemm_bf16_workspace_bytes(int id, const QMat &w, int64_t m) {
     if (!gemm_bf16_supported(id, w.cols) || m <= 0 || w.rows <= 0) return 0;
-    const Shape t = shape_of(id, w, m);
+    const Shape t = shape_of(id, w, m, true);
     return t.splits > 1 ? (uint64_t)t.splits * (uint64_t)m * (uint64_t)w.rows * 4u : 0;
 }
 
 hipError_t launch_gemm_bf16(int id, const QMat &w, const uint16_t *x, float *y, int64_t m, const Workspace &ws, hipStream_t s) {
     if (m <= 0 || w.rows <= 0) return hipSuccess;
-    const Shape t = shape_of(id, w, m);
+    const Shape t = shape_of(id, w, m, ws.ptr != nullptr);
     if (id == Q8_0 && !t.tm) return launch_gemm_q8_bf16(w, x, y, m, s);
     if (!gemm_bf16_supported(id, w.cols) || (uint64_t)m * (uint64_t)w.cols * 2u > 0x7fffffffull ||
         (uint64_t)w.rows * (uint64_t)w.cols / (id == Q8_0 ? 1u : 2u) > 0x7fffffffull)

@@ -178,7 +178,8 @@ hipError_t launch_gemm_q8_int8(const QMat &w, const int8_t *xq, const float *xs,
 hipError_t launch_gemm_q8_bf16(const QMat &w, const uint16_t *x, float *y, int64_t m, hipStream_t s);
 // Prefill GEMM, bf16 variant, over Q8_0, Q4_0 (cols % 128 == 0), Q4_K and Q6_K weights.
 bool gemm_bf16_supported(int id, int64_t cols);
-// Workspace the call needs (bytes, at most 32 MiB; 0: none): the partial products of its K splits.
+// Workspace the call needs (bytes, at most 32 MiB; 0: none): the partial products of its K splits. Without
+// one (ws.ptr null) launch_gemm_bf16 does not split K.
 uint64_t gemm_bf16_workspace_bytes(int id, const QMat &w, int64_t m);
 hipError_t launch_gemm_bf16(int id, const QMat &w, const uint16_t *x, float *y, int64_t m, const Workspace &ws, hipStream_t s);
 hipError_t launch_synth_quant(int id, uint64_t seed, int64_t rows, int64_t cols, uint8_t *gguf,

@@ -13,7 +13,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from jax4j_amd import QuantType
+from jax4j_amd import DType, QuantType
 from jax4j_amd import _native as N
 from jax4j_amd import synthetic as S
 
@@ -146,6 +146,39 @@ def test_workspace_call_under_capture_replays(backend, b, r, k):
         if b == 16:
             assert np.array_equal(backend.download(z).view(np.uint32), ref)
     hip.ok("hipGraphExecDestroy", run)
+    hip.ok("hipGraphDestroy", graph)
+    for h in (w, x, y, z, nan):
+        backend.release(h)
+    hip.close()
+
+
+def test_captured_matmul_replays(backend):
+    """A GEMM that splits K over a workspace when called does not under capture: the same products in another
+    order of their fp32 sums, on every replay."""
+    m, n, k = 24, 512, 8192
+    hip = Hip()
+    w = upload(backend, QuantType.Q6_K, n, k, 51)
+    x = backend.upload(S.activations_bf16(9, m * k).reshape(m, k), shape=(m, k), dtype=DType.BF16)
+    y, z, nan = (backend.upload(np.full((m, n), np.nan, np.float32)) for _ in range(3))
+    px, py, pz, pnan = (backend.buffer_desc(h).device_ptr for h in (x, y, z, nan))
+    graph, runs = C.c_void_p(), [C.c_void_p(), C.c_void_p()]
+    hip.ok("hipStreamBeginCapture", hip.stream, 2)  # relaxed
+    backend.quant_matmul_into(w, px, m, "bf16", 0, 0, py, hip.stream.value)
+    hip.ok("hipStreamEndCapture", hip.stream, C.byref(graph))
+    for run in runs:  # a graph without memory nodes may be instantiated more than once
+        hip.ok("hipGraphInstantiate", C.byref(run), graph, None, None, C.c_size_t(0))
+    first = None
+    for i in range(4):
+        assert N.load().j4q_copy(py, pnan, 4 * m * n, hip.stream) == 0
+        hip.ok("hipGraphLaunch", runs[i % 2], hip.stream)
+        backend.quant_matmul_into(w, px, m, "bf16", 0, 0, pz)
+        hip.wait()
+        got, eager = backend.download(y), backend.download(z)
+        first = got if first is None else first
+        assert np.array_equal(got.view(np.uint32), first.view(np.uint32))
+        assert np.abs(got - eager).max() <= 4e-5 * np.abs(eager).max()  # each within 2e-5 of the exact sums
+    for run in runs:
+        hip.ok("hipGraphExecDestroy", run)
     hip.ok("hipGraphDestroy", graph)
     for h in (w, x, y, z, nan):
         backend.release(h)

@@ -208,3 +208,19 @@ def test_decode_plans_are_made_with_the_memory_of_16_row_launches(shim, batch):
     """)
     assert small > full
     assert jobs[1] == 0 and (jobs[0] > 0) == (batch <= 16)
+
+
+@pytest.mark.parametrize("m,rows,cols", [(24, 512, 14336), (16, 1024, 4096), (508, 1474, 14080)])
+def test_captured_matmuls_take_no_memory_nodes(shim, m, rows, cols):
+    eager, captured = fakehip.run(shim, f"""
+        w = zeros(QuantType.Q4_K, {rows}, {cols})
+        call = lambda: lib.j4q_quant_matmul_into(w.handle, 4096, {m}, 1, None, None, 4096, 0x77770)
+        log()
+        assert call() == 0
+        eager = log("malloc", "malloc_async", "launch")
+        fake.fake_capture(0x77770, 1)
+        assert call() == 0
+        result = eager, log("malloc", "malloc_async", "launch")
+    """)
+    assert len(eager) == 3 and "sum_splits" in eager[-1]
+    assert len(captured) == 1 and "gemm_tile" in captured[0]
