@@ -427,59 +427,63 @@ hipError_t launch_gemm_q8_int8(const QMat &w, const int8_t *xq, const float *xs,
     return launch_gemm<kVarInt8, 128, 128, 4, 3>(w, xq, xs, y, m, s);
 }
 
-// The calls that gemm_tile.hip leaves to these kernels: K % 64 != 0, and the small grids on which
-// they are faster (q8_wide_us there models their times by the rules below).
+// Q8_0 weights, bf16 variant, on the kernels of gemm_wide.h and the 4-wave one: which, and about how many us
+// it takes (a workgroup's stage times the stages of the busiest CU, measured at N = K = 4096, and 3 us
+// for the launch). gemm_tile.hip runs the faster one of its own tiles and this. With K % 64 == 0 that
+// leaves these kernels the grids that do not fill the GPU; the ones priced at kSlower then always lose
+// to a tile (M = 2048 at 128 x 128: 84-90 us against 71-72; M = 200, N = 700, K = 1024 on the 4-wave kernel: 12.0
+// against 8.0) and serve K % 64 == 32 alone, which the tiles do not take. The counts are compared with a
+// constant number of CUs, so that results do not depend on the device.
+Q8Choice choose_q8_bf16(const QMat &w, int64_t m) {
+    constexpr float kSlower = 1e30f;
+    const int64_t n = w.rows, k = w.cols, cus = 256;
+    auto tiles = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
+    auto choice = [&](Q8Kernel kernel, int64_t t, int64_t stage, float per) {
+        return Q8Choice{kernel, t, per == kSlower ? kSlower : (float)((t + cus - 1) / cus * ((k + stage - 1) / stage)) * per + 3.0f};
+    };
+    if (m > 64 && n % 2 == 0) {
+        // tiles loaded straight into LDS, the largest whose grid still fills the GPU (N = K = 4096: M = 512 in
+        // 29-30 us at 128 x 64; M = 128..256 in 18.5-19.9 us at 64 x 64, against 20.8-36.4 us on the kernels
+        // below; with fewer than 128 workgroups those are faster: M = 64, or N = 1024 at M = 128)
+        if (tiles(128, 128) >= 256) return choice(Q8Kernel::kLds128x128, tiles(128, 128), 128, kSlower);
+        if (tiles(128, 64) >= 192) return choice(Q8Kernel::kLds128x64, tiles(128, 64), 128, .75f);
+        if (tiles(64, 64) >= 128) return choice(Q8Kernel::kLds64x64, tiles(64, 64), 128, tiles(64, 64) > cus ? .40f : .46f);
+    }
+    if (m >= 512) {
+        // register-staged (odd N, or too few tiles for the kernel above): 128 x 128 tiles when they fill the
+        // GPU, else 128 x 64
+        if (tiles(128, 128) >= 256) return choice(Q8Kernel::kWide128x128, tiles(128, 128), 64, kSlower);
+        return choice(Q8Kernel::kWide128x64, tiles(128, 64), 64, .53f);
+    }
+    // small M: 16 weight rows per workgroup, all of K (N = K = 4096: M = 32 in 11.7 us, M = 128 in 23.0 us with
+    // 64-row tiles, M = 192 in 31.6 us against 34.1 on the 4-wave kernel; 128-row tiles are no faster at M = 128)
+    if (m <= 32) return choice(Q8Kernel::kNarrow32, tiles(32, 16), 512, .85f);
+    if (m <= 192) return choice(Q8Kernel::kNarrow64, tiles(64, 16), 256, .62f);
+    return choice(Q8Kernel::kFourWaves, 1, 1, kSlower);
+}
+
 hipError_t launch_gemm_q8_bf16(const QMat &w, const uint16_t *x, float *y, int64_t m, hipStream_t s) {
     if (m <= 0 || w.rows <= 0) return hipSuccess;
-    if (m > 65535 * 64 || w.cols % 32 != 0 || (uint64_t)m * w.cols * 2 > 0x7fffffffull) return hipErrorInvalidValue;
-    if (m > 64 && w.rows % 2 == 0 && (uint64_t)w.rows * w.cols <= 0x7fffffffull) {
-        // gemm_wide.h, tiles loaded straight into LDS: the largest tile whose grid still
-        // fills the GPU (measured on MI355X, K = 4096: M = 512, N = 4096 in 29-30 us at
-        // 128 x 64; M = 2048 in 90 us at 128 x 128; M = 128..256, N = 4096 in 18.5-19.9 us at
-        // 64 x 64, against 20.8-36.4 us on the small-M and 4-wave kernels; with fewer than 128
-        // workgroups those kernels are faster: M = 64, or N = 1024 at M = 128)
-        const int64_t nt64 = (w.rows + 63) / 64, nt128 = (w.rows + 127) / 128;
-        const int64_t g128x128 = ((m + 127) / 128) * nt128, g128 = ((m + 127) / 128) * nt64, g64 = ((m + 63) / 64) * nt64;
-        if (g64 > 0x7fffffff) return hipErrorInvalidValue;
-        if (g128x128 >= 256) {
-            gw::gemm_bf16_lds<128, 2, true><<<(unsigned)g128x128, 512, 0, s>>>(w, x, y, (int)m);
-            return hipGetLastError();
-        }
-        if (g128 >= 192) {
-            // the next stage's loads spread between the MFMAs here too, since the waves' priority
-            // follows their place in the stage (A/B on one box, three rounds: M = 512 31.6-32.1 ->
-            // 30.2-30.9 us; without the priority the spread did not pay at this tile)
-            gw::gemm_bf16_lds<128, 1, true><<<(unsigned)g128, 512, 0, s>>>(w, x, y, (int)m);
-            return hipGetLastError();
-        }
-        if (g64 >= 128) {
-            gw::gemm_bf16_lds<64, 1, false><<<(unsigned)g64, 512, 0, s>>>(w, x, y, (int)m);
-            return hipGetLastError();
-        }
+    if (m > 65535 * 64 || w.cols % 32 != 0 || (uint64_t)m * w.cols * 2 > 0x7fffffffull ||
+        (uint64_t)w.rows * w.cols > 0x7fffffffull)
+        return hipErrorInvalidValue;
+    const Q8Choice c = choose_q8_bf16(w, m);
+    if (c.grid > 0x7fffffff) return hipErrorInvalidValue;
+    const unsigned g = (unsigned)c.grid;
+    switch (c.kernel) {
+    case Q8Kernel::kLds128x128: gw::gemm_bf16_lds<128, 2, true><<<g, 512, 0, s>>>(w, x, y, (int)m); break;
+    // the next stage's loads spread between the MFMAs here too, since the waves' priority follows their
+    // place in the stage (A/B on one box, three rounds: M = 512 31.6-32.1 -> 30.2-30.9 us; without the
+    // priority the spread did not pay at this tile)
+    case Q8Kernel::kLds128x64: gw::gemm_bf16_lds<128, 1, true><<<g, 512, 0, s>>>(w, x, y, (int)m); break;
+    case Q8Kernel::kLds64x64: gw::gemm_bf16_lds<64, 1, false><<<g, 512, 0, s>>>(w, x, y, (int)m); break;
+    case Q8Kernel::kWide128x128: gw::gemm_bf16_wide<128, 2, 4><<<g, 512, 0, s>>>(w, x, y, (int)m); break;
+    case Q8Kernel::kWide128x64: gw::gemm_bf16_wide<128, 1, 4><<<g, 512, 0, s>>>(w, x, y, (int)m); break;
+    case Q8Kernel::kNarrow32: gw::gemm_bf16_narrow<32, 2, 2><<<g, 512, 0, s>>>(w, x, y, (int)m); break;
+    case Q8Kernel::kNarrow64: gw::gemm_bf16_narrow<64, 1, 2><<<g, 512, 0, s>>>(w, x, y, (int)m); break;
+    case Q8Kernel::kFourWaves: return launch_gemm<kVarBf16, 128, 64, 4, 3, 2>(w, x, nullptr, y, m, s);
     }
-    if (m >= 512 && (uint64_t)w.rows * w.cols <= 0x7fffffffull) {
-        // gemm_wide.h, register-staged (odd N, or too few tiles for the kernel above): 128 x 128
-        // tiles when they fill the GPU, else 128 x 64
-        const int64_t mt = (m + 127) / 128, t128 = mt * ((w.rows + 127) / 128), t64 = mt * ((w.rows + 63) / 64);
-        if (t64 > 0x7fffffff) return hipErrorInvalidValue;
-        if (t128 >= 256) gw::gemm_bf16_wide<128, 2, 4><<<(unsigned)t128, 512, 0, s>>>(w, x, y, (int)m);
-        else gw::gemm_bf16_wide<128, 1, 4><<<(unsigned)t64, 512, 0, s>>>(w, x, y, (int)m);
-        return hipGetLastError();
-    }
-    if (m <= 192 && (uint64_t)w.rows * w.cols <= 0x7fffffffull) {
-        // gemm_wide.h, small M: 16 weight rows per workgroup, all of K (measured on MI355X,
-        // N = K = 4096: M = 32 in 11.7 us, M = 128 in 23.0 us with 64-row tiles, M = 192 in
-        // 31.6 us against 34.1 on the 4-wave kernel; 128-row tiles are no faster at M = 128)
-        const int64_t nt = (w.rows + 15) / 16, bm = m <= 32 ? 32 : 64;
-        const int64_t grid = ((m + bm - 1) / bm) * nt;
-        if (grid > 0x7fffffff) return hipErrorInvalidValue;
-        if (bm == 32) gw::gemm_bf16_narrow<32, 2, 2><<<(unsigned)grid, 512, 0, s>>>(w, x, y, (int)m);
-        else gw::gemm_bf16_narrow<64, 1, 2><<<(unsigned)grid, 512, 0, s>>>(w, x, y, (int)m);
-        return hipGetLastError();
-    }
-    if (m <= 64) return launch_gemm<kVarBf16, 64, 64, 4, 3, 2>(w, x, nullptr, y, m, s);
-    if (m <= 512) return launch_gemm<kVarBf16, 128, 64, 4, 3, 2>(w, x, nullptr, y, m, s);
-    return launch_gemm<kVarBf16, 128, 128, 2, 3, 1>(w, x, nullptr, y, m, s);
+    return hipGetLastError();
 }
 
 }  // namespace j4q

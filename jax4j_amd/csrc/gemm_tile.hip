@@ -85,31 +85,12 @@ Shape pick(int id, const QMat &w, int64_t m, bool split, float *us_out) {
     return best;
 }
 
-// The same model of the Q8_0 kernels of gemm_wide.h (launch_gemm_q8_bf16 picks among them by these
-// rules): us per stage of one workgroup, measured at N = K = 4096. Where none of them applies,
-// the 4-wave kernel would run, which is slower at every size tried (M = 200, N = 700, K = 1024:
-// 12.0 us against 8.0).
-float q8_wide_us(const QMat &w, int64_t m) {
-    const int64_t n = w.rows, k = w.cols;
-    auto tiles = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
-    auto us = [&](int64_t t, int64_t stage, float per) { return (float)((t + kCus - 1) / kCus * ((k + stage - 1) / stage)) * per + 3.0f; };
-    if (m > 64 && n % 2 == 0) {
-        if (tiles(128, 128) >= 256) return 1e30f;  // M = 2048: 84-90 us against 71-72
-        if (tiles(128, 64) >= 192) return us(tiles(128, 64), 128, .75f);
-        if (tiles(64, 64) >= 128) return us(tiles(64, 64), 128, tiles(64, 64) > kCus ? .40f : .46f);
-    }
-    if (m >= 512) return us(tiles(128, 64), 64, .53f);
-    if (m <= 32) return us(tiles(32, 16), 512, .85f);
-    if (m <= 192) return us(tiles(64, 16), 256, .62f);
-    return 1e30f;
-}
-
 // Whether the tile kernel takes the call; the shape it runs with. split: K may be split over workgroups.
 Shape shape_of(int id, const QMat &w, int64_t m, bool split) {
     float us = 0.f;
     if (id == Q8_0 && w.cols % 64 != 0) return Shape{};
     const Shape t = pick(id, w, m, split, &us);
-    return id == Q8_0 && q8_wide_us(w, m) <= 1.05f * us ? Shape{} : t;
+    return id == Q8_0 && choose_q8_bf16(w, m).us <= 1.05f * us ? Shape{} : t;
 }
 
 // y[i] = ((part[0][i] + part[1][i]) + ...) for i < n: the K splits' partial products added

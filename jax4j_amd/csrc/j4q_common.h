@@ -175,6 +175,14 @@ hipError_t launch_quantize_act(const uint16_t *x, int64_t m, int64_t k, int8_t *
                                hipStream_t s);
 hipError_t launch_gemm_q8_int8(const QMat &w, const int8_t *xq, const float *xs, float *y, int64_t m,
                                hipStream_t s);
+// The kernel that launch_gemm_q8_bf16 runs for this size, its grid, and about how many us it takes.
+enum class Q8Kernel { kLds128x128, kLds128x64, kLds64x64, kWide128x128, kWide128x64, kNarrow32, kNarrow64, kFourWaves };
+struct Q8Choice {
+    Q8Kernel kernel;
+    int64_t grid;
+    float us;
+};
+Q8Choice choose_q8_bf16(const QMat &w, int64_t m);
 hipError_t launch_gemm_q8_bf16(const QMat &w, const uint16_t *x, float *y, int64_t m, hipStream_t s);
 // Prefill GEMM, bf16 variant, over Q8_0, Q4_0 (cols % 128 == 0), Q4_K and Q6_K weights.
 bool gemm_bf16_supported(int id, int64_t cols);
