@@ -16,6 +16,7 @@ from __future__ import annotations
 import ctypes as C
 import os
 import threading
+from operator import index
 
 import numpy as np
 
@@ -44,6 +45,12 @@ def check(rc: int, op: str) -> None:
         return
     msg = N.last_error() or f"{op} failed (code {rc})"
     raise _ERRORS.get(rc, RuntimeError)(msg)
+
+
+def _address(p) -> int | None:
+    """A device address as the library takes it; 0 and None are NULL. Integers only: the library's pointer
+    arguments would take bytes, strings and arrays by their host address."""
+    return index(p) or None if p is not None else None
 
 
 def _as_u8(blocks) -> np.ndarray:
@@ -269,7 +276,7 @@ class Mi355xBackend:
         workspace, which the engine keeps for later calls on any stream."""
         check(
             self._lib().j4q_quant_matvec_into(
-                weights.handle, x_ptr, add_ptr or None, y_ptr, batch, stream or None
+                weights.handle, _address(x_ptr), _address(add_ptr), _address(y_ptr), batch, _address(stream)
             ),
             "quantMatvec_into",
         )
@@ -278,7 +285,7 @@ class Mi355xBackend:
         v = {"int8": N.GEMM_INT8, "bf16": N.GEMM_BF16}[variant]
         check(
             self._lib().j4q_quant_matmul_into(
-                weights.handle, x_ptr, m, v, xq_ptr or None, xs_ptr or None, y_ptr, stream or None
+                weights.handle, _address(x_ptr), m, v, _address(xq_ptr), _address(xs_ptr), _address(y_ptr), _address(stream)
             ),
             "quantMatmul_into",
         )
@@ -327,7 +334,7 @@ class DecodePlan:
 
     def run(self, stream: int = 0) -> None:
         """Enqueue one step on ``stream`` (0 = the engine stream); no synchronisation."""
-        check(self._be._lib().j4q_decode_plan_run(self.handle, stream or None), "decode plan run")
+        check(self._be._lib().j4q_decode_plan_run(self.handle, _address(stream)), "decode plan run")
 
     def info(self) -> dict:
         d = N.DecodePlanDesc()

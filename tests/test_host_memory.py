@@ -224,3 +224,25 @@ def test_captured_matmuls_take_no_memory_nodes(shim, m, rows, cols):
     """)
     assert len(eager) == 3 and "sum_splits" in eager[-1]
     assert len(captured) == 1 and "gemm_tile" in captured[0]
+
+
+def test_addresses_are_integers(shim):
+    """Host objects whose address ctypes would pass on are refused, as pointers to GPU memory."""
+    refused, launched = fakehip.run(shim, """
+        w = zeros(QuantType.Q8_0, 64, 512)
+        x, y = address(4 * 512), address(4 * 64)
+        refused = 0
+        log()
+        for bad in (b"x" * 2048, "x", (C.c_float * 512)(), np.zeros(512, np.float32), 1.0):
+            for call in (lambda: be.quant_matvec_into(w, bad, 0, y), lambda: be.quant_matvec_into(w, x, bad, y),
+                         lambda: be.quant_matvec_into(w, x, 0, y, 1, bad),
+                         lambda: be.quant_matmul_into(w, bad, 1, "bf16", 0, 0, y), lambda: be.quant_matmul_into(w, x, 1, "bf16", bad, 0, y)):
+                try:
+                    call()
+                except TypeError:
+                    refused += 1
+        n = len(launches())
+        be.quant_matvec_into(w, np.int64(x), 0, np.uint64(y))
+        result = refused, n
+    """)
+    assert refused == 25 and launched == 0
