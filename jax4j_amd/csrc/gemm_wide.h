@@ -960,7 +960,7 @@ namespace gw {
 //    with half the barriers ran 39.7 us at M = 512).
 // Requires K % 32 == 0, N % 8 == 0, M * K < 2^31 and N * K < 2^31. Internal linkage: this header
 // is included by more than one source.
-// 1.5 * 2^23, whose bits plus I (|I| < 2^22; a block's |I| <= 32 * 127^2) are the float 1.5 * 2^23 + I: the
+// 1.5 * 2^23, whose bits plus I (|I| < 2^22; a block's |I| <= 32 * 128^2, codes of -128 included) are the float 1.5 * 2^23 + I: the
 // products start from its bits, and a subtraction instead of the slower conversion gives (float)I
 // exactly (N = K = 4096: M = 300 29.5 -> 28.5 us, M = 2048 117 -> 114.5). The kernel is bound by its
 // fold: MFMA and vector instructions of two waves hardly overlap on a SIMD (16 us of the two at
