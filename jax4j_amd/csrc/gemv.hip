@@ -300,6 +300,7 @@ hipError_t launch_valu(int id, const QMat &m, const float *x, const float *add, 
 // scales and block sums, the K splits' partial sums.
 struct TileShape {
     int rows = 0, tm = 1, splits = 1, split_stages = 0;
+    bool all = false;  // a workgroup runs every split
     int64_t x_bytes = 0, scale_bytes = 0, sum_bytes = 0, bytes = 0;
 };
 
@@ -323,35 +324,60 @@ bool tile_supported(int id, const QMat &m) {
     return unit && m.cols % unit == 0 && m.rows <= (id == Q8_0 ? 0x7fffffff : 0xffffffff) / m.cols;
 }
 
+// About how many us a launch of the tile kernel takes: `groups` workgroups of tm tiles of 32 rows, with so
+// many 64-column stages each. us a stage of a workgroup alone on its CU, and of each one of several, by
+// type (fmt_slot) and tm: fitted to 89 sizes (N = 3000 .. 128256, K = 768 .. 14336, 19 to 300 rows, split over
+// workgroups and not), 9 % off on average.
+float tile_us(int id, int tm, int64_t groups, int64_t stages) {
+    constexpr float kStage[4][2][2] = {{{.438f, .328f}, {.667f, .524f}}, {{.485f, .386f}, {.726f, .606f}},
+                                       {{.543f, .372f}, {.905f, .609f}}, {{.565f, .479f}, {.846f, .714f}}};
+    const float *const c = kStage[fmt_slot(id)][tm - 1];
+    const float per_cu = (float)groups / (float)g_cus, n = per_cu > 2.f ? per_cu + .3f : per_cu > 1.f ? 2.f : 1.f;
+    return (c[1] * n > c[0] ? c[1] * n : c[0]) * (float)stages + (tm == 1 ? 8.f : 9.5f);
+}
+
 TileShape tile_shape(int id, const QMat &m, int64_t batch) {
     TileShape t;
     if (batch < tile_min_rows(id, m.cols) || !tile_supported(id, m)) return t;
     const int64_t K = m.cols, N = m.rows, stages = K / 64;
     // K splits of a quarter of the columns, within 512 .. 1024 (28672 x 4096 Q4_K, 64 rows: 512 columns
     // 78.2 us, 1024 66.7, as the partial sums halve; 4096 x 4096, 32 tiles: 24.5, 26.1; 1000 x 2048 Q6_K:
-    // 18.8, 24.2). W's rows have no say here either.
+    // 18.8, 24.2). W's rows have no say here either, but whether the splits run in as many workgroups or
+    // one after another in one is theirs, since the sums are the same bit for bit. Measured (us, over
+    // workgroups -> in one): Q4_K 26769 x 2048 at 42 rows 37.9 -> 29.9, 128256 x 4096 at 64 rows 225 -> 190,
+    // 32000 x 1024 at 64 rows 27.6 -> 19.5, 256 rows of 14336 x 4096 94 -> 86; 14336 x 4096 at 64 rows 34.7 -> 43.2.
     int per = (int)((stages / 4 + 3) / 4 * 4);
     per = per < 8 ? 8 : per > 16 ? 16 : per;
     const int64_t splits = (stages + per - 1) / per;
-    // Chunks of up to 256 rows, of fewer where the partial sums would pass kTileWorkspace.
-    const int64_t row_bytes = K * 4 + splits * 4 + (id == Q4_K ? K / 8 : 0) + (splits > 1 ? splits * N * 4 : 0);
-    int64_t rows = batch < 256 ? batch : 256;
-    if (rows * row_bytes > kTileWorkspace) rows = kTileWorkspace / row_bytes;
-    if (rows < batch && rows > 32) rows = rows / 32 * 32;
-    if (rows < 1 || rows * K * 4 > 0x7fffffff) return t;
-    t.rows = (int)rows;
     // Tiles of 32 rows unpack W twice as often as tiles of 64, but three workgroups of them fit a CU
     // instead of two: they win while all of them run at once (61 rows, 32-row and 64-row tiles:
     // Q4_K 4096 x 4096, 256 workgroups of 32 rows, 21.5 and 26.3 us; Q4_0 11008 x 4096, 688, 30.0 and
     // 32.1; Q6_K 4096 x 14336, 896, 49.6 and 44.3). A row's sums are the same either way.
-    t.tm = (rows + 31) / 32 * ((N + 127) / 128) * splits <= 3 * g_cus ? 1 : 2;
+    const int64_t col_tiles = (N + 127) / 128, most = batch < 256 ? batch : 256;
+    auto groups = [&](int tm) { return (most + 32 * tm - 1) / (32 * tm) * col_tiles; };
+    t.tm = most <= 32 || groups(1) * splits <= 3 * g_cus ? 1 : 2;
+    if (splits > 1) {  // where W's rows fill the chip, a workgroup runs every split: no partial sums in memory
+        const float traffic = (float)((2 * splits + 1) * most * N * 4) / 8e6f + 2.f;
+        const float apart = tile_us(id, t.tm, groups(t.tm) * splits, per) + traffic;
+        const float all1 = tile_us(id, 1, groups(1), stages), all2 = most > 32 ? tile_us(id, 2, groups(2), stages) : 1e30f;
+        t.all = (all1 < all2 ? all1 : all2) < .95f * apart;
+        if (t.all) t.tm = all1 < all2 ? 1 : 2;
+    }
+    // Chunks of up to 256 rows, of fewer where the partial sums would pass kTileWorkspace.
+    const int64_t part_bytes = splits > 1 && !t.all ? splits * N * 4 : 0;
+    const int64_t row_bytes = K * 4 + splits * 4 + (id == Q4_K ? K / 8 : 0) + part_bytes;
+    int64_t rows = most;
+    if (rows * row_bytes > kTileWorkspace) rows = kTileWorkspace / row_bytes;
+    if (rows < batch && rows > 32) rows = rows / 32 * 32;
+    if (rows < 1 || rows * K * 4 > 0x7fffffff) return t;
+    t.rows = (int)rows;
     if (rows <= 32) t.tm = 1;
     t.splits = (int)splits;
     t.split_stages = per;
     t.x_bytes = (int64_t)align256((uint64_t)(rows * K * 4));
     t.scale_bytes = (int64_t)align256((uint64_t)(rows * splits) * 4);
     t.sum_bytes = id == Q4_K ? (int64_t)align256((uint64_t)(rows * (K / 32) * 4)) : 0;
-    t.bytes = t.x_bytes + t.scale_bytes + t.sum_bytes + (splits > 1 ? splits * rows * N * 4 : 0);
+    t.bytes = t.x_bytes + t.scale_bytes + t.sum_bytes + rows * part_bytes;
     return t;
 }
 
@@ -363,7 +389,7 @@ hipError_t launch_tile_fmt(const QMat &m, const float *x, const float *add, floa
     _Float16 *const hi = (_Float16 *)ws;
     float *const unscale = (float *)(ws + t.x_bytes);
     float *const sums = t.sum_bytes ? (float *)(ws + t.x_bytes + t.scale_bytes) : nullptr;
-    float *const part = t.splits > 1 ? (float *)(ws + t.x_bytes + t.scale_bytes + t.sum_bytes) : nullptr;
+    float *const part = t.splits > 1 && !t.all ? (float *)(ws + t.x_bytes + t.scale_bytes + t.sum_bytes) : nullptr;
     for (int64_t b0 = 0; b0 < batch; b0 += t.rows) {
         const int rows = (int)(batch - b0 < t.rows ? batch - b0 : t.rows);
         const float *const ab = add ? add + b0 * m.rows : nullptr;
@@ -373,12 +399,14 @@ hipError_t launch_tile_fmt(const QMat &m, const float *x, const float *add, floa
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         const unsigned tiles = (unsigned)(((rows + 32 * t.tm - 1) / (32 * t.tm)) * ((m.rows + 127) / 128));
-        const dim3 grid(tiles, (unsigned)t.splits);
+        const dim3 grid(tiles, (unsigned)(t.all ? 1 : t.splits));
         const uint16_t *const xs = (const uint16_t *)ws;
-        e = launch_with_event(t.tm == 1 ? gvt::gemv_tile<FMT, 1> : gvt::gemv_tile<FMT, 2>, grid, dim3(256), s,
-                              t.splits > 1 ? nullptr : space.done, m, xs, unscale, sums, ab, yb, rows, t.split_stages, part);
+        const auto kernel = t.all ? (t.tm == 1 ? gvt::gemv_tile<FMT, 1, true> : gvt::gemv_tile<FMT, 2, true>)
+                                  : (t.tm == 1 ? gvt::gemv_tile<FMT, 1, false> : gvt::gemv_tile<FMT, 2, false>);
+        e = launch_with_event(kernel, grid, dim3(256), s, part ? nullptr : space.done, m, xs, unscale, sums, ab, yb, rows,
+                              t.split_stages, part);
         if (e != hipSuccess) return e;
-        if (t.splits > 1) {
+        if (part) {
             e = launch_sum(part, t.splits, (int64_t)rows * m.rows, ab, yb, s, space.done);
             if (e != hipSuccess) return e;
         }
@@ -484,7 +512,7 @@ hipError_t launch_gemv(int id, const QMat &m, const float *x, const float *add, 
     const bool ws_ok = mfma && ws.ptr && ws.bytes >= gemv_window_bytes(id, m, batch);
     if (in.part && !(gemv_carries(id, m, batch, in) && (ws_ok || gemv_window_bytes(id, m, batch) == 0)))
         return hipErrorInvalidValue;
-    if (ws_ok) {
+    if (mfma && ws.ptr) {
         const TileShape t = tile_shape(id, m, batch);
         if (t.rows && ws.bytes >= (uint64_t)t.bytes) return launch_tile(id, m, x, add, y, batch, t, ws, s);
     }

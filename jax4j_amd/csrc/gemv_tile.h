@@ -98,7 +98,9 @@ split_x_kernel(const float *__restrict__ x, int K, int per, _Float16 *__restrict
     }
 }
 
-template <int FMT, int TM>
+// ALL: a workgroup takes every K split in turn (grid.y = 1) and adds their sums in its registers, in the
+// order and with the roundings of sum_windows_kernel, so results are the same bit for bit.
+template <int FMT, int TM, bool ALL>
 __global__ void __launch_bounds__(256, 2)
 gemv_tile(QMat w, const uint16_t *__restrict__ xs, const float *__restrict__ unscale, const float *__restrict__ sums,
           const float *add, float *y, int B, int split_stages, float *__restrict__ part) {
@@ -117,8 +119,8 @@ gemv_tile(QMat w, const uint16_t *__restrict__ xs, const float *__restrict__ uns
     __shared__ __attribute__((aligned(1024))) uint8_t xs0[kXs], xs1[kXs];
     __shared__ __attribute__((aligned(1024))) uint8_t ws0[U::kBytes], ws1[U::kBytes];
     const int N = (int)w.rows, K = (int)w.cols;
-    const int sbeg = (int)blockIdx.y * split_stages, send = sbeg + split_stages, all = K / 64;
-    const int ns = send < all ? send : all;  // stages [sbeg, ns)
+    const int sbeg = ALL ? 0 : (int)blockIdx.y * split_stages, send = sbeg + split_stages, all = K / 64;
+    const int ns = ALL || send > all ? all : send;  // stages [sbeg, ns)
     // each XCD takes a contiguous range of tiles, row tiles of x fastest: they share the W rows
     const int mt = (B + BM - 1) / BM, total = (int)gridDim.x;
     int tile = (int)blockIdx.x;
@@ -319,6 +321,38 @@ gemv_tile(QMat w, const uint16_t *__restrict__ xs, const float *__restrict__ uns
         }
     };
 
+    // The sum of split s of element v of tile t (row 32 t + 8 (v / 4) + 4 h + v % 4 of x), unscaled.
+    auto unscaled = [&](int s, int t, int v) __attribute__((always_inline)) -> float {
+        // both halves' scales by uniform loads, which do not wait for the loads into LDS
+        const int row = m0 + 32 * t + 8 * (v >> 2) + (v & 3), last = B - 1;
+        const float *const u = unscale + (int64_t)s * B;
+        const float u0 = u[row < last ? row : last], u1 = u[row + 4 < last ? row + 4 : last];
+        float r = acc[t][v];
+        if constexpr (MIN) r -= corr[t][v];
+        return r * (h ? u1 : u0);
+    };
+    f32x16 run[ALL ? TM : 1];
+    int split = 0, left = split_stages;  // ALL: the current split, and its stages still to come
+    if constexpr (ALL) {
+#pragma unroll
+        for (int t = 0; t < TM; t++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) run[t][v] = -0.f;
+    }
+    auto flush = [&]() __attribute__((always_inline)) {
+        fold(1);
+        fs[1] = 0.f;
+#pragma unroll
+        for (int t = 0; t < TM; t++) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) run[t][v] += unscaled(split, t, v);
+            acc[t] = sum[1][t] = f32x16{};
+            if constexpr (MIN) corr[t] = f32x16{};
+        }
+        split++;
+        left = split_stages;
+    };
+
     load_w(sbeg / 2, ws0);
     load_order();
     load_x(sbeg, xs0);
@@ -331,6 +365,10 @@ gemv_tile(QMat w, const uint16_t *__restrict__ xs, const float *__restrict__ uns
     int i = sbeg;
     for (; i + 4 <= ns; i += 4) {
         J4Q_STAGE(0) J4Q_STAGE(1) J4Q_STAGE(2) J4Q_STAGE(3)
+        if constexpr (ALL) {
+            left -= 4;
+            if (left == 0) flush();
+        }
     }
     if constexpr (FMT == Q8_0 || FMT == Q4_0) {
         if (i < ns) {
@@ -342,10 +380,13 @@ gemv_tile(QMat w, const uint16_t *__restrict__ xs, const float *__restrict__ uns
         }
     }
 #undef J4Q_STAGE
-    fold(1);  // GS is even: the last fold of a stage is its number 1
+    if constexpr (ALL) {
+        if (split * split_stages < all) flush();
+    } else {
+        fold(1);  // GS is even: the last fold of a stage is its number 1
+    }
     __builtin_amdgcn_s_waitcnt(0);  // no LDS load outlives the workgroup
 
-    // Result element v of tile t: row 32 t + 8 (v / 4) + 4 h + v % 4 of x, column r32.
     float *const out = part ? part + (int64_t)blockIdx.y * B * N : y;
     const int col = nw + r32;
     if (col >= N) return;
@@ -355,9 +396,7 @@ gemv_tile(QMat w, const uint16_t *__restrict__ xs, const float *__restrict__ uns
         for (int v = 0; v < 16; v++) {
             const int row = m0 + 32 * t + 8 * (v >> 2) + 4 * h + (v & 3);
             if (row < B) {
-                float r = acc[t][v];
-                if constexpr (MIN) r -= corr[t][v];
-                r *= unscale[(int)blockIdx.y * B + row];
+                const float r = ALL ? run[t][v] : unscaled((int)blockIdx.y, t, v);
                 const int64_t o = (int64_t)row * N + col;
                 out[o] = !part && add ? r + add[o] : r;
             }

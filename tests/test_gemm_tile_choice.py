@@ -7,14 +7,14 @@ import re
 
 import fakehip
 from test_gpu_gemm_tile import DEEP
-from test_gpu_gemv_tile import SHAPES as GEMV_SHAPES
+from test_gpu_gemv_tile import ALL_SPLITS, SHAPES as GEMV_SHAPES
 
 FORMATS = {2: "Q4_0", 8: "Q8_0", 12: "Q4_K", 14: "Q6_K"}
 
 
 def instance(kernel, name):
-    m = re.search(name + r"I((?:Li\d+E)+)E", kernel)
-    return m and tuple(map(int, re.findall(r"Li(\d+)E", m[1])))
+    m = re.search(name + r"I((?:L[ib]\d+E)+)E", kernel)
+    return m and tuple(map(int, re.findall(r"L[ib](\d+)E", m[1])))
 
 
 def picked(shim, call, sizes, name):
@@ -45,6 +45,8 @@ def test_every_gemm_tile_is_tested_at_depth(tmp_path):
 
 
 def test_every_gemv_tile_is_tested(tmp_path):
-    library, runs = picked(fakehip.build_shim(tmp_path), "j4q_quant_matvec_into(w.handle, 4096, None, 4096, m, None)", GEMV_SHAPES, "gemv_tile")
-    assert len(library) == 8
-    assert library == {i for *_, i, splits in runs if int(splits) > 1} == {i for *_, i, splits in runs if splits == "1"}
+    library, runs = picked(fakehip.build_shim(tmp_path), "j4q_quant_matvec_into(w.handle, 4096, None, 4096, m, None)",
+                           GEMV_SHAPES + ALL_SPLITS, "gemv_tile")
+    one, several = ({i for *_, i, splits in runs if (int(splits) > 1) == s} for s in (False, True))
+    assert len(library) == 16  # (format, row tiles of 32, whether a workgroup runs every split)
+    assert library == one and {i for i in library if not i[2]} == several

@@ -39,10 +39,13 @@ def matvec(backend, w, xs):
 # 1024; 2816: 768 three times and 512), of many splits (9216, 33024).
 SHAPES = [(19, 129, 512), (27, 127, 5120), (32, 300, 768), (33, 1, 2816), (35, 257, 2048), (64, 128, 512),
           (65, 130, 768), (257, 70, 512), (35, 40, 9216), (36, 33, 33024), (257, 12500, 512), (130, 5001, 2816)]
+# All K splits in one workgroup: tiles of 32 and of 64 rows, three splits and two, the last one shorter.
+ALL_SPLITS = [(65, 9001, 1280), (250, 15001, 768)]
 
 
 @pytest.mark.parametrize("qt", ALL, ids=lambda q: q.name)
-@pytest.mark.parametrize("b,n,k", SHAPES + [(19, 65, 64), (20, 140, 576), (40, 129, 1088), (70, 20, 640), (65, 20001, 576)])
+@pytest.mark.parametrize("b,n,k", SHAPES + ALL_SPLITS + [(19, 65, 64), (20, 140, 576), (40, 129, 1088), (70, 20, 640), (65, 20001, 576),
+                                                       (65, 9001, 1344), (66, 9001, 1408)])
 def test_gemv_tiles_match_oracle(backend, qt, b, n, k):
     if k % (64 if qt is QuantType.Q8_0 else 128 if qt is QuantType.Q4_0 else 256):
         pytest.skip("K of a whole number of blocks of the split layout")
@@ -96,6 +99,21 @@ def test_gemv_tile_sums_do_not_depend_on_the_launch(backend, qt):
         assert np.abs(got - want).max() <= 2.0**-20 * np.abs(want).max()
     else:
         assert np.abs(got - want).max() <= 2.0**-23 * np.abs(want).max()
+    for h in (*ws, both):
+        backend.release(h)
+
+
+@pytest.mark.parametrize("qt", ALL, ids=lambda q: q.name)
+@pytest.mark.parametrize("b,n,k", ALL_SPLITS)
+def test_gemv_tile_sums_do_not_depend_on_where_the_splits_run(backend, qt, b, n, k):
+    """Rows of W in a matrix so large that a workgroup runs every split give the bits that they give
+    alone, with a workgroup per split."""
+    blobs = [S.quant_blocks(qt, 91 + i, r, k) for i, r in enumerate((100, n - 100))]
+    ws = [backend.upload_quantized(blob, qt, (r, k)) for blob, r in zip(blobs, (100, n - 100))]
+    both = backend.concat_rows(ws)
+    xs = S.activations_f32(6, b * k).reshape(b, k)
+    xs[3] = 0
+    assert np.array_equal(bits(matvec(backend, both, xs)[:, :100]), bits(matvec(backend, ws[0], xs)))
     for h in (*ws, both):
         backend.release(h)
 
