@@ -843,9 +843,9 @@ int j4q_quant_matmul(j4q_buffer wh, j4q_buffer xh, int variant, j4q_buffer *out)
     if ((rc = alloc_buf(J4Q_KIND_F32, 2, M, N, (uint64_t)(M * N) * 4, out, &ydev, {x}))) return rc;
     if (variant == J4Q_GEMM_BF16) {
         j4q::Workspace ws;
-        const uint64_t wsb = capturing(g_stream) ? 0 : j4q::gemm_bf16_workspace_bytes(qt, m, M);
-        if (wsb) LAUNCH_INTO("quantMatmul workspace", out, g_workspaces.begin(g_stream, g_stream, wsb, &ws));
-        const hipError_t e = j4q::launch_gemm_bf16(qt, m, xdev, (float *)ydev, M, ws, g_stream);
+        const j4q::GemmShape shape = j4q::gemm_bf16_shape(qt, m, M, !capturing(g_stream));
+        if (shape.workspace) LAUNCH_INTO("quantMatmul workspace", out, g_workspaces.begin(g_stream, g_stream, shape.workspace, &ws));
+        const hipError_t e = j4q::launch_gemm_bf16(qt, m, xdev, (float *)ydev, M, shape, ws, g_stream);
         g_workspaces.end(g_stream, ws, e == hipSuccess);
         LAUNCH_INTO("quantMatmul", out, e);
         return J4Q_OK;
@@ -905,9 +905,9 @@ int j4q_quant_matmul_into(j4q_buffer wh, const uint16_t *x, int64_t m, int varia
     if (variant == J4Q_GEMM_BF16) {
         j4q::Workspace ws;
         // under capture K is not split: the workspace would be memory nodes (see run_gemv)
-        const uint64_t wsb = capturing(s) ? 0 : j4q::gemm_bf16_workspace_bytes(w->qtype, mm, m);
-        if (wsb) HIP_TRY("quantMatmul_into workspace", g_workspaces.begin(s, g_stream, wsb, &ws));
-        const hipError_t e = j4q::launch_gemm_bf16(w->qtype, mm, x, y, m, ws, s);
+        const j4q::GemmShape shape = j4q::gemm_bf16_shape(w->qtype, mm, m, !capturing(s));
+        if (shape.workspace) HIP_TRY("quantMatmul_into workspace", g_workspaces.begin(s, g_stream, shape.workspace, &ws));
+        const hipError_t e = j4q::launch_gemm_bf16(w->qtype, mm, x, y, m, shape, ws, s);
         g_workspaces.end(s, ws, e == hipSuccess);
         HIP_TRY("quantMatmul_into", e);
         return J4Q_OK;
@@ -959,7 +959,8 @@ int j4q_quant_matmul_noalloc(j4q_buffer wh, const uint16_t *x, int64_t m, int va
         j4q::Workspace ws;
         ws.ptr = (float *)g_scratch;
         ws.bytes = kScratchBytes;
-        HIP_TRY("quantMatmul_noalloc", j4q::launch_gemm_bf16(w->qtype, mm, x, y, m, ws, s));
+        const j4q::GemmShape shape = j4q::gemm_bf16_shape(w->qtype, mm, m, true);
+        HIP_TRY("quantMatmul_noalloc", j4q::launch_gemm_bf16(w->qtype, mm, x, y, m, shape, ws, s));
         return J4Q_OK;
     }
     int8_t *xq = (int8_t *)g_scratch;

@@ -6,13 +6,6 @@
 namespace j4q {
 namespace {
 
-// A launch of gemm_tile: tiles of 32 tm rows x 32 waves columns, K in `splits` ranges of
-// split_stages 64-element stages. tm = 0: the call does not run on it.
-struct Shape {
-    int waves = 0, tm = 0, splits = 1, split_stages = 0;
-    int groups = 1;  // of waves in a workgroup, each with split_stages of K
-};
-
 // The tiles, and what one stage of one workgroup takes in us on MI355X: few workgroups, each
 // alone on its CU (few); one on every CU (all: the chip's clock and its memory are shared); and as
 // a share of the CU's time when every CU runs several, one after another or side by side (shared).
@@ -46,10 +39,10 @@ constexpr int kCus = 256;  // of an MI355X; a constant, so that results do not d
 // at 5.5 MB/us. Over the sweeps (38 sizes) its choice takes 1.2 % longer than the best of all
 // shapes on average, 11 % at worst (with the groups of kGroups, 162 sizes: 0.5 %). Splits are whole multiples of four stages, and their workspace
 // is at most 32 MiB; a Q8_0 call takes no workspace, so it does not split.
-Shape pick(int id, const QMat &w, int64_t m, bool split, float *us_out) {
+GemmShape pick(int id, const QMat &w, int64_t m, bool split, float *us_out) {
     const int64_t n = w.rows, ns = w.cols / 64;
     const float alone_add = id == Q6_K ? .12f : id == Q8_0 ? .05f : 0.f, shared_add = id == Q6_K ? .09f : id == Q8_0 ? .05f : 0.f;
-    Shape best;
+    GemmShape best;
     float best_us = 0.f;
     for (const Cost &c : kCost) {
         const int64_t tiles = ((m + 32 * c.tm - 1) / (32 * c.tm)) * ((n + 32 * c.waves - 1) / (32 * c.waves));
@@ -64,7 +57,7 @@ Shape pick(int id, const QMat &w, int64_t m, bool split, float *us_out) {
             if (s > 1) us += 2.0f + .25f * (float)s + (float)((2 * s + 1) * m * n * 4) / 5.5e6f;
             if (!best.tm || us < best_us) {
                 best_us = us;
-                best = Shape{c.waves, c.tm, (int)s, (int)per, 1};
+                best = GemmShape{c.waves, c.tm, (int)s, (int)per, 1, 0};
             }
         }
     }
@@ -77,20 +70,12 @@ Shape pick(int id, const QMat &w, int64_t m, bool split, float *us_out) {
             const float us = (few + (all - few) * (float)tiles / kCus) * (float)per + c.base;
             if (us < best_us) {
                 best_us = us;
-                best = Shape{c.waves, c.tm, 1, (int)per, c.groups};
+                best = GemmShape{c.waves, c.tm, 1, (int)per, c.groups, 0};
             }
         }
     }
     *us_out = best_us;
     return best;
-}
-
-// Whether the tile kernel takes the call; the shape it runs with. split: K may be split over workgroups.
-Shape shape_of(int id, const QMat &w, int64_t m, bool split) {
-    float us = 0.f;
-    if (id == Q8_0 && w.cols % 64 != 0) return Shape{};
-    const Shape t = pick(id, w, m, split, &us);
-    return id == Q8_0 && choose_q8_bf16(w, m).us <= 1.05f * us ? Shape{} : t;
 }
 
 // y[i] = ((part[0][i] + part[1][i]) + ...) for i < n: the K splits' partial products added
@@ -116,9 +101,9 @@ sum_splits_kernel(const float *__restrict__ part, int splits, int64_t n, float *
 }
 
 template <int FMT>
-hipError_t launch_fmt(const QMat &w, const uint16_t *x, float *y, int64_t m, const Shape &t, const Workspace &ws, hipStream_t s) {
+hipError_t launch_fmt(const QMat &w, const uint16_t *x, float *y, int64_t m, const GemmShape &t, const Workspace &ws, hipStream_t s) {
     const int64_t tiles = ((m + 32 * t.tm - 1) / (32 * t.tm)) * ((w.rows + 32 * t.waves - 1) / (32 * t.waves));
-    if (tiles > 0x7fffffff || (t.splits > 1 && ws.bytes < (uint64_t)t.splits * (uint64_t)m * (uint64_t)w.rows * 4u)) return hipErrorInvalidValue;
+    if (tiles > 0x7fffffff || ws.bytes < t.workspace) return hipErrorInvalidValue;
     const dim3 grid((unsigned)tiles, (unsigned)t.splits);
     float *const part = t.splits > 1 ? ws.ptr : nullptr;
     bool launched = false;
@@ -169,15 +154,18 @@ bool gemm_bf16_supported(int id, int64_t cols) {
     }
 }
 
-uint64_t gemm_bf16_workspace_bytes(int id, const QMat &w, int64_t m) {
-    if (!gemm_bf16_supported(id, w.cols) || m <= 0 || w.rows <= 0) return 0;
-    const Shape t = shape_of(id, w, m, true);
-    return t.splits > 1 ? (uint64_t)t.splits * (uint64_t)m * (uint64_t)w.rows * 4u : 0;
+GemmShape gemm_bf16_shape(int id, const QMat &w, int64_t m, bool split) {
+    if (!gemm_bf16_supported(id, w.cols) || m <= 0 || w.rows <= 0 || (id == Q8_0 && w.cols % 64 != 0)) return GemmShape{};
+    float us = 0.f;
+    GemmShape t = pick(id, w, m, split, &us);
+    if (id == Q8_0 && choose_q8_bf16(w, m).us <= 1.05f * us) return GemmShape{};
+    t.workspace = t.splits > 1 ? (uint64_t)t.splits * (uint64_t)m * (uint64_t)w.rows * 4u : 0;
+    return t;
 }
 
-hipError_t launch_gemm_bf16(int id, const QMat &w, const uint16_t *x, float *y, int64_t m, const Workspace &ws, hipStream_t s) {
+hipError_t launch_gemm_bf16(int id, const QMat &w, const uint16_t *x, float *y, int64_t m, const GemmShape &t,
+                            const Workspace &ws, hipStream_t s) {
     if (m <= 0 || w.rows <= 0) return hipSuccess;
-    const Shape t = shape_of(id, w, m, ws.ptr != nullptr);
     if (id == Q8_0 && !t.tm) return launch_gemm_q8_bf16(w, x, y, m, s);
     if (!gemm_bf16_supported(id, w.cols) || (uint64_t)m * (uint64_t)w.cols * 2u > 0x7fffffffull ||
         (uint64_t)w.rows * (uint64_t)w.cols / (id == Q8_0 ? 1u : 2u) > 0x7fffffffull)

@@ -186,10 +186,16 @@ Q8Choice choose_q8_bf16(const QMat &w, int64_t m);
 hipError_t launch_gemm_q8_bf16(const QMat &w, const uint16_t *x, float *y, int64_t m, hipStream_t s);
 // Prefill GEMM, bf16 variant, over Q8_0, Q4_0 (cols % 128 == 0), Q4_K and Q6_K weights.
 bool gemm_bf16_supported(int id, int64_t cols);
-// Workspace the call needs (bytes, at most 32 MiB; 0: none): the partial products of its K splits. Without
-// one (ws.ptr null) launch_gemm_bf16 does not split K.
-uint64_t gemm_bf16_workspace_bytes(int id, const QMat &w, int64_t m);
-hipError_t launch_gemm_bf16(int id, const QMat &w, const uint16_t *x, float *y, int64_t m, const Workspace &ws, hipStream_t s);
+// How launch_gemm_bf16 runs a call, from a model of the launch: gemm_tile.h with tiles of 32 tm rows x 32 waves
+// columns (tm = 0: a kernel of gemm.hip instead, Q8_0 alone), K in `splits` ranges of split_stages 64-element
+// stages over workgroups, or in `groups` of a workgroup's waves. Without `split` K stays in one workgroup.
+struct GemmShape {
+    int waves = 0, tm = 0, splits = 1, split_stages = 0, groups = 1;
+    uint64_t workspace = 0;  // bytes, at most 32 MiB: the partial products of the K splits
+};
+GemmShape gemm_bf16_shape(int id, const QMat &w, int64_t m, bool split);
+hipError_t launch_gemm_bf16(int id, const QMat &w, const uint16_t *x, float *y, int64_t m, const GemmShape &shape,
+                            const Workspace &ws, hipStream_t s);
 hipError_t launch_synth_quant(int id, uint64_t seed, int64_t rows, int64_t cols, uint8_t *gguf,
                               hipStream_t s);
 hipError_t launch_synth_f32(uint64_t seed, int64_t n, float *out, hipStream_t s);
