@@ -243,6 +243,7 @@ def test_addresses_are_integers(shim):
                     refused += 1
         n = len(launches())
         be.quant_matvec_into(w, np.int64(x), 0, np.uint64(y))
+        be.quant_matvec_into(w, x, None, y, 1, None)
         result = refused, n
     """)
     assert refused == 25 and launched == 0
