@@ -158,9 +158,9 @@ struct Tile {
     static_assert(4 * TM % WV == 0, "whole X loads per wave");
 };
 
-// KG = 2 or 4 (WV = 2; KG = 2 also WV = 4): as many groups of waves, each with buffers of its own, take a part of the range of K
-// each (split_stages, a multiple of 4; K a multiple of 256). Their sums meet through LDS, a quarter of
-// the rows of a 32-row tile or a half in each group, and are added in group order.
+// KG = 2 or 4 (WV = 2; KG = 2 also WV = 4): as many groups of waves, each with buffers of its own, take a part
+// of the range of K each (split_stages, a multiple of 4; K a multiple of 256). Their sums meet through LDS, a
+// quarter of the rows of a 32-row tile or a half in each group, and are added in group order.
 template <int FMT, int WV, int TM, int KG = 1>
 __global__ void __launch_bounds__(64 * WV * KG, 2)
 gemm_tile(QMat w, const uint16_t *__restrict__ x, float *__restrict__ y, int M, int split_stages,

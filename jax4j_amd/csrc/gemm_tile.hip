@@ -37,8 +37,9 @@ constexpr int kCus = 256;  // of an MI355X; a constant, so that results do not d
 // longer to decode, Q8_0's to load), a launch's fixed 3 us, and with K split the sum kernel: 2 us,
 // a quarter per split, and its traffic (the partial products written and read, the result written)
 // at 5.5 MB/us. Over the sweeps (38 sizes) its choice takes 1.2 % longer than the best of all
-// shapes on average, 11 % at worst (with the groups of kGroups, 162 sizes: 0.5 %). Splits are whole multiples of four stages, and their workspace
-// is at most 32 MiB; a Q8_0 call takes no workspace, so it does not split.
+// shapes on average, 11 % at worst (with the groups of kGroups, 162 sizes: 0.5 %). Splits are whole
+// multiples of four stages, and their workspace is at most 32 MiB; a Q8_0 call takes no workspace, so
+// it does not split.
 GemmShape pick(int id, const QMat &w, int64_t m, bool split, float *us_out) {
     const int64_t n = w.rows, ns = w.cols / 64;
     const float alone_add = id == Q6_K ? .12f : id == Q8_0 ? .05f : 0.f, shared_add = id == Q6_K ? .09f : id == Q8_0 ? .05f : 0.f;

@@ -1,7 +1,8 @@
 // Device memory that the engine keeps between calls, for one device and under the engine's mutex.
-// hipMalloc + hipFree cost an SPI call ~8 us and a wait for the device; hipMallocAsync + hipFreeAsync
-// cost a call with a workspace ~15 us and, on this runtime, a wait for the work before it (two
-// launches of 50 us each: the host returns after 106 us with them, after 6 without).
+// hipMalloc + hipFree cost an SPI call and a wait for the device (quantMatvec + release in a loop 14.9 -> 5.1 us
+// a call without them; a token of ten calls, whose downloads wait anyhow, 66.4 -> 62.9);
+// hipMallocAsync + hipFreeAsync cost a call with a workspace ~15 us and, on this runtime, a wait for the
+// work before it (two launches of 50 us each: the host returns after 106 us with them, after 6 without).
 //  - Blocks of released F32 / BF16 / I8 buffers, in powers of two from 256 bytes to 4 MiB, at
 //    most 64 MiB in all: work on such a buffer runs on the engine stream alone, so its block may
 //    be written again behind it with no wait. A buffer whose address left the engine
