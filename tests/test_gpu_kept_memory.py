@@ -220,3 +220,42 @@ def test_workspaces_of_many_streams(backend):
         assert np.array_equal(backend.download(y).view(np.uint32), ref[i])
     for h in [*ws, *xs, *(y for _, y in results)]:
         backend.release(h)
+
+
+# 1 row: no workspace; 24 rows: tiles, the event on the GEMV's launch; 16 rows: on the window sums'
+@pytest.mark.parametrize("handle", [1, 2], ids=["hipStreamLegacy", "hipStreamPerThread"])
+@pytest.mark.parametrize("qt,b,r,k", [(QuantType.Q8_0, 1, 640, 1024), (QuantType.Q8_0, 24, 1000, 1024), (QuantType.Q4_K, 16, 640, 4096)])
+def test_workspaces_on_the_runtimes_own_streams(backend, handle, qt, b, r, k):
+    """The runtime's two stream handles that name no stream object of their own."""
+    hip = Hip()
+    w = upload(backend, qt, r, k, 61)
+    x = backend.upload(S.activations_f32(3, b * k), shape=(b, k))
+    ref = backend.quant_matvec(w, x)
+    y = backend.upload(np.full((b, r), np.nan, np.float32))
+    px, py = (backend.buffer_desc(h).device_ptr for h in (x, y))
+    print("[case]", qt.name, b, r, k, "stream handle", handle, flush=True)
+    for _ in range(3):
+        backend.quant_matvec_into(w, px, 0, py, b, handle)
+    hip.wait()
+    assert np.array_equal(backend.download(y).view(np.uint32).reshape(-1), backend.download(ref).view(np.uint32).reshape(-1))
+    for h in (w, x, ref, y):
+        backend.release(h)
+    hip.close()
+
+
+@pytest.mark.parametrize("handle", [1, 2], ids=["hipStreamLegacy", "hipStreamPerThread"])
+def test_matmul_workspaces_on_the_runtimes_own_streams(backend, handle):
+    m, n, k = 24, 512, 8192  # K split, the event on the sums' launch
+    hip = Hip()
+    w = upload(backend, QuantType.Q6_K, n, k, 51)
+    x = backend.upload(S.activations_bf16(9, m * k).reshape(m, k), shape=(m, k), dtype=DType.BF16)
+    ref = backend.quant_matmul(w, x, "bf16")
+    y = backend.upload(np.full((m, n), np.nan, np.float32))
+    px, py = (backend.buffer_desc(h).device_ptr for h in (x, y))
+    for _ in range(3):
+        backend.quant_matmul_into(w, px, m, "bf16", 0, 0, py, handle)
+    hip.wait()
+    assert np.array_equal(backend.download(y).view(np.uint32), backend.download(ref).view(np.uint32))
+    for h in (w, x, ref, y):
+        backend.release(h)
+    hip.close()
